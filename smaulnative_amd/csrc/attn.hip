@@ -33,92 +33,266 @@ namespace {
 
 // 1 / max(||k||, 1e-6) of one key (attn_cpu.cpp:40-51): the norm summed in
 // double in index order, rounded to fp32, clamped, one fp32 reciprocal.
+__device__ __forceinline__ float attn_inv_norm2(double n2) {
+  const float n = (float)__builtin_sqrt(n2);
+  const float nc = (!__builtin_isfinite(n) || n < 1e-6f) ? 1e-6f : n;
+  return 1.0f / nc;
+}
+
 __device__ __forceinline__ float attn_inv_norm(const float* k, int D) {
   double n2 = 0.0;
   for (int i = 0; i < D; ++i) {
     const double ki = (double)k[i];
     n2 = n2 + ki * ki;
   }
-  const float n = (float)__builtin_sqrt(n2);
-  const float nc = (!__builtin_isfinite(n) || n < 1e-6f) ? 1e-6f : n;
-  return 1.0f / nc;
+  return attn_inv_norm2(n2);
 }
 
-constexpr int ATTN_CH = 16;  // time steps staged per chunk (register kernel)
+// ---------------------------------------------------------------------------
+// D <= 128: a systolic array over (row i, time t)
+// ---------------------------------------------------------------------------
+// Step t of row i needs S[i] of step t - 1 and the partial num of row i - 1 at
+// step t, and nothing else: along an anti-diagonal of (t, i) every row can
+// work at once without touching the reference's order.  Lane i of a wave owns
+// row i (RPL consecutive rows for D > 64) of J columns of S in registers and
+// at tick tau works on step t = tau - i; num and den move to lane i + 1
+// between ticks as the DPP operand of the add itself (wave_shr:1, lane 0
+// starts from +0), and leave the array at the lane of row D - 1.  A tick is 4
+// VALU operations per column and row (multiply and add kept apart) plus about
+// a dozen shared by the columns, and a task of D x D takes T + D ticks on D /
+// J waves instead of T * D dependent steps on one.
+//
+// A workgroup is AC_W such waves on neighbouring columns of one task and one
+// wave that stages the next AttnCol::CH steps of q, kn and v meanwhile (the
+// key norms are a serial double sum, one lane per step).  The steps sit in a
+// ring of AC_RN, which holds the 64 a wave's lanes are spread over and the
+// chunk being written; steps outside [0, T) are zeros, which leave S and z as
+// they are (+0 + +-0 = +0, x + +-0 = x).  Row strides (in the units the lanes
+// read, 8 or 16 bytes) are chosen odd against the lanes' one-row skew, so the
+// reads meet no bank twice.
+//
+// What bounds it: the length of the array in ticks, T + D, at the issue rate
+// of one wave per SIMD.  B 2, T 256, H 8, D 64: 993 us with one workgroup and
+// one thread per column (16 workgroups, every thread walking all D rows per
+// step with three LDS reads each).
+constexpr int AC_W = 4;                     // computing waves of a workgroup
+constexpr int AC_NT = (AC_W + 1) * 64;      // and the staging wave
+constexpr int AC_RN = 128;                  // ring of time steps in LDS
 
-// S in registers: thread j owns column j (S[0..D-1][j]) and z[j].
-template <int DMAX>
-__global__ void __launch_bounds__(DMAX)
-attn_fwd_reg_kernel(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
+// lane i takes lane i - 1's value, lane 0 takes +0
+__device__ __forceinline__ float wave_shr1(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x138, 0xf, 0xf, true));
+}
+
+// LDS written by other lanes of this wave: the hardware runs a wave's LDS
+// operations in order, so only the compiler must keep them so
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int RPL, int J>
+struct AttnCol {
+  static constexpr int CH = RPL == 1 ? 32 : 16;    // steps staged at once: 64 + 2 CH <= AC_RN
+  static constexpr int CW = AC_W * J;              // columns of a workgroup
+  static constexpr int RS = RPL == 1 ? 66 : 132;   // (q, kn) pairs of a ring row
+  static constexpr int VS = CW + J;                // floats of a ring row of v
+  static constexpr int VN = CH * CW / 64;          // v values a staging lane loads per chunk
+  __attribute__((aligned(16))) float2 qk[AC_RN * RS];
+  __attribute__((aligned(16))) float v[AC_RN * VS];
+  float out[AC_W][CH][J + 1];                      // num (J) and den of the chunk's ticks
+};
+
+template <int RPL, int J>
+__global__ void __launch_bounds__(AC_NT)
+attn_fwd_col_kernel(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
                     float* __restrict__ Y, float* __restrict__ DEN, float* __restrict__ S_out,
-                    float* __restrict__ z_out, int64_t T, int H, int D, float eps) {
-  __shared__ __attribute__((aligned(16))) float s_q[ATTN_CH][DMAX];
-  __shared__ __attribute__((aligned(16))) float s_k[ATTN_CH][DMAX];
-  __shared__ __attribute__((aligned(16))) float s_v[ATTN_CH][DMAX];
-  __shared__ __attribute__((aligned(16))) float s_kn[DMAX];
-  __shared__ __attribute__((aligned(16))) float s_z[DMAX];
-  __shared__ float s_inv[ATTN_CH];
-  const int64_t task = blockIdx.x;
+                    float* __restrict__ z_out, int64_t T, int H, int D, int groups, float eps) {
+  using L = AttnCol<RPL, J>;
+  constexpr int CH = L::CH, RS = L::RS, VS = L::VS, CW = L::CW;
+  __shared__ L sm;
+  const int64_t task = blockIdx.x / groups;
+  const int cg = (int)(blockIdx.x - task * groups);
   const int64_t b = task / H, h = task % H;
-  const int j = threadIdx.x;
-  const bool col = j < D;
-  float S[DMAX];
-#pragma unroll
-  for (int i = 0; i < DMAX; ++i) S[i] = 0.0f;
-  float zj = 0.0f;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int64_t rs = (int64_t)H * D;          // stride between time steps
   const int64_t base = (b * T * H + h) * D;   // (b, t = 0, h)
-  for (int64_t t0 = 0; t0 < T; t0 += ATTN_CH) {
-    const int nt = (int)(T - t0 < ATTN_CH ? T - t0 : ATTN_CH);
-    // stage the chunk: every thread loads its column of each step
-    if (col) {
+  const int last = (D - 1) / RPL;             // the lane that holds row D - 1
+  const bool half = RPL == 2 && (D & 1);      // whose second row does not exist
+  const int64_t chunks = (T + last + CH - 1) / CH;
+
+  for (int e = tid; e < AC_RN * RS; e += AC_NT) sm.qk[e] = make_float2(0.0f, 0.0f);
+  for (int e = tid; e < AC_RN * VS; e += AC_NT) sm.v[e] = 0.0f;
+
+  // staging wave: lane = column (columns lane, lane + 64) of q and k
+  float sq[CH * RPL], sk[CH * RPL], sv[L::VN];
+  auto load = [&](int64_t c) {
 #pragma unroll
-      for (int tt = 0; tt < ATTN_CH; ++tt)
-        if (tt < nt) {
-          const int64_t o = base + (t0 + tt) * rs + j;
-          s_q[tt][j] = Q[o];
-          s_k[tt][j] = K[o];
-          s_v[tt][j] = V[o];
-        }
-    }
-    __syncthreads();
-    if (j < nt) s_inv[j] = attn_inv_norm(s_k[j], D);
-    __syncthreads();
-    for (int tt = 0; tt < nt; ++tt) {
-      float vj = 0.0f;
-      if (col) {
-        const float knj = s_k[tt][j] * s_inv[tt];
-        zj = zj + knj;
-        s_kn[j] = knj;
-        s_z[j] = zj;
-        vj = s_v[tt][j];
-      }
-      __syncthreads();
-      float num = 0.0f, den = 0.0f;
+    for (int r = 0; r < CH; ++r) {
+      const int64_t t = c * CH + r;
 #pragma unroll
-      for (int i = 0; i < DMAX; ++i) {
-        if (i < D) {
-          const float qi = s_q[tt][i];
-          S[i] = S[i] + s_kn[i] * vj;
-          num = num + qi * S[i];
-          den = den + qi * s_z[i];
-        }
+      for (int p = 0; p < RPL; ++p) {
+        const int col = lane + 64 * p;
+        const bool in = t < T && col < D;
+        const int64_t o = base + t * rs + col;
+        sq[r * RPL + p] = in ? Q[o] : 0.0f;
+        sk[r * RPL + p] = in ? K[o] : 0.0f;
       }
-      const float denc = den < eps ? eps : den;
-      const int64_t t = t0 + tt;
-      if (col) Y[base + t * rs + j] = num / denc;
-      if (DEN && j == 0) DEN[(b * T + t) * H + h] = denc;
-      __syncthreads();  // s_kn / s_z are rewritten by the next step
     }
+#pragma unroll
+    for (int n = 0; n < L::VN; ++n) {
+      const int e = lane + 64 * n, col = cg * CW + e % CW;
+      const int64_t t = c * CH + e / CW;
+      sv[n] = t < T && col < D ? V[base + t * rs + col] : 0.0f;
+    }
+  };
+  auto stage = [&](int64_t c) {
+    const int row0 = (int)(c * CH) & (AC_RN - 1);
+#pragma unroll
+    for (int r = 0; r < CH; ++r)
+#pragma unroll
+      for (int p = 0; p < RPL; ++p) sm.qk[(row0 + r) * RS + lane + 64 * p].y = sk[r * RPL + p];
+    wave_lds_fence();
+    float inv = 0.0f;
+    if (lane < CH) {  // the norm of step lane, as attn_inv_norm sums it
+      const float2* row = sm.qk + (row0 + lane) * RS;
+      double n2 = 0.0;
+      int i = 0;
+      for (; i + 8 <= D; i += 8) {
+        double k2[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const double ki = (double)row[i + u].y;
+          k2[u] = ki * ki;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) n2 = n2 + k2[u];
+      }
+      for (; i < D; ++i) {
+        const double ki = (double)row[i].y;
+        n2 = n2 + ki * ki;
+      }
+      inv = attn_inv_norm2(n2);
+    }
+    wave_lds_fence();
+#pragma unroll
+    for (int r = 0; r < CH; ++r) {
+      const float ir = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), r));
+#pragma unroll
+      for (int p = 0; p < RPL; ++p)
+        sm.qk[(row0 + r) * RS + lane + 64 * p] = make_float2(sq[r * RPL + p], sk[r * RPL + p] * ir);
+    }
+#pragma unroll
+    for (int n = 0; n < L::VN; ++n) {
+      const int e = lane + 64 * n;
+      sm.v[(row0 + e / CW) * VS + e % CW] = sv[n];
+    }
+  };
+
+  // computing waves: rows lane * RPL .., columns c0 ..
+  const int c0 = cg * CW + wave * J;
+  float S[RPL][J], z[RPL], num[J], den = 0.0f;
+#pragma unroll
+  for (int p = 0; p < RPL; ++p) {
+    z[p] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < J; ++j) S[p][j] = 0.0f;
   }
-  if (col) {
-    if (S_out) {
-      float* so = S_out + task * D * D + j;
 #pragma unroll
-      for (int i = 0; i < DMAX; ++i)
-        if (i < D) so[(int64_t)i * D] = S[i];
+  for (int j = 0; j < J; ++j) num[j] = 0.0f;
+
+  if (wave == AC_W) load(0);
+  __syncthreads();
+  if (wave == AC_W) {
+    stage(0);
+    load(1);
+  }
+  __syncthreads();
+  for (int64_t c = 0; c < chunks; ++c) {
+    if (wave == AC_W) {
+      if (c + 1 < chunks) {
+        stage(c + 1);
+        load(c + 2);
+      }
+    } else {
+      const int tick0 = (int)(c * CH) & (AC_RN - 1);
+      float* out = &sm.out[wave][0][0];
+#pragma unroll 8
+      for (int tt = 0; tt < CH; ++tt) {
+        const int row = (tick0 + tt - lane) & (AC_RN - 1);
+        float x[RPL], u[RPL], v[J];
+        if constexpr (RPL == 1) {
+          const float2 a = sm.qk[row * RS + lane];
+          x[0] = a.x;
+          u[0] = a.y;
+        } else {
+          const float4 a = *(const float4*)&sm.qk[row * RS + 2 * lane];
+          x[0] = a.x;
+          u[0] = a.y;
+          x[1] = a.z;
+          u[1] = a.w;
+        }
+        if constexpr (J == 4) {
+          const float4 a = *(const float4*)&sm.v[row * VS + wave * J];
+          v[0] = a.x;
+          v[1] = a.y;
+          v[2] = a.z;
+          v[3] = a.w;
+        } else {
+          const float2 a = *(const float2*)&sm.v[row * VS + wave * J];
+          v[0] = a.x;
+          v[1] = a.y;
+        }
+        float first[J + 1];  // after row lane * RPL
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+          S[0][j] = S[0][j] + u[0] * v[j];
+          num[j] = wave_shr1(num[j]) + x[0] * S[0][j];
+          first[j] = num[j];
+        }
+        z[0] = z[0] + u[0];
+        den = wave_shr1(den) + x[0] * z[0];
+        first[J] = den;
+        if constexpr (RPL == 2) {
+#pragma unroll
+          for (int j = 0; j < J; ++j) {
+            S[1][j] = S[1][j] + u[1] * v[j];
+            num[j] = num[j] + x[1] * S[1][j];
+          }
+          z[1] = z[1] + u[1];
+          den = den + x[1] * z[1];
+        }
+        if (lane == last) {
+#pragma unroll
+          for (int j = 0; j < J; ++j) out[tt * (J + 1) + j] = half ? first[j] : num[j];
+          out[tt * (J + 1) + J] = half ? first[J] : den;
+        }
+      }
+      wave_lds_fence();
+      const int64_t t = c * CH + lane - last;  // the step that left the array at tick c * CH + lane
+      if (lane < CH && t >= 0 && t < T) {
+        const float d = out[lane * (J + 1) + J];
+        const float denc = d < eps ? eps : d;
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+          if (c0 + j < D) Y[base + t * rs + c0 + j] = out[lane * (J + 1) + j] / denc;
+        if (DEN && c0 == 0) DEN[(b * T + t) * H + h] = denc;
+      }
+      wave_lds_fence();
     }
-    if (z_out) z_out[task * D + j] = zj;
+    __syncthreads();
+  }
+  if (S_out && wave < AC_W) {
+#pragma unroll
+    for (int p = 0; p < RPL; ++p) {
+      const int i = lane * RPL + p;
+      if (i >= D) continue;
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        if (c0 + j < D) S_out[(task * D + i) * D + c0 + j] = S[p][j];
+      if (c0 == 0) z_out[task * D + i] = z[p];
+    }
   }
 }
 
@@ -414,13 +588,23 @@ int smaul_attn_forward(const float* Q, const float* K, const float* V, float* Y,
   const dim3 grid((unsigned)(B * H));
   if (D <= 128) {
     if (T == 0 && !S_out) return SMAUL_OK;  // T == 0 with a state: the kernel writes zeros
+    // Columns per wave: with 2 a tick is shorter (19 instructions against 27)
+    // but the shared ones are repeated more often, so it pays only while the
+    // narrower workgroups still find a CU each
+    const int64_t tasks = B * H;
+    const int64_t narrow = (D + AC_W * 2 - 1) / (AC_W * 2), wide = (D + AC_W * 4 - 1) / (AC_W * 4);
+    const bool two = tasks * narrow <= 256;
+    const int64_t groups = two ? narrow : wide;
+    const dim3 cgrid((unsigned)(tasks * groups));
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, cgrid, dim3(AC_NT), 0, stream, Q, K, V, Y, DEN, S_out, z_out, T, (int)H, (int)D,
+                         (int)groups, eps);
+    };
     if (D <= 64)
-      hipLaunchKernelGGL((attn_fwd_reg_kernel<64>), grid, dim3(64), 0, stream, Q, K, V, Y, DEN, S_out, z_out, T,
-                         (int)H, (int)D, eps);
+      two ? go(attn_fwd_col_kernel<1, 2>) : go(attn_fwd_col_kernel<1, 4>);
     else
-      hipLaunchKernelGGL((attn_fwd_reg_kernel<128>), grid, dim3(128), 0, stream, Q, K, V, Y, DEN, S_out, z_out, T,
-                         (int)H, (int)D, eps);
-    return check_launch("attn_fwd_reg_kernel");
+      two ? go(attn_fwd_col_kernel<2, 2>) : go(attn_fwd_col_kernel<2, 4>);
+    return check_launch("attn_fwd_col_kernel");
   }
   float* state = S_out;
   if (!state) {

@@ -67,6 +67,24 @@ def test_attn_forward_bit_exact(B, T, H, D):
     assert torch.equal(Y2.cpu(), Yr)
 
 
+@pytest.mark.parametrize("B,T,H,D", [
+    # D <= 128 runs as a systolic array over (row, step): widths about a wave
+    # (one row a lane up to 64, two above, the odd one alone), steps about the
+    # staged chunks (32 / 16) and the ring of 128, columns about a workgroup's
+    (1, 31, 1, 63), (1, 33, 2, 65), (2, 130, 1, 64), (1, 129, 1, 127), (1, 16, 1, 100), (1, 161, 3, 9),
+    (8, 70, 8, 64), (4, 40, 16, 48), (5, 35, 16, 32), (3, 17, 8, 128),   # four columns a wave
+])
+def test_attn_forward_array_edges(B, T, H, D):
+    print(f"case attn_forward array B={B} T={T} H={H} D={D}", flush=True)
+    Q, K, V = attn_inputs(B, T, H, D, B * 5 + T + D)
+    K[0, T // 2, 0] = 0.0                      # the norm's clamp inside a chunk
+    Q[0, T // 3] = -Q[0, T // 3]               # den below eps
+    Yr, DENr, Sr, zr = oracle.attn_forward(Q, K, V)
+    Y, DEN, S, z = be().attn_forward(Q.to(DEV), K.to(DEV), V.to(DEV), 1e-6, True, need_state=True)
+    assert torch.equal(Y.cpu(), Yr) and torch.equal(DEN.cpu(), DENr)
+    assert torch.equal(S.cpu(), Sr) and torch.equal(z.cpu(), zr)
+
+
 def test_attn_forward_empty_and_zero_keys():
     # T = 0 with the state requested: zeros (attn_cpu.cpp:176-188)
     Q, K, V = attn_inputs(2, 0, 3, 64, 1)
