@@ -400,10 +400,13 @@ int smaul_attn_step(float* S, float* z, const float* q, const float* k, const fl
  * native two-pass kernel kernel/attn_cpu.cpp attn_backward (:227-368),
  * reached through the backend entry kernel/compute.py:314-322 from
  * model.py:249,262; results are bit-identical to it.  All fp32 contiguous;
- * 0 < D <= 2048, eps positive and finite (the forward's).  For D > 128 the
- * per-task state lives in `workspace` (smaul_attn_workspace_size(B, H, D, 0)
- * bytes; 0 otherwise).
+ * 0 < D <= 2048, eps positive and finite (the forward's).  `workspace`:
+ * smaul_attn_backward_workspace_size(B, T, H, D) bytes.  With less (or NULL)
+ * D <= 128 still runs, on one slower kernel; D > 128 needs
+ * smaul_attn_workspace_size(B, H, D, 0) bytes for the per-task state.
  */
+int64_t smaul_attn_backward_workspace_size(int64_t B, int64_t T, int64_t H, int64_t D);
+
 int smaul_attn_backward(const float* dY, const float* Q, const float* K, const float* V, const float* Y,
                         const float* DEN, float* dQ, float* dK, float* dV, int64_t B, int64_t T, int64_t H, int64_t D,
                         float eps, void* workspace, int64_t workspace_bytes, hipStream_t stream);

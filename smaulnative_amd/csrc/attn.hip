@@ -17,13 +17,13 @@
 // correctly rounded.  Element (i, j) of S and entry j of num are owned by one
 // thread (column j), so the reference's per-element order holds exactly.
 //
-// Parallelism is over (b, h) tasks, one workgroup each; within a task over
-// the D columns of S.  For D <= 128 (every preset of the reference:
-// model.py:1020-1085) the task's S lives in registers, one column per
-// thread, and a chunk of CH time steps of q/k/v is staged through LDS with
-// coalesced loads, the chunk's key norms computed by CH threads in parallel.
-// Larger D (the reference accepts D <= 2048) keeps S in global memory: the
-// caller's S_out, or a workspace when the state is not wanted.
+// For D <= 128 (every preset of the reference: model.py:1020-1085) the forward
+// and the backward run as systolic arrays over (row, step) that keep every
+// sum's order (below); larger D (the reference accepts D <= 2048) keeps S in
+// global memory, the caller's S_out or a workspace, with one workgroup per
+// (b, h) task.
+#include <type_traits>
+
 #include "smaul_common.h"
 
 using smaul::check_launch;
@@ -62,22 +62,25 @@ __device__ __forceinline__ float attn_inv_norm(const float* k, int D) {
 // a dozen shared by the columns, and a task of D x D takes T + D ticks on D /
 // J waves instead of T * D dependent steps on one.
 //
-// A workgroup is AC_W such waves on neighbouring columns of one task and one
-// wave that stages the next AttnCol::CH steps of q, kn and v meanwhile (the
-// key norms are a serial double sum, one lane per step).  The steps sit in a
-// ring of AC_RN, which holds the 64 a wave's lanes are spread over and the
+// A workgroup is AC_W such waves on neighbouring columns of one task, one
+// wave that stages the next AttnCol::CH steps of q, kn and v meanwhile, and
+// one that computes the key norms of the steps after those (a serial double
+// sum, one lane per step).  The steps sit in a
+// ring, which holds the 64 a wave's lanes are spread over and the
 // chunk being written; steps outside [0, T) are zeros, which leave S and z as
 // they are (+0 + +-0 = +0, x + +-0 = x).  Row strides (in the units the lanes
 // read, 8 or 16 bytes) are chosen odd against the lanes' one-row skew, so the
 // reads meet no bank twice.
 //
 // What bounds it: the length of the array in ticks, T + D, at the issue rate
-// of one wave per SIMD.  B 2, T 256, H 8, D 64: 993 us with one workgroup and
-// one thread per column (16 workgroups, every thread walking all D rows per
-// step with three LDS reads each).
+// of one wave per SIMD (4.6 cycles an instruction, 8.7 an add with a DPP
+// operand: about 140 cycles a tick at J = 2).  B 2, T 256, H 8, D 64: 32 us,
+// against 990 us with one workgroup per task and one thread per column (16
+// workgroups, every thread walking all D rows of a step with three LDS reads
+// each); 44 us before the staging was spread over two waves and the operands
+// were read a batch ahead.
 constexpr int AC_W = 4;                     // computing waves of a workgroup
-constexpr int AC_NT = (AC_W + 1) * 64;      // and the staging wave
-constexpr int AC_RN = 128;                  // ring of time steps in LDS
+constexpr int AC_NT = (AC_W + 2) * 64;      // and the staging and the norm wave
 
 // lane i takes lane i - 1's value, lane 0 takes +0
 __device__ __forceinline__ float wave_shr1(float x) {
@@ -92,103 +95,211 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int RPL, int J>
-struct AttnCol {
-  static constexpr int CH = RPL == 1 ? 32 : 16;    // steps staged at once: 64 + 2 CH <= AC_RN
-  static constexpr int CW = AC_W * J;              // columns of a workgroup
-  static constexpr int RS = RPL == 1 ? 66 : 132;   // (q, kn) pairs of a ring row
-  static constexpr int VS = CW + J;                // floats of a ring row of v
-  static constexpr int VN = CH * CW / 64;          // v values a staging lane loads per chunk
-  __attribute__((aligned(16))) float2 qk[AC_RN * RS];
-  __attribute__((aligned(16))) float v[AC_RN * VS];
-  float out[AC_W][CH][J + 1];                      // num (J) and den of the chunk's ticks
-};
+template <int N>
+using Set = std::integral_constant<int, N>;  // a register set by number, known when compiled
 
 template <int RPL, int J>
-__global__ void __launch_bounds__(AC_NT)
-attn_fwd_col_kernel(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
-                    float* __restrict__ Y, float* __restrict__ DEN, float* __restrict__ S_out,
-                    float* __restrict__ z_out, int64_t T, int H, int D, int groups, float eps) {
+struct AttnCol {
+  static constexpr int CH = RPL == 1 ? 32 : 16;    // steps staged at once
+  static constexpr int RN = RPL == 1 ? 128 : 96;   // steps in the ring, at least 64 + 2 CH
+  static constexpr int NB = J == 8 ? 4 : 8;        // ticks whose operands are read together
+  static constexpr int CW = AC_W * J;              // columns of a workgroup
+  static constexpr int RS = RPL == 1 ? 66 : 132;   // (x, u) pairs of a ring row
+  static constexpr int VS = CW + (J == 2 ? 2 : 4); // floats of a ring row of v
+  static constexpr int VN = CH * CW / 64;          // v values a staging lane loads per chunk
+  __attribute__((aligned(16))) float2 xu[RN * RS];
+  __attribute__((aligned(16))) float v[RN * VS];
+  float out[AC_W][CH][J + 1];                      // num (J) and den of the chunk's ticks
+  float k[2 * CH][64 * RPL + 1];                   // raw keys of the norm wave's two chunks
+  float inv[4][CH];                                // 1 / norm of a chunk's keys, by chunk mod 4
+};
+
+// REV is the adjoint's column pass of the backward: time runs backwards, the
+// state is Dm += q (x) dnum with dnum = V (1 / DEN_in) (V is dY), and what
+// leaves the array is dv = Dm^T kn, stored as it is.
+template <int RPL, int J, bool REV>
+__device__ __forceinline__ void
+attn_col(AttnCol<RPL, J>& sm, const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
+         const float* __restrict__ DEN_in, float* __restrict__ Y, float* __restrict__ DEN, float* __restrict__ S_out,
+         float* __restrict__ z_out, int64_t T, int H, int D, int groups, float eps) {
   using L = AttnCol<RPL, J>;
-  constexpr int CH = L::CH, RS = L::RS, VS = L::VS, CW = L::CW;
-  __shared__ L sm;
+  constexpr int CH = L::CH, RS = L::RS, VS = L::VS, CW = L::CW, RN = L::RN, NB = L::NB;
   const int64_t task = blockIdx.x / groups;
   const int cg = (int)(blockIdx.x - task * groups);
   const int64_t b = task / H, h = task % H;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int64_t rs = (int64_t)H * D;          // stride between time steps
-  const int64_t base = (b * T * H + h) * D;   // (b, t = 0, h)
+  const int tid = threadIdx.x, lane = tid & 63;
+  // uniform, so that the two roles are scalar branches and each wave meets its own barriers only
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // stride between steps and the first one
+  const int64_t rs = REV ? -(int64_t)H * D : (int64_t)H * D;
+  const int64_t base = ((b * T + (REV ? T - 1 : 0)) * H + h) * D;
   const int last = (D - 1) / RPL;             // the lane that holds row D - 1
   const bool half = RPL == 2 && (D & 1);      // whose second row does not exist
-  const int64_t chunks = (T + last + CH - 1) / CH;
+  const int64_t chunks = T > 0 ? (T + last + CH - 1) / CH : 0;
 
-  for (int e = tid; e < AC_RN * RS; e += AC_NT) sm.qk[e] = make_float2(0.0f, 0.0f);
-  for (int e = tid; e < AC_RN * VS; e += AC_NT) sm.v[e] = 0.0f;
+  for (int e = tid; e < RN * RS; e += AC_NT) sm.xu[e] = make_float2(0.0f, 0.0f);
+  for (int e = tid; e < RN * VS; e += AC_NT) sm.v[e] = 0.0f;
 
-  // staging wave: lane = column (columns lane, lane + 64) of q and k
-  float sq[CH * RPL], sk[CH * RPL], sv[L::VN];
-  auto load = [&](int64_t c) {
+  if (wave == AC_W) {
+    // staging wave: lane = column (columns lane, lane + 64) of q and k, the
+    // last one again past D (such lanes' values reach no result); steps past
+    // T are zero.  Two register sets: the loads of a chunk are issued two
+    // periods before its values are written to the ring
+    float sq[2][CH * RPL], sk[2][CH * RPL], sv[2][L::VN], sd[2][REV ? L::VN : 1];
+    constexpr int VR = 64 / CW;  // rows of v that a load of the wave covers
+    const int vr0 = lane / CW;
+    uint32_t col[RPL];
 #pragma unroll
-    for (int r = 0; r < CH; ++r) {
-      const int64_t t = c * CH + r;
+    for (int p = 0; p < RPL; ++p) col[p] = lane + 64 * p < D ? lane + 64 * p : D - 1;
+    const int64_t voff = vr0 * rs + (cg * CW + lane % CW < D ? cg * CW + lane % CW : D - 1);
+    const int64_t doff = REV ? (b * T + T - 1 - vr0) * H + h : 0;  // DEN of step vr0
+    auto load = [&](auto set, int64_t c) {
+      const int64_t left = T - c * CH;  // steps of this chunk on
+      if (left >= CH) {
+        const float *qr = Q + base + c * CH * rs, *kr = K + base + c * CH * rs;
+        const float* vr = V + base + c * CH * rs;
+        const float* dr = REV ? DEN_in - c * CH * H : nullptr;
 #pragma unroll
-      for (int p = 0; p < RPL; ++p) {
-        const int col = lane + 64 * p;
-        const bool in = t < T && col < D;
-        const int64_t o = base + t * rs + col;
-        sq[r * RPL + p] = in ? Q[o] : 0.0f;
-        sk[r * RPL + p] = in ? K[o] : 0.0f;
-      }
-    }
+        for (int r = 0; r < CH; ++r, qr += rs, kr += rs)
 #pragma unroll
-    for (int n = 0; n < L::VN; ++n) {
-      const int e = lane + 64 * n, col = cg * CW + e % CW;
-      const int64_t t = c * CH + e / CW;
-      sv[n] = t < T && col < D ? V[base + t * rs + col] : 0.0f;
-    }
-  };
-  auto stage = [&](int64_t c) {
-    const int row0 = (int)(c * CH) & (AC_RN - 1);
+          for (int p = 0; p < RPL; ++p) {
+            sq[set][r * RPL + p] = qr[col[p]];
+            sk[set][r * RPL + p] = kr[col[p]];
+          }
 #pragma unroll
-    for (int r = 0; r < CH; ++r)
-#pragma unroll
-      for (int p = 0; p < RPL; ++p) sm.qk[(row0 + r) * RS + lane + 64 * p].y = sk[r * RPL + p];
-    wave_lds_fence();
-    float inv = 0.0f;
-    if (lane < CH) {  // the norm of step lane, as attn_inv_norm sums it
-      const float2* row = sm.qk + (row0 + lane) * RS;
-      double n2 = 0.0;
-      int i = 0;
-      for (; i + 8 <= D; i += 8) {
-        double k2[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-          const double ki = (double)row[i + u].y;
-          k2[u] = ki * ki;
+        for (int n = 0; n < L::VN; ++n, vr += VR * rs) {
+          sv[set][n] = vr[voff];
+          if constexpr (REV) {
+            sd[set][n] = dr[doff];
+            dr -= (int64_t)VR * H;
+          }
         }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) n2 = n2 + k2[u];
+        return;
       }
-      for (; i < D; ++i) {
-        const double ki = (double)row[i].y;
+#pragma unroll
+      for (int r = 0; r < CH; ++r) {
+        const int64_t o = base + (c * CH + r) * rs;
+#pragma unroll
+        for (int p = 0; p < RPL; ++p) {
+          sq[set][r * RPL + p] = r < left ? Q[o + col[p]] : 0.0f;
+          sk[set][r * RPL + p] = r < left ? K[o + col[p]] : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < L::VN; ++n) {
+        const int64_t t = c * CH + n * VR;
+        const bool in = n * VR + vr0 < left;
+        sv[set][n] = in ? V[base + t * rs + voff] : 0.0f;
+        if constexpr (REV) sd[set][n] = in ? DEN_in[doff - t * H] : 1.0f;
+      }
+    };
+    auto stage = [&](auto set, int64_t c) {
+      const int row0 = (int)(c % (RN / CH)) * CH;
+      const float inv = lane < CH ? sm.inv[c & 3][lane] : 0.0f;
+#pragma unroll
+      for (int r = 0; r < CH; ++r) {
+        const float ir = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), r));
+#pragma unroll
+        for (int p = 0; p < RPL; ++p) {
+          const float q = sq[set][r * RPL + p], kn = sk[set][r * RPL + p] * ir;
+          sm.xu[(row0 + r) * RS + lane + 64 * p] = REV ? make_float2(kn, q) : make_float2(q, kn);
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < L::VN; ++n) {
+        sm.v[(row0 + n * VR + vr0) * VS + lane % CW] = REV ? sv[set][n] * (1.0f / sd[set][n]) : sv[set][n];
+      }
+    };
+    if (T > 0) {
+      load(Set<0>(), 0);
+      load(Set<1>(), 1);
+    }
+    __syncthreads();
+    if (T > 0) {
+      stage(Set<0>(), 0);
+      load(Set<0>(), 2);
+    }
+    __syncthreads();
+    for (int64_t c = 0; c < chunks; c += 2) {  // period c stages chunk c + 1
+      if (c + 1 < chunks) {
+        stage(Set<1>(), c + 1);
+        load(Set<1>(), c + 3);
+      }
+      __syncthreads();
+      if (c + 1 < chunks) {
+        if (c + 2 < chunks) {
+          stage(Set<0>(), c + 2);
+          load(Set<0>(), c + 4);
+        }
+        __syncthreads();
+      }
+    }
+    return;
+  }
+
+  if (wave == AC_W + 1) {
+    // norm wave, lane = step: the norms of chunks 2 m and 2 m + 1 in the two
+    // periods that end before period 2 m - 1, which stages the first of them
+    float sk[2 * CH * RPL];
+    double n2 = 0.0;
+    auto load = [&](int64_t m) {
+      const int64_t left = T - 2 * m * CH;
+      const float* kr = K + base + (left > 0 ? 2 * m * CH : T - 1) * rs;
+#pragma unroll
+      for (int r = 0; r < 2 * CH; ++r) {
+#pragma unroll
+        for (int p = 0; p < RPL; ++p) sk[r * RPL + p] = kr[lane + 64 * p < D ? lane + 64 * p : D - 1];
+        kr += r + 1 < left ? rs : 0;  // steps past T: the last one again
+      }
+    };
+    const int mid = D / 32 * 16;
+    auto sum = [&](int i, int end) {  // as attn_inv_norm does
+      const float* row = sm.k[lane & (2 * CH - 1)];
+      for (; i + 16 <= end; i += 16) {
+        float k[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) k[u] = row[i + u];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) n2 = n2 + (double)k[u] * (double)k[u];
+      }
+      for (; i < end; ++i) {
+        const double ki = (double)row[i];
         n2 = n2 + ki * ki;
       }
-      inv = attn_inv_norm2(n2);
-    }
-    wave_lds_fence();
+    };
+    auto first_half = [&](int64_t m) {
 #pragma unroll
-    for (int r = 0; r < CH; ++r) {
-      const float ir = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(inv), r));
+      for (int r = 0; r < 2 * CH; ++r)
 #pragma unroll
-      for (int p = 0; p < RPL; ++p)
-        sm.qk[(row0 + r) * RS + lane + 64 * p] = make_float2(sq[r * RPL + p], sk[r * RPL + p] * ir);
+        for (int p = 0; p < RPL; ++p) sm.k[r][lane + 64 * p] = sk[r * RPL + p];
+      wave_lds_fence();
+      load(m + 1);
+      n2 = 0.0;
+      sum(0, mid);
+    };
+    auto second_half = [&](int64_t m) {
+      sum(mid, D);
+      if (lane < 2 * CH) sm.inv[(2 * m + lane / CH) & 3][lane % CH] = attn_inv_norm2(n2);
+      wave_lds_fence();
+    };
+    if (T > 0) {
+      load(0);
+      first_half(0);
+      second_half(0);
     }
-#pragma unroll
-    for (int n = 0; n < L::VN; ++n) {
-      const int e = lane + 64 * n;
-      sm.v[(row0 + e / CW) * VS + e % CW] = sv[n];
+    __syncthreads();
+    for (int64_t c = -1; c < chunks; ++c) {
+      const int64_t m = (c + 3) >> 1;
+      if (2 * m < chunks) {
+        if (c & 1)
+          first_half(m);
+        else
+          second_half(m);
+      }
+      __syncthreads();
     }
-  };
+    return;
+  }
 
   // computing waves: rows lane * RPL .., columns c0 ..
   const int c0 = cg * CW + wave * J;
@@ -201,89 +312,109 @@ attn_fwd_col_kernel(const float* __restrict__ Q, const float* __restrict__ K, co
   }
 #pragma unroll
   for (int j = 0; j < J; ++j) num[j] = 0.0f;
-
-  if (wave == AC_W) load(0);
   __syncthreads();
-  if (wave == AC_W) {
-    stage(0);
-    load(1);
-  }
   __syncthreads();
   for (int64_t c = 0; c < chunks; ++c) {
-    if (wave == AC_W) {
-      if (c + 1 < chunks) {
-        stage(c + 1);
-        load(c + 2);
+    // in batches of NB ticks, the operands of the next batch read meanwhile
+    const int tick0 = (int)(c % (RN / CH)) * CH;
+    float* out = &sm.out[wave][0][0];
+    float x[2][NB][RPL], u[2][NB][RPL], v[2][NB][J];
+    auto fetch = [&](int set, int tt, int tick) {
+      int row = tick0 + tick - lane;
+      if constexpr (RN == 128)
+        row &= RN - 1;
+      else
+        row = (int)min((unsigned)row, (unsigned)(row + RN));
+      const float* a = (const float*)&sm.xu[row * RS + RPL * lane];
+      if constexpr (RPL == 1) {
+        const float2 w = *(const float2*)a;
+        x[set][tt][0] = w.x;
+        u[set][tt][0] = w.y;
+      } else {
+        const float4 w = *(const float4*)a;
+        x[set][tt][0] = w.x;
+        u[set][tt][0] = w.y;
+        x[set][tt][1] = w.z;
+        u[set][tt][1] = w.w;
       }
-    } else {
-      const int tick0 = (int)(c * CH) & (AC_RN - 1);
-      float* out = &sm.out[wave][0][0];
-#pragma unroll 8
-      for (int tt = 0; tt < CH; ++tt) {
-        const int row = (tick0 + tt - lane) & (AC_RN - 1);
-        float x[RPL], u[RPL], v[J];
-        if constexpr (RPL == 1) {
-          const float2 a = sm.qk[row * RS + lane];
-          x[0] = a.x;
-          u[0] = a.y;
-        } else {
-          const float4 a = *(const float4*)&sm.qk[row * RS + 2 * lane];
-          x[0] = a.x;
-          u[0] = a.y;
-          x[1] = a.z;
-          u[1] = a.w;
-        }
-        if constexpr (J == 4) {
-          const float4 a = *(const float4*)&sm.v[row * VS + wave * J];
-          v[0] = a.x;
-          v[1] = a.y;
-          v[2] = a.z;
-          v[3] = a.w;
-        } else {
-          const float2 a = *(const float2*)&sm.v[row * VS + wave * J];
-          v[0] = a.x;
-          v[1] = a.y;
-        }
-        float first[J + 1];  // after row lane * RPL
+      if constexpr (J == 2) {
+        const float2 w = *(const float2*)&sm.v[row * VS + wave * J];
+        v[set][tt][0] = w.x;
+        v[set][tt][1] = w.y;
+      } else {
 #pragma unroll
-        for (int j = 0; j < J; ++j) {
-          S[0][j] = S[0][j] + u[0] * v[j];
-          num[j] = wave_shr1(num[j]) + x[0] * S[0][j];
-          first[j] = num[j];
+        for (int j = 0; j < J; j += 4) {
+          const float4 w = *(const float4*)&sm.v[row * VS + wave * J + j];
+          v[set][tt][j] = w.x;
+          v[set][tt][j + 1] = w.y;
+          v[set][tt][j + 2] = w.z;
+          v[set][tt][j + 3] = w.w;
         }
-        z[0] = z[0] + u[0];
-        den = wave_shr1(den) + x[0] * z[0];
-        first[J] = den;
-        if constexpr (RPL == 2) {
+      }
+    };
 #pragma unroll
-          for (int j = 0; j < J; ++j) {
-            S[1][j] = S[1][j] + u[1] * v[j];
-            num[j] = num[j] + x[1] * S[1][j];
+    for (int tt = 0; tt < NB; ++tt) fetch(0, tt, tt);
+#pragma unroll
+    for (int tt0 = 0; tt0 < CH; tt0 += NB) {
+      const int s = (tt0 / NB) & 1;
+      float left[NB][J + 1];  // what leaves the array at the lane of row D - 1
+#pragma unroll
+      for (int tt = 0; tt < NB; ++tt) {
+        if (tt0 + NB < CH) fetch(s ^ 1, tt, tt0 + NB + tt);
+        // groups of operations that do not depend on one another: a DPP read
+        // wants two instructions between it and what it reads
+        float g[J], gz = 0.0f;
+#pragma unroll
+        for (int p = 0; p < RPL; ++p) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < J; ++j) g[j] = u[s][tt][p] * v[s][tt][j];
+          if constexpr (!REV) z[p] = z[p] + u[s][tt][p];
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < J; ++j) S[p][j] = S[p][j] + g[j];
+          if constexpr (!REV) gz = x[s][tt][p] * z[p];
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = 0; j < J; ++j) g[j] = x[s][tt][p] * S[p][j];
+          __builtin_amdgcn_sched_barrier(0);
+          if constexpr (!REV) {
+            den = (p ? den : wave_shr1(den)) + gz;
+            left[tt][J] = p && half ? left[tt][J] : den;
           }
-          z[1] = z[1] + u[1];
-          den = den + x[1] * z[1];
-        }
-        if (lane == last) {
 #pragma unroll
-          for (int j = 0; j < J; ++j) out[tt * (J + 1) + j] = half ? first[j] : num[j];
-          out[tt * (J + 1) + J] = half ? first[J] : den;
+          for (int j = 0; j < J; ++j) num[j] = (p ? num[j] : wave_shr1(num[j])) + g[j];
+#pragma unroll
+          for (int j = 0; j < J; ++j) left[tt][j] = p && half ? left[tt][j] : num[j];
         }
       }
-      wave_lds_fence();
-      const int64_t t = c * CH + lane - last;  // the step that left the array at tick c * CH + lane
-      if (lane < CH && t >= 0 && t < T) {
-        const float d = out[lane * (J + 1) + J];
-        const float denc = d < eps ? eps : d;
+      if (lane == last) {
 #pragma unroll
-        for (int j = 0; j < J; ++j)
-          if (c0 + j < D) Y[base + t * rs + c0 + j] = out[lane * (J + 1) + j] / denc;
+        for (int tt = 0; tt < NB; ++tt)
+#pragma unroll
+          for (int j = 0; j < J + !REV; ++j) out[(tt0 + tt) * (J + 1) + j] = left[tt][j];
+      }
+    }
+    wave_lds_fence();
+    const int64_t t = c * CH + lane - last;  // the step that left the array at tick c * CH + lane
+    if (lane < CH && t >= 0 && t < T) {
+      float denc = 1.0f;
+      if constexpr (!REV) {
+        const float d = out[lane * (J + 1) + J];
+        denc = d < eps ? eps : d;
         if (DEN && c0 == 0) DEN[(b * T + t) * H + h] = denc;
       }
-      wave_lds_fence();
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+        if (c0 + j < D) {
+          const float n = out[lane * (J + 1) + j];
+          Y[base + t * rs + c0 + j] = REV ? n : n / denc;
+        }
     }
+    wave_lds_fence();
     __syncthreads();
   }
-  if (S_out && wave < AC_W) {
+  if (S_out) {
 #pragma unroll
     for (int p = 0; p < RPL; ++p) {
       const int i = lane * RPL + p;
@@ -294,6 +425,25 @@ attn_fwd_col_kernel(const float* __restrict__ Q, const float* __restrict__ K, co
       if (c0 == 0) z_out[task * D + i] = z[p];
     }
   }
+}
+
+template <int RPL, int J>
+__global__ void __launch_bounds__(AC_NT)
+attn_fwd_col_kernel(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
+                    float* __restrict__ Y, float* __restrict__ DEN, float* __restrict__ S_out,
+                    float* __restrict__ z_out, int64_t T, int H, int D, int groups, float eps) {
+  __shared__ AttnCol<RPL, J> sm;
+  attn_col<RPL, J, false>(sm, Q, K, V, nullptr, Y, DEN, S_out, z_out, T, H, D, groups, eps);
+}
+
+// Columns per wave: the fewest of 2, 4, 8 whose workgroups (tasks of them,
+// times the passes of one launch) still find a CU each.  A tick costs about
+// 4 J + 15 instructions, so fewer columns finish sooner as long as no CU has
+// to run two workgroups, and beyond that more of them share the 15.
+int attn_col_width(int64_t tasks, int64_t D) {
+  for (int j = 2; j < 8; j *= 2)
+    if (tasks * ((D + AC_W * j - 1) / (AC_W * j)) <= 256) return j;
+  return 8;
 }
 
 constexpr int ATTN_GTHREADS = 256;
@@ -553,6 +703,365 @@ attn_bwd_kernel(const float* __restrict__ dY, const float* __restrict__ Q, const
   }
 }
 
+// ---- the backward for D in {16, 32, 48, 64, 96, 128} ------------------------
+// The same sums in the same order, spread over four launches:
+//  1. attn_bwd_col_kernel: the column passes (sums over i), num / den of pass A
+//     and dv of pass B, as the forward's systolic array (attn_col), both in
+//     one launch; pass A's y goes to dQ, which is free until step 3.
+//  2. attn_bwd_scalars_kernel: per (b, t, h) the serial sums over D: the key
+//     norm, dy . y of both passes.
+//  3. attn_bwd_row_kernel: the row passes, dq = S dnum + dden z and dk~ = Dm v
+//     + dz, again both in one launch.
+//  4. attn_bwd_dk_kernel: the key normalisation's backward, in place on dk~.
+// One workgroup per task walking 2 T dependent steps (attn_bwd_kernel, which
+// the other widths and callers without the workspace keep) takes 5004 us at B
+// 8, T 256, H 8, D 64, these four 124 us; at D = 128 (B 8, T 256, H 16) 10340
+// and 636 us.
+template <int RPL, int J>
+__global__ void __launch_bounds__(AC_NT)
+attn_bwd_col_kernel(const float* __restrict__ dY, const float* __restrict__ Q, const float* __restrict__ K,
+                    const float* __restrict__ V, const float* __restrict__ DEN, float* __restrict__ Yp,
+                    float* __restrict__ DENp, float* __restrict__ dV, int64_t T, int H, int D, int groups, float eps) {
+  __shared__ AttnCol<RPL, J> sm;
+  if (blockIdx.y == 0)
+    attn_col<RPL, J, false>(sm, Q, K, V, nullptr, Yp, DENp, nullptr, nullptr, T, H, D, groups, eps);
+  else
+    attn_col<RPL, J, true>(sm, Q, K, dY, DEN, dV, nullptr, nullptr, nullptr, T, H, D, groups, eps);
+}
+
+// Per row r = (b, t, h), each [rows]: inv = 1 / max(||k||, 1e-6); 1 / den and
+// -(dy . y) / den of pass A (its own y and den) and of pass B (the caller's).
+struct BwdScalars {
+  float *inv, *invA, *ddenA, *invB, *ddenB;
+};
+
+template <int DMAX>
+__global__ void __launch_bounds__(192)
+attn_bwd_scalars_kernel(const float* __restrict__ K, const float* __restrict__ dY, const float* __restrict__ Yp,
+                        const float* __restrict__ Y, const float* __restrict__ DENp, const float* __restrict__ DEN,
+                        BwdScalars o, int64_t rows, int D) {
+  __shared__ float sm[4][64 * (DMAX + 1)];
+  const int64_t r0 = (int64_t)blockIdx.x * 64;
+  const int nr = (int)(rows - r0 < 64 ? rows - r0 : 64);
+  for (int e = threadIdx.x; e < nr * D; e += 192) {
+    const int r = e / D, j = e - r * D, d = r * (D + 1) + j;
+    const int64_t g = r0 * D + e;
+    sm[0][d] = K[g];
+    sm[1][d] = dY[g];
+    sm[2][d] = Yp[g];
+    sm[3][d] = Y[g];
+  }
+  __syncthreads();
+  const int what = threadIdx.x >> 6, r = threadIdx.x & 63;
+  if (r >= nr) return;
+  if (what == 0) {
+    o.inv[r0 + r] = attn_inv_norm(sm[0] + r * (D + 1), D);
+    return;
+  }
+  const float *dy = sm[1] + r * (D + 1), *y = sm[1 + what] + r * (D + 1);
+  float yd = 0.0f;
+  for (int j = 0; j < D; ++j) yd = yd + dy[j] * y[j];
+  const float inv = 1.0f / (what == 1 ? DENp : DEN)[r0 + r];
+  (what == 1 ? o.invA : o.invB)[r0 + r] = inv;
+  (what == 1 ? o.ddenA : o.ddenB)[r0 + r] = -yd * inv;
+}
+
+// dk = dk~ / nc - k (k . dk~) / nc^3 per row, dK holding dk~ (sums in double).
+template <int DMAX>
+__global__ void __launch_bounds__(256)
+attn_bwd_dk_kernel(const float* __restrict__ K, float* __restrict__ dK, int64_t rows, int D) {
+  __shared__ float sk[64 * (DMAX + 1)], st[64 * (DMAX + 1)];
+  __shared__ float s_inv[64], s_sc[64];
+  const int64_t r0 = (int64_t)blockIdx.x * 64;
+  const int nr = (int)(rows - r0 < 64 ? rows - r0 : 64);
+  for (int e = threadIdx.x; e < nr * D; e += 256) {
+    const int r = e / D, d = e + r;  // rows of D + 1
+    sk[d] = K[r0 * D + e];
+    st[d] = dK[r0 * D + e];
+  }
+  __syncthreads();
+  const int r = threadIdx.x;
+  if (r < nr) {
+    double n2 = 0.0, kd = 0.0;
+    for (int i = 0; i < D; ++i) {
+      const double ki = (double)sk[r * (D + 1) + i];
+      n2 = n2 + ki * ki;
+      kd = kd + ki * (double)st[r * (D + 1) + i];
+    }
+    const float n = (float)__builtin_sqrt(n2);
+    const float nc = (!__builtin_isfinite(n) || n < 1e-6f) ? 1e-6f : n;
+    float sc = (float)(kd / ((double)nc * nc * nc));
+    if (!__builtin_isfinite(sc)) sc = 0.0f;
+    s_sc[r] = sc;
+    s_inv[r] = 1.0f / nc;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < nr * D; e += 256) {
+    const int rr = e / D, d = e + rr;
+    dK[r0 * D + e] = st[d] * s_inv[rr] - sk[d] * s_sc[rr];
+  }
+}
+
+// The row passes: row i of the state belongs to 8 lanes, lane l of them to its
+// columns l, l + 8, ... (the 8 partial sums of dot8_lanes), M = D / 8 of them
+// in registers.  The partials are added left to right by moving the running
+// sum one lane on per tick (row_shr:1 on the add), so lane l works on step t =
+// tau - l and lane 7 finishes a step every tick.  Pass A: state S += kn (x) v,
+// dq = S dnum + dden z; pass B (REV, time backwards): Dm += q (x) dnum, dk~ =
+// Dm v + dz.  A workgroup is 4 computing waves (8 rows each) and one that
+// stages the next 16 steps into a ring of 64.
+//
+// What bounds it: LDS reads (4 of 16 bytes per tick and wave for M = 8, all
+// rows reading the same 8 lanes' columns) about level with the 4 M VALU
+// operations per tick, on 2 T / 256 workgroups a CU.
+constexpr int AR_W = 4, AR_NT = (AR_W + 1) * 64, AR_CH = 16, AR_RN = 64, AR_ROWS = AR_W * 8;
+
+template <int M>
+struct AttnRow {
+  static constexpr int DP = (8 * M + 63) / 64;  // columns of a staging lane
+  // b [l][m], c [l][m], a (the rows), dden; padded so that the 8 lanes' reads,
+  // one ring row apart, fall in different banks
+  static constexpr int RB = 16 * M + (M % 8 == 4 ? 40 : 36);
+  static constexpr int NB = M <= 8 ? 4 : 2;     // ticks whose operands are read together
+  __attribute__((aligned(16))) float row[AR_RN * RB];
+};
+
+template <int M>
+__device__ __forceinline__ void attn_read_cols(const float* p, float (&d)[M]) {
+  if constexpr (M % 4 == 0) {
+#pragma unroll
+    for (int m = 0; m < M; m += 4) {
+      const float4 w = *(const float4*)(p + m);
+      d[m] = w.x;
+      d[m + 1] = w.y;
+      d[m + 2] = w.z;
+      d[m + 3] = w.w;
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < M; m += 2) {
+      const float2 w = *(const float2*)(p + m);
+      d[m] = w.x;
+      d[m + 1] = w.y;
+    }
+  }
+}
+
+template <int M, bool REV>
+__device__ __forceinline__ void
+attn_row(AttnRow<M>& sm, const float* __restrict__ dY, const float* __restrict__ Q, const float* __restrict__ K,
+         const float* __restrict__ V, const BwdScalars& sc, float* __restrict__ out, int64_t T, int H, int groups) {
+  using L = AttnRow<M>;
+  constexpr int D = 8 * M, RB = L::RB, DP = L::DP, NB = L::NB, CH = AR_CH;
+  const int64_t task = blockIdx.x / groups;
+  const int i0 = (int)(blockIdx.x - task * groups) * AR_ROWS;
+  const int64_t b = task / H, h = task % H;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t hs = REV ? -H : H;                            // stride between steps, in rows of D
+  const int64_t base = (b * T + (REV ? T - 1 : 0)) * H + h;   // and the first one
+  const int64_t chunks = (T + 7 + CH - 1) / CH;
+
+  for (int e = tid; e < AR_RN * RB; e += AR_NT) sm.row[e] = 0.0f;
+
+  if (wave == AR_W) {
+    constexpr int AN = CH * AR_ROWS / 64;
+    const float* A = REV ? Q : K;
+    float sv[2][CH * DP], sg[2][CH * DP], sa[2][AN], s1[2], s2[2], s3[2];
+    uint32_t col[DP];
+#pragma unroll
+    for (int p = 0; p < DP; ++p) col[p] = lane + 64 * p < D ? lane + 64 * p : D - 1;
+    const int ai = i0 + (lane & 31) < D ? i0 + (lane & 31) : D - 1;
+    auto load = [&](auto set, int64_t c) {
+      const int64_t left = T - c * CH;
+      const int64_t row = base + (left > 0 ? c * CH : 0) * hs;
+      int64_t o = row;
+#pragma unroll
+      for (int r = 0; r < CH; ++r) {  // steps past T: the last one again, cleared when staged
+#pragma unroll
+        for (int p = 0; p < DP; ++p) {
+          sv[set][r * DP + p] = V[o * D + col[p]];
+          sg[set][r * DP + p] = dY[o * D + col[p]];
+        }
+        o += r + 1 < left ? hs : 0;
+      }
+#pragma unroll
+      for (int n = 0; n < AN; ++n) {
+        const int r = 2 * n + (lane >> 5);
+        sa[set][n] = A[(row + (r < left ? r : 0) * hs) * D + ai];
+      }
+      const int64_t rr = row + ((lane & (CH - 1)) < left ? lane & (CH - 1) : 0) * hs;
+      s1[set] = REV ? sc.invB[rr] : sc.invA[rr];
+      s2[set] = REV ? sc.ddenB[rr] : sc.ddenA[rr];
+      if constexpr (!REV) s3[set] = sc.inv[rr];
+    };
+    auto stage = [&](auto set, int64_t c) {
+      const int64_t left = T - c * CH;
+      float* rows = sm.row + (int)(c % (AR_RN / CH)) * CH * RB;
+#pragma unroll
+      for (int r = 0; r < CH; ++r) {
+        const float invd = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s1[set]), r));
+#pragma unroll
+        for (int p = 0; p < DP; ++p) {
+          const int j = lane + 64 * p;
+          const float v = r < left ? sv[set][r * DP + p] : 0.0f;
+          const float dn = r < left ? sg[set][r * DP + p] * invd : 0.0f;
+          if (DP * 64 == D || j < D) {
+            rows[r * RB + (j & 7) * M + (j >> 3)] = REV ? dn : v;
+            rows[r * RB + 8 * M + (j & 7) * M + (j >> 3)] = REV ? v : dn;
+          }
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < AN; ++n) {
+        const int r = 2 * n + (lane >> 5);
+        float a = sa[set][n];
+        if constexpr (!REV) a = a * __shfl(s3[set], r, 64);
+        rows[r * RB + 16 * M + (lane & 31)] = r < left ? a : 0.0f;
+      }
+      if (lane < CH) rows[lane * RB + 16 * M + AR_ROWS] = lane < left ? s2[set] : 0.0f;
+    };
+    load(Set<0>(), 0);
+    load(Set<1>(), 1);
+    __syncthreads();
+    stage(Set<0>(), 0);
+    load(Set<0>(), 2);
+    __syncthreads();
+    for (int64_t c = 0; c < chunks; c += 2) {  // period c stages chunk c + 1
+      if (c + 1 < chunks) {
+        stage(Set<1>(), c + 1);
+        load(Set<1>(), c + 3);
+      }
+      __syncthreads();
+      if (c + 1 < chunks) {
+        if (c + 2 < chunks) {
+          stage(Set<0>(), c + 2);
+          load(Set<0>(), c + 4);
+        }
+        __syncthreads();
+      }
+    }
+    return;
+  }
+
+  const int l = lane & 7, ri = wave * 8 + (lane >> 3), i = i0 + ri;
+  float S[M], z = 0.0f, s = 0.0f;
+#pragma unroll
+  for (int m = 0; m < M; ++m) S[m] = 0.0f;
+  const bool writes = l == 7 && i < D;
+  float* op = out + (base - 7 * hs) * D + i;  // lane 7's step at tick 0 is -7
+  __syncthreads();
+  __syncthreads();
+  int64_t tau = 0;
+  for (int64_t c = 0; c < chunks; ++c) {
+    const int tick0 = (int)(c % (AR_RN / CH)) * CH;
+    float bb[2][NB][M], cc[2][NB][M], aa[2][NB], dd[2][NB];
+    auto fetch = [&](int set, int tt, int tick) {
+      const float* p = sm.row + ((tick0 + tick - l) & (AR_RN - 1)) * RB;
+      attn_read_cols<M>(p + l * M, bb[set][tt]);
+      attn_read_cols<M>(p + 8 * M + l * M, cc[set][tt]);
+      aa[set][tt] = p[16 * M + ri];
+      dd[set][tt] = p[16 * M + AR_ROWS];
+    };
+#pragma unroll
+    for (int tt = 0; tt < NB; ++tt) fetch(0, tt, tt);
+#pragma unroll
+    for (int tt0 = 0; tt0 < CH; tt0 += NB) {
+      const int g = (tt0 / NB) & 1;
+#pragma unroll
+      for (int tt = 0; tt < NB; ++tt) {
+        if (tt0 + NB < CH) fetch(g ^ 1, tt, tt0 + NB + tt);
+        const float a = aa[g][tt];
+        float acc = 0.0f;
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          S[m] = S[m] + a * bb[g][tt][m];
+          acc = acc + S[m] * cc[g][tt][m];
+        }
+        // lane 0 of the 8 starts the sum
+        const float before = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(s), 0x111, 0xf, 0xf, true));
+        s = l == 0 ? acc : before + acc;
+        float r;
+        if constexpr (REV) {
+          z = z + dd[g][tt] * a;
+          r = z + s;
+        } else {
+          z = z + a;
+          r = s + dd[g][tt] * z;
+        }
+        if (writes && tau >= 7 && tau < T + 7) *op = r;
+        op += hs * D;
+        ++tau;
+      }
+    }
+    __syncthreads();
+  }
+}
+
+template <int M>
+__global__ void __launch_bounds__(AR_NT)
+attn_bwd_row_kernel(const float* __restrict__ dY, const float* __restrict__ Q, const float* __restrict__ K,
+                    const float* __restrict__ V, BwdScalars sc, float* __restrict__ dQ, float* __restrict__ dK,
+                    int64_t T, int H, int groups) {
+  __shared__ AttnRow<M> sm;
+  if (blockIdx.y == 0)
+    attn_row<M, false>(sm, dY, Q, K, V, sc, dQ, T, H, groups);
+  else
+    attn_row<M, true>(sm, dY, Q, K, V, sc, dK, T, H, groups);
+}
+
+// Whether the four-launch backward takes a head width: whole 8-lane rows of a
+// width that is instantiated (the others run attn_bwd_kernel).
+bool attn_bwd_split(int64_t D) { return D == 16 || D == 32 || D == 48 || D == 64 || D == 96 || D == 128; }
+
+int attn_bwd_launch(const float* dY, const float* Q, const float* K, const float* V, const float* Y, const float* DEN,
+                    float* dQ, float* dK, float* dV, int64_t B, int64_t T, int64_t H, int64_t D, float eps, float* ws,
+                    hipStream_t stream) {
+  const int64_t rows = B * T * H;
+  const BwdScalars sc = {ws + rows, ws + 2 * rows, ws + 3 * rows, ws + 4 * rows, ws + 5 * rows};
+  const int j = attn_col_width(2 * B * H, D);
+  const int64_t groups = (D + AC_W * j - 1) / (AC_W * j);
+  auto col = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(B * H * groups), 2), dim3(AC_NT), 0, stream, dY, Q, K, V, DEN, dQ, ws,
+                       dV, T, (int)H, (int)D, (int)groups, eps);
+  };
+  if (D <= 64)
+    j == 2 ? col(attn_bwd_col_kernel<1, 2>) : j == 4 ? col(attn_bwd_col_kernel<1, 4>) : col(attn_bwd_col_kernel<1, 8>);
+  else
+    j == 2 ? col(attn_bwd_col_kernel<2, 2>) : j == 4 ? col(attn_bwd_col_kernel<2, 4>) : col(attn_bwd_col_kernel<2, 8>);
+  int rc = check_launch("attn_bwd_col_kernel");
+  if (rc) return rc;
+  const dim3 rgrid((unsigned)((rows + 63) / 64));
+  if (D <= 64)
+    hipLaunchKernelGGL((attn_bwd_scalars_kernel<64>), rgrid, dim3(192), 0, stream, K, dY, dQ, Y, ws, DEN, sc, rows,
+                       (int)D);
+  else
+    hipLaunchKernelGGL((attn_bwd_scalars_kernel<128>), rgrid, dim3(192), 0, stream, K, dY, dQ, Y, ws, DEN, sc, rows,
+                       (int)D);
+  rc = check_launch("attn_bwd_scalars_kernel");
+  if (rc) return rc;
+  const int64_t rgroups = (D + AR_ROWS - 1) / AR_ROWS;
+  auto row = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(B * H * rgroups), 2), dim3(AR_NT), 0, stream, dY, Q, K, V, sc, dQ, dK,
+                       T, (int)H, (int)rgroups);
+  };
+  switch (D) {
+    case 16: row(attn_bwd_row_kernel<2>); break;
+    case 32: row(attn_bwd_row_kernel<4>); break;
+    case 48: row(attn_bwd_row_kernel<6>); break;
+    case 64: row(attn_bwd_row_kernel<8>); break;
+    case 96: row(attn_bwd_row_kernel<12>); break;
+    default: row(attn_bwd_row_kernel<16>); break;
+  }
+  rc = check_launch("attn_bwd_row_kernel");
+  if (rc) return rc;
+  if (D <= 64)
+    hipLaunchKernelGGL((attn_bwd_dk_kernel<64>), rgrid, dim3(256), 0, stream, K, dK, rows, (int)D);
+  else
+    hipLaunchKernelGGL((attn_bwd_dk_kernel<128>), rgrid, dim3(256), 0, stream, K, dK, rows, (int)D);
+  return check_launch("attn_bwd_dk_kernel");
+}
+
 int check_attn_shape(int64_t B, int64_t T, int64_t H, int64_t D, float eps, const char* what) {
   if (B < 0 || T < 0 || H < 0 || D <= 0)
     return fail(SMAUL_ERR_INVALID, "%s: bad shape [%lld,%lld,%lld,%lld]", what, (long long)B, (long long)T,
@@ -576,6 +1085,12 @@ int64_t smaul_attn_workspace_size(int64_t B, int64_t H, int64_t D, int need_stat
   return B * H * D * D * (int64_t)sizeof(float);
 }
 
+int64_t smaul_attn_backward_workspace_size(int64_t B, int64_t T, int64_t H, int64_t D) {
+  if (B < 0 || T < 0 || H < 0 || D <= 0) return -1;
+  if (attn_bwd_split(D)) return 6 * B * T * H * (int64_t)sizeof(float);
+  return smaul_attn_workspace_size(B, H, D, 0);
+}
+
 int smaul_attn_forward(const float* Q, const float* K, const float* V, float* Y, float* DEN, float* S_out,
                        float* z_out, int64_t B, int64_t T, int64_t H, int64_t D, float eps, void* workspace,
                        int64_t workspace_bytes, hipStream_t stream) {
@@ -588,22 +1103,16 @@ int smaul_attn_forward(const float* Q, const float* K, const float* V, float* Y,
   const dim3 grid((unsigned)(B * H));
   if (D <= 128) {
     if (T == 0 && !S_out) return SMAUL_OK;  // T == 0 with a state: the kernel writes zeros
-    // Columns per wave: with 2 a tick is shorter (19 instructions against 27)
-    // but the shared ones are repeated more often, so it pays only while the
-    // narrower workgroups still find a CU each
-    const int64_t tasks = B * H;
-    const int64_t narrow = (D + AC_W * 2 - 1) / (AC_W * 2), wide = (D + AC_W * 4 - 1) / (AC_W * 4);
-    const bool two = tasks * narrow <= 256;
-    const int64_t groups = two ? narrow : wide;
-    const dim3 cgrid((unsigned)(tasks * groups));
+    const int j = attn_col_width(B * H, D);
+    const int64_t groups = (D + AC_W * j - 1) / (AC_W * j);
     auto go = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, cgrid, dim3(AC_NT), 0, stream, Q, K, V, Y, DEN, S_out, z_out, T, (int)H, (int)D,
-                         (int)groups, eps);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(B * H * groups)), dim3(AC_NT), 0, stream, Q, K, V, Y, DEN, S_out,
+                         z_out, T, (int)H, (int)D, (int)groups, eps);
     };
     if (D <= 64)
-      two ? go(attn_fwd_col_kernel<1, 2>) : go(attn_fwd_col_kernel<1, 4>);
+      j == 2 ? go(attn_fwd_col_kernel<1, 2>) : j == 4 ? go(attn_fwd_col_kernel<1, 4>) : go(attn_fwd_col_kernel<1, 8>);
     else
-      two ? go(attn_fwd_col_kernel<2, 2>) : go(attn_fwd_col_kernel<2, 4>);
+      j == 2 ? go(attn_fwd_col_kernel<2, 2>) : j == 4 ? go(attn_fwd_col_kernel<2, 4>) : go(attn_fwd_col_kernel<2, 8>);
     return check_launch("attn_fwd_col_kernel");
   }
   float* state = S_out;
@@ -639,6 +1148,8 @@ int smaul_attn_backward(const float* dY, const float* Q, const float* K, const f
   if (B == 0 || H == 0 || T == 0) return SMAUL_OK;
   if (!dY || !Q || !K || !V || !Y || !DEN || !dQ || !dK || !dV)
     return fail(SMAUL_ERR_INVALID, "attn_backward: null pointer");
+  if (attn_bwd_split(D) && workspace && workspace_bytes >= smaul_attn_backward_workspace_size(B, T, H, D))
+    return attn_bwd_launch(dY, Q, K, V, Y, DEN, dQ, dK, dV, B, T, H, D, eps, (float*)workspace, stream);
   const dim3 grid((unsigned)(B * H));
   if (D <= 64) {
     hipLaunchKernelGGL((attn_bwd_kernel<64, 16, 64, true>), grid, dim3(64), 0, stream, dY, Q, K, V, Y, DEN, dQ, dK,

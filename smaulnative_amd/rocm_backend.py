@@ -313,7 +313,7 @@ class RocmBackend:
         dYc, Qc, Kc, Vc, Yc, DENc = (t if t.is_contiguous() else t.contiguous() for t in (dY, Q, K, V, Y, DEN))
         dev = Q.device
         dQ, dK, dV = torch.empty_like(Qc), torch.empty_like(Qc), torch.empty_like(Qc)
-        ws_bytes = lib.smaul_attn_workspace_size(B, H, D, 0)
+        ws_bytes = lib.smaul_attn_backward_workspace_size(B, T, H, D)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
         with torch.cuda.device(dev):
             rc = lib.smaul_attn_backward(dYc.data_ptr(), Qc.data_ptr(), Kc.data_ptr(), Vc.data_ptr(), Yc.data_ptr(),

@@ -72,7 +72,8 @@ def test_attn_forward_bit_exact(B, T, H, D):
     # (one row a lane up to 64, two above, the odd one alone), steps about the
     # staged chunks (32 / 16) and the ring of 128, columns about a workgroup's
     (1, 31, 1, 63), (1, 33, 2, 65), (2, 130, 1, 64), (1, 129, 1, 127), (1, 16, 1, 100), (1, 161, 3, 9),
-    (8, 70, 8, 64), (4, 40, 16, 48), (5, 35, 16, 32), (3, 17, 8, 128),   # four columns a wave
+    (5, 70, 8, 64), (4, 40, 8, 48), (3, 17, 8, 128),    # four columns a wave
+    (9, 40, 8, 64), (8, 35, 17, 32), (5, 20, 8, 128),   # eight
 ])
 def test_attn_forward_array_edges(B, T, H, D):
     print(f"case attn_forward array B={B} T={T} H={H} D={D}", flush=True)
@@ -234,6 +235,35 @@ def test_attn_backward_bit_exact_vs_oracle(B, T, H, D, eps):
     got = be().attn_backward(*(t.to(DEV) for t in (dY, Q, K, V, Y, DEN)), eps)
     torch.cuda.synchronize()
     for name, a, r in zip(("dQ", "dK", "dV"), got, ref):
+        assert torch.equal(a.cpu(), r), name
+
+
+@pytest.mark.parametrize("B,T,H,D", [
+    # the split backward (D = 16, 32, 48, 64, 96, 128): steps about its staged
+    # chunks of 16 and 32, every width, 2 / 4 / 8 columns a wave in its first pass
+    (1, 1, 1, 64), (1, 15, 3, 16), (2, 33, 2, 32), (1, 70, 3, 48), (1, 17, 2, 96), (2, 129, 1, 128),
+    (3, 20, 8, 64), (5, 18, 8, 64), (3, 18, 4, 128), (3, 20, 6, 128),
+])
+def test_attn_backward_split_edges(B, T, H, D):
+    print(f"case attn_backward split B={B} T={T} H={H} D={D}", flush=True)
+    Q, K, V = attn_inputs(B, T, H, D, B * 3 + T * 11 + D)
+    K[0, T // 2, 0] = 0.0
+    Q[0, T // 3] = -Q[0, T // 3]   # den clamped to eps
+    dY = torch.randn(B, T, H, D, generator=torch.Generator().manual_seed(T + D))
+    Y, DEN, _, _ = oracle.attn_forward(Q, K, V)
+    Y = Y * 1.25                   # pass A takes its own y, pass B the caller's
+    ref = oracle.attn_backward(dY, Q, K, V, Y, DEN)
+    dev = [t.to(DEV) for t in (dY, Q, K, V, Y, DEN)]
+    got = be().attn_backward(*dev, 1e-6)
+    for name, a, r in zip(("dQ", "dK", "dV"), got, ref):
+        assert torch.equal(a.cpu(), r), name
+    # without a workspace: the one-kernel backward, the same bits
+    from smaulnative_amd import _lib
+    plain = [torch.empty_like(dev[0]) for _ in range(3)]
+    rc = _lib.load().smaul_attn_backward(*[t.data_ptr() for t in dev + plain], B, T, H, D, 1e-6, None, 0,
+                                         torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "attn_backward")
+    for name, a, r in zip(("dQ", "dK", "dV"), plain, ref):
         assert torch.equal(a.cpu(), r), name
 
 
