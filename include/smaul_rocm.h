@@ -440,6 +440,16 @@ int smaul_fp8_backward_input(const float* g, const uint8_t* w, const float* s, f
                              int64_t in_f, int64_t out_f, int64_t tile, hipStream_t stream);
 
 /*
+ * Weight gradient of the tiled-FP8 linear, added to its bf16 accumulator:
+ * gw[out_f, in_f] = bf16(gw + g^T x), the sums over the rows in fp32, one
+ * rounding (kernel/fp8_tile.py:172-197, which forms the same sums 64 output
+ * rows at a time).  g fp32 [rows, out_f], x [rows, in_f] fp32 or bf16, both
+ * row-major; fresh != 0 takes gw as zero without reading it.
+ */
+int smaul_fp8_weight_grad(const float* g, const void* x, int x_dtype, void* gw, int64_t rows, int64_t in_f,
+                          int64_t out_f, int fresh, hipStream_t stream);
+
+/*
  * Measured ceilings for the roofline figures (bench.py --peaks); no
  * counterpart in the reference and not on the MoE path.
  * smaul_peak_mfma: `workgroups` x 4 waves, each issuing `iters` rounds of 8

@@ -127,16 +127,26 @@ class _FP8Matmul(torch.autograd.Function):
         if m is not None:
             # the weight gradient accumulates in the module's bf16 _gw, which the
             # reference's optimizers read and clear (kernel/fp8_tile.py:172-197):
-            # each 64-row block of g^T x is formed in fp32 and rounded once
-            xr = x.reshape(-1, in_f).float()
+            # g^T x is formed in fp32 and rounded once, in one launch where the
+            # backend has the kernel, else in blocks of 64 rows
+            be = get_backend()
+            xr = x.reshape(-1, in_f)
             with _GW_LOCK:  # backward passes on several threads add to one _gw
-                if m._gw is None:
-                    m._gw = torch.zeros(out_f, in_f, dtype=GRAD_DTYPE, device=g.device)
-                elif m._gw.device != g.device:  # the module moved: keep what it accumulated
-                    m._gw = m._gw.to(g.device)
-                for o0 in range(0, out_f, _GRAD_ROWS):
-                    o1 = min(o0 + _GRAD_ROWS, out_f)
-                    m._gw[o0:o1].add_(g[:, o0:o1].t() @ xr)
+                fresh = m._gw is None
+                if fresh:
+                    gw = torch.empty(out_f, in_f, dtype=GRAD_DTYPE, device=g.device)
+                else:  # where the module moved, keep what it accumulated
+                    gw = m._gw if m._gw.device == g.device else m._gw.to(g.device)
+                if g.is_cuda and hasattr(be, "fp8_weight_grad") and gw.dtype == torch.bfloat16 and gw.is_contiguous():
+                    be.fp8_weight_grad(g, xr if xr.dtype == torch.bfloat16 else xr.float(), gw, fresh)
+                else:
+                    if fresh:
+                        gw.zero_()
+                    xr = xr.float()
+                    for o0 in range(0, out_f, _GRAD_ROWS):
+                        o1 = min(o0 + _GRAD_ROWS, out_f)
+                        gw[o0:o1].add_(g[:, o0:o1].t() @ xr)
+                m._gw = gw
         return gx, None, None, None, None, None, None
 
 

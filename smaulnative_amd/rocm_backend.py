@@ -194,6 +194,26 @@ class RocmBackend:
         _lib.check(rc, "fp8_backward_input")
         return dx
 
+    def fp8_weight_grad(self, g, x, gw, fresh=False):
+        """gw[out_f, in_f] (bf16, in place) += g[rows, out_f]^T . x[rows, in_f] on
+        the device, summed in fp32 and rounded once (kernel/fp8_tile.py:172-197).
+        ``fresh`` takes gw as zero without reading it."""
+        lib = _lib.load()
+        _need_device("fp8_weight_grad", g, x, gw)
+        if g.dtype != torch.float32 or x.dtype not in _ACT or gw.dtype != torch.bfloat16:
+            raise RuntimeError(f"fp8_weight_grad: expected dtypes f32/(f32|bf16)/bf16, got "
+                               f"{g.dtype}/{x.dtype}/{gw.dtype}")
+        if gw.dim() != 2 or tuple(g.shape) != (x.shape[0], gw.shape[0]) or x.dim() != 2 or x.shape[1] != gw.shape[1]:
+            raise RuntimeError(f"fp8_weight_grad: g [rows, out_f], x [rows, in_f] and gw [out_f, in_f] expected, got "
+                               f"{tuple(g.shape)}, {tuple(x.shape)}, {tuple(gw.shape)}")
+        if not gw.is_contiguous():
+            raise RuntimeError("fp8_weight_grad: gw must be contiguous (it is updated in place)")
+        gc, xc = (t if t.is_contiguous() else t.contiguous() for t in (g, x))
+        with torch.cuda.device(g.device):
+            rc = lib.smaul_fp8_weight_grad(gc.data_ptr(), xc.data_ptr(), _ACT[x.dtype], gw.data_ptr(), x.shape[0],
+                                           x.shape[1], gw.shape[0], int(bool(fresh)), _stream_handle(g.device))
+        _lib.check(rc, "fp8_weight_grad")
+
     def fp8_quantize_tiles(self, w32, tile):
         """(codes uint8 [out_f, nt*tile], scales fp32 [out_f, nt], non-finite count) on the device.
 

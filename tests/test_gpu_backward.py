@@ -40,6 +40,31 @@ def test_backward_input_vs_oracle(rows, in_f, out_f, tile):
     assert rel_max(dx, ref) < 1e-5, rel_max(dx, ref)
 
 
+@pytest.mark.parametrize("rows,in_f,out_f,dtype", [
+    # rows about the kernel's chunks of 16 (four waves take every fourth) and
+    # outputs about its 64 x 64 tiles
+    (1, 64, 64, torch.float32), (15, 65, 63, torch.float32), (64, 1, 129, torch.bfloat16),
+    (129, 192, 100, torch.float32), (1000, 512, 320, torch.bfloat16), (0, 40, 24, torch.float32)])
+def test_weight_grad_vs_float64(rows, in_f, out_f, dtype):
+    """gw += g^T x in fp32, one rounding to bf16: against the float64 sum the
+    fp32 sum is within rows * 2^-24 * sum |g||x| (any order), and the rounding
+    within half a bf16 step: 8 significant bits, so 2^-8 of the result at most."""
+    print(f"case weight grad rows={rows} in_f={in_f} out_f={out_f} {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(rows + in_f + out_f)
+    g = torch.randn(rows, out_f, generator=gen)
+    x = torch.randn(rows, in_f, generator=gen).to(dtype)
+    gw = torch.randn(out_f, in_f, generator=gen).to(torch.bfloat16)
+    be = get_backend("rocm")
+    for fresh in (False, True):
+        got = gw.to(DEV)
+        be.fp8_weight_grad(g.to(DEV), x.to(DEV), got, fresh)
+        start = torch.zeros_like(gw) if fresh else gw
+        ref = start.double() + g.double().t() @ x.double()
+        slack = (rows + 1) * 2.0 ** -24 * (g.double().abs().t() @ x.double().abs() + start.double().abs())
+        bound = slack + (ref.abs() + slack) * 2.0 ** -8
+        assert bool(((got.cpu().double() - ref).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_fp8linear_training_step(dtype):
     from smaulnative_amd import FP8Linear
