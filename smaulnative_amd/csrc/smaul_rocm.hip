@@ -133,10 +133,9 @@ struct GemmArgs {
   int64_t R;
   int E;
   int tiled;                   // codes/scales in the tiled layout (SMAUL_FLAG_TILED_LAYOUT)
-  // Weight K blocks when the activations carry two K planes (the LDS-DMA
-  // GEMM of fp32 x split into bf16 hi and lo halves, K = 2 * kw): stage kt
-  // reads activation block kt and weight / scale block kt mod (kw / 64).
-  // 0: the weights span K.
+  // The weights' K when the activations carry two K planes (the LDS-DMA GEMM
+  // of fp32 x split into bf16 hi and lo halves side by side, K = 2 * kw, the
+  // ACT_PLANES kernels); 0: the weights span K.
   int64_t kw;
   // SwiGLU with fp32 output only: when > 0 the products are stored as their
   // bf16 hi / lo split (split_bf16), hi at y[row * ldy + col] and lo at
@@ -665,7 +664,11 @@ __device__ __forceinline__ void wait_vm() {
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 
-template <int BM, int BN, int WM, int WN, int NSTAGE, bool SWIGLU, bool X32 = false>
+// How the activations reach the LDS-DMA GEMM: bf16 rows; fp32 rows split in
+// LDS; or the bf16 hi and lo planes of fp32 rows, split beforehand.
+enum ActMode { ACT_BF16 = 0, ACT_X32 = 1, ACT_PLANES = 2 };
+
+template <int BM, int BN, int WM, int WN, int NSTAGE, bool SWIGLU, ActMode AM = ACT_BF16>
 struct DmaGemmCfg {
   static constexpr int NW = WM * WN;
   static constexpr int BNO = SWIGLU ? BN / 2 : BN;       // output columns per workgroup
@@ -673,9 +676,10 @@ struct DmaGemmCfg {
   static constexpr int TN = BN / WN;                     // staged weight columns per wave
   static constexpr int TNO = SWIGLU ? TN / 2 : TN;       // output columns per wave
   static constexpr int FM = TM / 32, FN = TN / 32, FNO = TNO / 32;
-  // X32: the activation rows arrive as fp32 (256 B per 64-wide K block) and
-  // are split in place into a bf16 hi plane and a lo plane of 128 B rows
-  static constexpr int A_BYTES = BM * 128 * (X32 ? 2 : 1), B_BYTES = BN * 64, S_BYTES = BN * 4;
+  // ACT_X32: the activation rows arrive as fp32 (256 B per 64-wide K block)
+  // and are split in place into a bf16 hi plane and a lo plane of 128 B rows;
+  // ACT_PLANES: the two planes arrive so
+  static constexpr int A_BYTES = BM * 128 * (AM != ACT_BF16 ? 2 : 1), B_BYTES = BN * 64, S_BYTES = BN * 4;
   static constexpr int STAGE = A_BYTES + B_BYTES + S_BYTES;
   static constexpr int A_INS = A_BYTES / 1024 / NW;      // 1 KB DMA instructions per wave per stage
   static constexpr int B_INS = B_BYTES / 1024 / NW;
@@ -708,13 +712,23 @@ struct DmaGemmCfg {
 // (split_bf16, |x - hi - lo| <= 2^-18 |x|) in two bf16 planes of the usual
 // layout; each k-step then runs hi and lo MFMAs into the same partial, so the
 // scale multiplies s * (hi . w + lo . w) per 64-wide K block.
+//
+// PLANES (OUT_F32 only): the same over planes split beforehand (SwiGLU FFN and
+// MoE layer with fp32 x, long fp8_forward calls): a stage brings the hi and lo
+// rows of one K block, so its codes are staged and decoded once for both and
+// one scale FMA serves the eight MFMAs of a partial.  (As two stages per
+// weight block, all hi blocks and then all lo, each had its own codes, decode
+// and FMAs, which keep the VALU as busy as the matrix cores.)
 template <int BM, int BN, int WM, int WN, int NSTAGE, bool SWIGLU, bool CANON, bool REMAP, bool OUT_F32 = false,
-          bool X32 = false>
-// Tiles of at most 128 x 128 staged columns fit three workgroups per CU.
-__global__ void __launch_bounds__(WM * WN * 64, (BM * BN <= 128 * 128 ? 3 : 2))
+          ActMode AM = ACT_BF16>
+// Tiles of at most 128 x 128 staged columns fit three workgroups per CU (two
+// with the two planes of 64 x 256).
+__global__ void __launch_bounds__(WM * WN * 64, (BM * BN <= 128 * 128 && (AM != ACT_PLANES || BM * BN <= 64 * 128) ? 3 : 2))
 fp8_gemm_dma_kernel(GemmArgs p) {
+  constexpr bool X32 = AM == ACT_X32, PLANES = AM == ACT_PLANES, TWO = X32 || PLANES;
   static_assert(!X32 || (OUT_F32 && !SWIGLU), "fp32 activations split in LDS are the fp8_forward path");
-  using C = DmaGemmCfg<BM, BN, WM, WN, NSTAGE, SWIGLU, X32>;
+  static_assert(!PLANES || OUT_F32, "planes are fp32 activations");
+  using C = DmaGemmCfg<BM, BN, WM, WN, NSTAGE, SWIGLU, AM>;
   constexpr int NW = C::NW, BNO = C::BNO, TM = C::TM, TN = C::TN, TNO = C::TNO, FM = C::FM, FN = C::FN,
                 FNO = C::FNO, A_BYTES = C::A_BYTES, B_BYTES = C::B_BYTES, STAGE = C::STAGE,
                 A_INS = C::A_INS, B_INS = C::B_INS, S_INS = C::S_INS;
@@ -778,11 +792,13 @@ fp8_gemm_dma_kernel(GemmArgs p) {
       const int64_t xr = p.row_idx ? (int64_t)p.row_idx[lr] : lr;
       a_off[a] = (uint32_t)(xr * p.ldx * 4 + (lane & 15) * 16);
     } else {
-      const int r = (wave * A_INS + a) * 8 + (lane >> 3);
+      // PLANES: the first half of the instructions are the hi rows, the other the lo rows
+      const int q = wave * A_INS + a, plane = PLANES && q >= BM / 8;
+      const int r = (q - plane * (BM / 8)) * 8 + (lane >> 3);
       const int c = (lane & 7) ^ swz_a(r);
       const int64_t lr = row0 + (r < rows_here ? r : rows_here - 1);
       const int64_t xr = p.row_idx ? (int64_t)p.row_idx[lr] : lr;
-      a_off[a] = (uint32_t)(xr * p.ldx * 2 + c * 16);
+      a_off[a] = (uint32_t)(xr * p.ldx * 2 + plane * p.kw * 2 + c * 16);
     }
   }
   // B instruction q stages weight columns 16q..16q+15 (64 B each).  The host
@@ -814,16 +830,14 @@ fp8_gemm_dma_kernel(GemmArgs p) {
   // per-lane offsets stay fixed.  Every wave issues DMA_MIN = A_INS + B_INS
   // loads per stage, waves < S_INS one more (the scales, issued first).
   const uint32_t lds0 = lds_offset(&smem[0]);
-  const int kwb = (int)(p.kw >> 6);  // weight K blocks of a two-plane activation (0: none)
   auto dma_stage = [&](int kt, int buf) {
     const uint32_t lbase = lds0 + (uint32_t)(buf * STAGE);
-    const int kb = kt >= kwb && kwb > 0 ? kt - kwb : kt;  // the weight block of activation block kt
-    if (S_INS == NW || wave < S_INS) dma4(s_src + kb * L.sk, s_off, lbase + A_BYTES + B_BYTES + wave * 256);
+    if (S_INS == NW || wave < S_INS) dma4(s_src + kt * L.sk, s_off, lbase + A_BYTES + B_BYTES + wave * 256);
     const char* xa = (const char*)p.x + kt * (X32 ? 256 : 128);
 #pragma unroll
     for (int a = 0; a < A_INS; ++a) dma16(xa, a_off[a], lbase + (wave * A_INS + a) * 1024);
 #pragma unroll
-    for (int b = 0; b < B_INS; ++b) dma16(b_src(b) + kb * L.wk, b_off, lbase + A_BYTES + (wave * B_INS + b) * 1024);
+    for (int b = 0; b < B_INS; ++b) dma16(b_src(b) + kt * L.wk, b_off, lbase + A_BYTES + (wave * B_INS + b) * 1024);
   };
 
   // ---- fragment addresses (fixed over K) -----------------------------------
@@ -891,11 +905,11 @@ fp8_gemm_dma_kernel(GemmArgs p) {
         bfr[j][ks] = __builtin_bit_cast(bf16x8_t, make_uint4(d[4 * ks], d[4 * ks + 1], d[4 * ks + 2], d[4 * ks + 3]));
     }
     bf16x8_t af[2][4];
-    bf16x8_t afl[X32 ? 2 : 1][4];  // X32: the lo plane, BM * 128 bytes after the hi plane
+    bf16x8_t afl[TWO ? 2 : 1][4];  // the lo plane, BM * 128 bytes after the hi plane
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       af[0][ks] = *(const bf16x8_t*)(base + a_addr[ks]);
-      if constexpr (X32) afl[0][ks] = *(const bf16x8_t*)(base + BM * 128 + a_addr[ks]);
+      if constexpr (TWO) afl[0][ks] = *(const bf16x8_t*)(base + BM * 128 + a_addr[ks]);
     }
     f32x16_t qp;
 #pragma unroll
@@ -905,7 +919,7 @@ fp8_gemm_dma_kernel(GemmArgs p) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
           af[(i + 1) & 1][ks] = *(const bf16x8_t*)(base + a_addr[ks] + (i + 1) * 32 * 128);
-          if constexpr (X32)
+          if constexpr (TWO)
             afl[(i + 1) & 1][ks] = *(const bf16x8_t*)(base + BM * 128 + a_addr[ks] + (i + 1) * 32 * 128);
         }
       }
@@ -916,7 +930,7 @@ fp8_gemm_dma_kernel(GemmArgs p) {
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
         q = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[i & 1][ks], bfr[j][ks], q, 0, 0, 0);
-        if constexpr (X32) q = __builtin_amdgcn_mfma_f32_32x32x16_bf16(afl[i & 1][ks], bfr[j][ks], q, 0, 0, 0);
+        if constexpr (TWO) q = __builtin_amdgcn_mfma_f32_32x32x16_bf16(afl[i & 1][ks], bfr[j][ks], q, 0, 0, 0);
         if (t > 0) {
 #pragma unroll
           for (int r = ks * 4; r < ks * 4 + 4; ++r) acc[pi][pj][r] = __builtin_fmaf(sc[pj], qp[r], acc[pi][pj][r]);
@@ -974,7 +988,7 @@ fp8_gemm_dma_kernel(GemmArgs p) {
   // Stages past the end re-load the last stage into a buffer nobody reads
   // again, so the loop body has no branch around its loads (a branch costs
   // registers and spills).
-  const int nk = (int)(K >> 6);
+  const int nk = (int)((PLANES ? p.kw : K) >> 6);
 #pragma unroll
   for (int s = 0; s + 1 < NSTAGE; ++s) dma_stage(s < nk ? s : nk - 1, s);
   int buf = 0, nbuf = NSTAGE - 1;
@@ -3903,14 +3917,14 @@ struct CfgDma32x128 {  // 32 rows x 128 outputs
   static constexpr int BM = 32, BN = 128, WM = 1, WN = 4, NSTAGE = 4;
 };
 
-template <class CF, bool SWIGLU, bool CANON, bool OUT_F32 = false, bool X32 = false>
+template <class CF, bool SWIGLU, bool CANON, bool OUT_F32 = false, ActMode AM = ACT_BF16>
 int launch_gemm_dma(const GemmArgs& a, int64_t m_tiles, hipStream_t stream) {
   constexpr int BNO = SWIGLU ? CF::BN / 2 : CF::BN;
   const int64_t n_tiles = (a.N + BNO - 1) / BNO;
   if (m_tiles <= 0 || n_tiles <= 0) return SMAUL_OK;
   if (m_tiles > 65535 || n_tiles > 65535) return fail(SMAUL_ERR_UNSUPPORTED, "gemm grid too large");
   hipLaunchKernelGGL(
-      (fp8_gemm_dma_kernel<CF::BM, CF::BN, CF::WM, CF::WN, CF::NSTAGE, SWIGLU, CANON, true, OUT_F32, X32>),
+      (fp8_gemm_dma_kernel<CF::BM, CF::BN, CF::WM, CF::WN, CF::NSTAGE, SWIGLU, CANON, true, OUT_F32, AM>),
       dim3((unsigned)n_tiles, (unsigned)m_tiles), dim3(CF::WM * CF::WN * 64), 0, stream, a);
   return check_launch("fp8_gemm_dma_kernel");
 }
@@ -3933,22 +3947,26 @@ int pick_dense_tile(bool swiglu, int64_t rows, int64_t N) {
   return tiles(64, 128) >= cus ? DT_64x128 : DT_32x128;
 }
 
-template <bool SWIGLU, bool CANON, bool OUT_F32, bool X32 = false>
+template <bool SWIGLU, bool CANON, bool OUT_F32, ActMode AM = ACT_BF16>
 int launch_dense_dma(const GemmArgs& a, int tile, hipStream_t stream) {
   const int64_t rows = a.R;
   switch (tile) {
     case DT_128x256:
-      return launch_gemm_dma<CfgDmaGU, SWIGLU, CANON, OUT_F32, X32>(a, (rows + 127) / 128, stream);
+      // two planes of 128 rows would leave one workgroup per CU: 64 rows
+      if constexpr (AM == ACT_PLANES)
+        return launch_gemm_dma<CfgDmaGU64, SWIGLU, CANON, OUT_F32, AM>(a, (rows + 63) / 64, stream);
+      else
+        return launch_gemm_dma<CfgDmaGU, SWIGLU, CANON, OUT_F32, AM>(a, (rows + 127) / 128, stream);
     case DT_64x256_GU:
-      if constexpr (SWIGLU) return launch_gemm_dma<CfgDmaGU64, SWIGLU, CANON, OUT_F32>(a, (rows + 63) / 64, stream);
+      if constexpr (SWIGLU) return launch_gemm_dma<CfgDmaGU64, SWIGLU, CANON, OUT_F32, AM>(a, (rows + 63) / 64, stream);
       break;
     case DT_64x128:
       if constexpr (!SWIGLU)
-        return launch_gemm_dma<CfgDma64x128, SWIGLU, CANON, OUT_F32, X32>(a, (rows + 63) / 64, stream);
+        return launch_gemm_dma<CfgDma64x128, SWIGLU, CANON, OUT_F32, AM>(a, (rows + 63) / 64, stream);
       break;
     case DT_32x128:
       if constexpr (!SWIGLU)
-        return launch_gemm_dma<CfgDma32x128, SWIGLU, CANON, OUT_F32, X32>(a, (rows + 31) / 32, stream);
+        return launch_gemm_dma<CfgDma32x128, SWIGLU, CANON, OUT_F32, AM>(a, (rows + 31) / 32, stream);
       break;
     default:
       break;
@@ -4065,8 +4083,8 @@ int smaul_fp8_linear(const void* x, int x_dtype, const uint8_t* w, const float* 
   // fp32 x, 64-wide tiles: the same kernel staging fp32 rows and splitting
   // them into bf16 hi / lo planes in LDS (X32)
   if (dt >= 0 && vec && x_dtype == SMAUL_DTYPE_F32 && x32_gemm_ok(a, rows))
-    return canon ? launch_dense_dma<false, true, true, true>(a, dt, stream)
-                 : launch_dense_dma<false, false, true, true>(a, dt, stream);
+    return canon ? launch_dense_dma<false, true, true, ACT_X32>(a, dt, stream)
+                 : launch_dense_dma<false, false, true, ACT_X32>(a, dt, stream);
   if (x_dtype == SMAUL_DTYPE_BF16) {
     const int64_t bm = small ? CfgSmall::BM : CfgBig::BM;
     const int64_t mt = (rows + bm - 1) / bm;
@@ -4114,7 +4132,7 @@ int launch_split_planes(const float* x, uint16_t* planes, int64_t rows, int64_t 
 // 64, shapes the DMA GEMM takes): the dense tile, else -1.
 int planes_tile(int x_dtype, const void* x, const uint8_t* w, int64_t rows, int64_t in_f, int64_t out_f,
                 int64_t tile, int flags) {
-  if (x_dtype != SMAUL_DTYPE_F32 || tile != 64 || rows <= 64 || in_f % 64 != 0) return -1;
+  if (x_dtype != SMAUL_DTYPE_F32 || tile != 64 || rows <= 64 || rows > DMA_SMALL_BM * 65535 || in_f % 64 != 0) return -1;
   if ((flags & SMAUL_FLAG_TILED_LAYOUT) || !aligned16(x) || !aligned16(w) || in_f % 16 != 0) return -1;
   return pick_dense_tile(false, rows, out_f);
 }
@@ -4162,7 +4180,8 @@ int smaul_fp8_linear_ws(const void* x, int x_dtype, const uint8_t* w, const floa
   const int rc = launch_split_planes((const float*)x, (uint16_t*)workspace, rows, in_f, stream);
   if (rc != SMAUL_OK) return rc;
   const bool canon = (flags & SMAUL_FLAG_CANONICAL_CODES) != 0;
-  return canon ? launch_dense_dma<false, true, true>(a, dt, stream) : launch_dense_dma<false, false, true>(a, dt, stream);
+  return canon ? launch_dense_dma<false, true, true, ACT_PLANES>(a, dt, stream)
+               : launch_dense_dma<false, false, true, ACT_PLANES>(a, dt, stream);
 }
 
 // router launch shape for E experts: (tokens per wave, expert register width)
@@ -4539,7 +4558,7 @@ static int dense_gemm(bool swiglu, const void* act, int act_dtype, const uint8_t
 static int swiffn_f32_planes(const float* x, const uint8_t* gw, const float* gs, const uint8_t* uw, const float* us,
                              const uint8_t* dw, const float* ds, float* out, char* ws, int64_t hdn_bytes,
                              int64_t rows, int64_t d, int64_t h, int64_t tile, int flags, hipStream_t stream) {
-  if (tile != 64 || d % 128 != 0 || h % 128 != 0 || d > h || rows <= 64) return -1;
+  if (tile != 64 || d % 128 != 0 || h % 128 != 0 || d > h || rows <= 64 || rows > DMA_SMALL_BM * 65535) return -1;
   uint16_t* xplanes = (uint16_t*)ws;
   uint16_t* hplanes = (uint16_t*)(ws + hdn_bytes);
   GemmArgs a{};
@@ -4582,9 +4601,11 @@ static int swiffn_f32_planes(const float* x, const uint8_t* gw, const float* gs,
   const bool canon = (flags & SMAUL_FLAG_CANONICAL_CODES) != 0;
   int rc = launch_split_planes(x, xplanes, rows, d, stream);
   if (rc != SMAUL_OK) return rc;
-  rc = canon ? launch_dense_dma<true, true, true>(a, dtg, stream) : launch_dense_dma<true, false, true>(a, dtg, stream);
+  rc = canon ? launch_dense_dma<true, true, true, ACT_PLANES>(a, dtg, stream)
+             : launch_dense_dma<true, false, true, ACT_PLANES>(a, dtg, stream);
   if (rc != SMAUL_OK) return rc;
-  return canon ? launch_dense_dma<false, true, true>(b, dtd, stream) : launch_dense_dma<false, false, true>(b, dtd, stream);
+  return canon ? launch_dense_dma<false, true, true, ACT_PLANES>(b, dtd, stream)
+               : launch_dense_dma<false, false, true, ACT_PLANES>(b, dtd, stream);
 }
 
 int smaul_swiffn_forward(const void* x, int act_dtype, const uint8_t* gate_w8, const float* gate_s,
@@ -4800,18 +4821,14 @@ __global__ void wait_timeouts_kernel(int32_t* out, int reset) {
   if (reset) __hip_atomic_fetch_sub(&g_wait_timeouts, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// fp32 activations through the LDS-DMA grouped GEMMs: the tile rows (128,
-// or 64 where a 128-row gate+up grid is under four workgroups per CU, as for
-// bf16) when the shapes fit (tile 64, d and h multiples of 128, codes
-// promised 16-byte aligned, the kernels' 32-bit offsets for the planes of x
-// and of hdn), else 0.
-static int64_t f32_planes_block_m(int64_t T, int64_t d, int64_t h, int64_t E, int64_t k, int64_t tile, int flags,
-                                  int64_t R, int cus) {
-  if (tile != 64 || d % 128 != 0 || h % 128 != 0 || !(flags & SMAUL_FLAG_ALIGNED_CODES)) return 0;
+// Whether fp32 activations run the LDS-DMA grouped GEMMs over planes, on
+// 64-row tiles: tile 64, d and h multiples of 128, codes promised 16-byte
+// aligned, the kernels' 32-bit offsets for the planes of x and of hdn.
+static bool f32_planes_ok(int64_t T, int64_t d, int64_t h, int64_t E, int64_t tile, int flags, int64_t R) {
+  if (tile != 64 || d % 128 != 0 || h % 128 != 0 || !(flags & SMAUL_FLAG_ALIGNED_CODES)) return false;
   const int64_t lim = (int64_t)1 << 31;
-  const int64_t hrows = ((R + CfgBig::BM - 1) / CfgBig::BM + E) * CfgBig::BM;  // >= the rows either tiling indexes
-  if (T * d * 4 >= lim || hrows * h * 4 >= lim || 2 * h * d >= lim) return 0;
-  return ((R + CfgBig::BM - 1) / CfgBig::BM + E) * (h / 128) < 4 * (int64_t)cus ? DMA_SMALL_BM : CfgBig::BM;
+  const int64_t hrows = ((R + CfgBig::BM - 1) / CfgBig::BM + E) * CfgBig::BM;  // >= the rows the tiling indexes
+  return T * d * 4 < lim && hrows * h * 4 < lim && 2 * h * d < lim;
 }
 
 // The grouped gate+up and down of fp32 x (after the dispatch, on the tile
@@ -4866,21 +4883,15 @@ static int moe_f32_planes(const float* x, uint16_t* xplanes, const int32_t* perm
   const bool canon = (flags & SMAUL_FLAG_CANONICAL_CODES) != 0;
   int rc = launch_split_planes(x, xplanes, T, d, stream);
   if (rc != SMAUL_OK) return rc;
-  if (bm == DMA_SMALL_BM) {
-    rc = canon ? launch_gemm_dma<CfgDmaGU64, true, true, true>(g, max_tiles, stream)
-               : launch_gemm_dma<CfgDmaGU64, true, false, true>(g, max_tiles, stream);
-    if (rc != SMAUL_OK) return rc;
-    return canon ? launch_gemm_dma<CfgDma64x128, false, true, true>(dn, max_tiles, stream)
-                 : launch_gemm_dma<CfgDma64x128, false, false, true>(dn, max_tiles, stream);
-  }
-  rc = canon ? launch_gemm_dma<CfgDmaGU, true, true, true>(g, max_tiles, stream)
-             : launch_gemm_dma<CfgDmaGU, true, false, true>(g, max_tiles, stream);
+  rc = canon ? launch_gemm_dma<CfgDmaGU64, true, true, true, ACT_PLANES>(g, max_tiles, stream)
+             : launch_gemm_dma<CfgDmaGU64, true, false, true, ACT_PLANES>(g, max_tiles, stream);
   if (rc != SMAUL_OK) return rc;
-  if (d % CfgDmaDown::BN != 0 || max_tiles * (d / CfgDmaDown::BN) < 8 * (int64_t)cu_count())
-    return canon ? launch_gemm_dma<CfgDmaDownN, false, true, true>(dn, max_tiles, stream)
-                 : launch_gemm_dma<CfgDmaDownN, false, false, true>(dn, max_tiles, stream);
-  return canon ? launch_gemm_dma<CfgDmaDown, false, true, true>(dn, max_tiles, stream)
-               : launch_gemm_dma<CfgDmaDown, false, false, true>(dn, max_tiles, stream);
+  // down: 64 x 256 where its grid is more than two rounds of two per CU
+  if (d % CfgDmaGU64::BN == 0 && max_tiles * (d / CfgDmaGU64::BN) >= 4 * (int64_t)cu_count())
+    return canon ? launch_gemm_dma<CfgDmaGU64, false, true, true, ACT_PLANES>(dn, max_tiles, stream)
+                 : launch_gemm_dma<CfgDmaGU64, false, false, true, ACT_PLANES>(dn, max_tiles, stream);
+  return canon ? launch_gemm_dma<CfgDma64x128, false, true, true, ACT_PLANES>(dn, max_tiles, stream)
+               : launch_gemm_dma<CfgDma64x128, false, false, true, ACT_PLANES>(dn, max_tiles, stream);
 }
 
 static int moe_forward_impl(const void* x, int act_dtype, const float* gate_w, const float* gate_b,
@@ -4930,12 +4941,10 @@ static int moe_forward_impl(const void* x, int act_dtype, const float* gate_w, c
   uint16_t* xplanes = act_dtype == SMAUL_DTYPE_F32 ? (uint16_t*)ws : nullptr;
 
   int64_t bm = pick_block_m(T, d, h, E, k, tile, act_dtype);
-  // fp32 x on the LDS-DMA kernels over bf16 hi / lo planes (128- or 64-row
-  // tiles, by the same grid rule as bf16), else the register-staged kernels
-  const int64_t f32p_bm = act_dtype == SMAUL_DTYPE_F32
-                              ? f32_planes_block_m(T, d, h, E, k, tile, flags, R, cu_count())
-                              : 0;
-  if (f32p_bm) bm = f32p_bm;
+  // fp32 x on the LDS-DMA kernels over bf16 hi / lo planes, else the
+  // register-staged kernels
+  const bool planes = act_dtype == SMAUL_DTYPE_F32 && f32_planes_ok(T, d, h, E, tile, flags, R);
+  if (planes) bm = DMA_SMALL_BM;
   if (bm == CfgBig::BM && act_dtype == SMAUL_DTYPE_BF16 &&
       ((R + CfgBig::BM - 1) / CfgBig::BM + E) * (h / 128) < 4 * (int64_t)cu_count()) {
     // a 128-row gate/up grid under four workgroups per CU: 64-row tiles
@@ -5078,7 +5087,7 @@ static int moe_forward_impl(const void* x, int act_dtype, const float* gate_w, c
                              T, E, k, bm, route_tpb(T, E, d, act_dtype), stream);
     if (rc) return rc;
   }
-  if (f32p_bm) {
+  if (planes) {
     rc = moe_f32_planes((const float*)x, xplanes, perm_row, gate_w8, gate_s, up_w8, up_s, down_w8, down_s,
                         (uint16_t*)hdn, (float*)yperm, seg_off, tile_off, max_tiles, T, d, h, E, bm, flags, stream);
   } else {
