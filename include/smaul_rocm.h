@@ -79,11 +79,17 @@ int smaul_fp8_linear(const void* x, int x_dtype, const uint8_t* w, const float* 
  * in LDS inside the GEMM (tile 64, in_f a multiple of 64, out_f a multiple of
  * 128, more than 64 rows, 16-byte aligned x and w); for more than 1024 rows
  * this entry instead writes the two planes into the workspace in a separate
- * pass and runs the GEMM over both (faster for long calls).  With fewer rows,
- * other shapes, or a workspace smaller than smaul_fp8_linear_workspace_size
- * (0 below 1025 rows or for bf16 x), it is smaul_fp8_linear.  Same arguments,
- * results and errors as smaul_fp8_linear within fp32 summation order.
+ * pass and runs the GEMM over both (faster for long calls).  With more than 64
+ * rows, the shapes that GEMM does not take as they are (x or w unaligned,
+ * other widths, scale tiles of 32 or 128 and more) are packed into the
+ * workspace in the form it reads.  With a workspace smaller than
+ * smaul_fp8_linear_workspace says for the call, it is smaul_fp8_linear (the
+ * planes alone need smaul_fp8_linear_workspace_size).  Same arguments, results
+ * and errors as smaul_fp8_linear within fp32 summation order.  The packed path
+ * needs a 256-byte aligned workspace, the planes 16.
  */
+int64_t smaul_fp8_linear_workspace(const void* x, int x_dtype, const uint8_t* w, int64_t rows, int64_t in_f,
+                                   int64_t out_f, int64_t tile);
 int64_t smaul_fp8_linear_workspace_size(int64_t rows, int64_t in_f, int x_dtype);
 int smaul_fp8_linear_ws(const void* x, int x_dtype, const uint8_t* w, const float* s,
                         void* y, int y_dtype, int64_t rows, int64_t in_f, int64_t out_f,

@@ -142,6 +142,8 @@ struct GemmArgs {
   // y[row * ldy + y_lo + col] (bf16 elements): the two planes the next GEMM
   // of fp32 activations reads.
   int64_t y_lo;
+  // Dense fp32 output only: columns stored, when N is padded past them (0: N).
+  int64_t n_out;
 };
 
 // Where an expert's codes and scales for column n and 64-wide K block kb
@@ -1009,17 +1011,21 @@ fp8_gemm_dma_kernel(GemmArgs p) {
     // tile j (gate) and tile j + FNO (up) hold the same output columns; split
     // into planes (y_lo > 0), the register epilogue below stores them.
     if (!SWIGLU || p.y_lo == 0) {  // uniform
+      const int64_t n_out = p.n_out ? p.n_out : p.N;
 #pragma unroll
       for (int i = 0; i < FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FNO; ++j)
+        for (int j = 0; j < FNO; ++j) {
+          const int64_t col = n0 + wn * TNO + j * 32 + l32;
+          if (col >= n_out) continue;
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
             const int lr = wm * TM + i * 32 + (r >> 2) * 8 + g * 4 + (r & 3);
             float v = acc[i][j][r];
             if constexpr (SWIGLU) v = silu_f(v) * acc[i][j + FNO][r];
-            if (lr < rows_here) ((float*)p.y)[(int64_t)(row0 + lr) * p.ldy + n0 + wn * TNO + j * 32 + l32] = v;
+            if (lr < rows_here) ((float*)p.y)[(int64_t)(row0 + lr) * p.ldy + col] = v;
           }
+        }
       return;
     }
   }
@@ -4139,6 +4145,180 @@ int planes_tile(int x_dtype, const void* x, const uint8_t* w, int64_t rows, int6
 
 }  // namespace
 
+namespace {
+
+// ---- fp8_linear for shapes the LDS-DMA GEMM does not take as they are --------
+// (in_f not a multiple of 64, out_f not of 128, scale tiles other than 64,
+// unaligned rows).  One pass rewrites the call's operands into a workspace the
+// way that GEMM reads them, zero-padded: x as rows of bf16 (its hi and lo
+// planes side by side for fp32), the codes canonical in the tiled layout and
+// one scale per 64-wide K block (a wider tile's scale repeated).  Tiles of 32
+// make a block of their 32 k twice: [hi | lo] of x against [w | w], so hi . w
+// and lo . w share the tile's scale (bf16: [x | 0]).
+//
+// What bounds it: at 3001 x 1000 -> 777 two launches and the K loop of one
+// round of tiles (35 us; the register-staged GEMM, which loads unaligned rows
+// a byte at a time, 124 us); at 16000 x 2000 -> 2000, tile 128, the GEMM
+// (318 against 749 us).
+struct LinPack {
+  const void* x;
+  const uint8_t* w;
+  const float* s;
+  uint16_t* xp;
+  uint8_t* wp;
+  float* sp;
+  int64_t rows, in_f, out_f, tile, nt;
+  int64_t nb, np, ldx;   // 64-wide K blocks, padded columns, packed row (0: x is read in place)
+  int f32;
+};
+
+// out: what the GEMM reads, offsets from the workspace; returns its bytes
+int64_t lin_pack_shape(LinPack& p, const void* x, int x_dtype, int64_t rows, int64_t in_f, int64_t out_f,
+                       int64_t tile, int64_t* w_off, int64_t* s_off) {
+  const bool t32 = tile == 32;
+  p.rows = rows;
+  p.in_f = in_f;
+  p.out_f = out_f;
+  p.tile = tile;
+  p.nt = (in_f + tile - 1) / tile;
+  p.nb = t32 ? p.nt : (in_f + 63) / 64;
+  p.np = (out_f + 127) / 128 * 128;
+  p.f32 = x_dtype == SMAUL_DTYPE_F32;
+  const bool in_place = !p.f32 && !t32 && in_f % 64 == 0 && aligned16(x);
+  p.ldx = in_place ? 0 : p.nb * 64 * (p.f32 && !t32 ? 2 : 1);
+  *w_off = align256(rows * p.ldx * 2);
+  *s_off = *w_off + align256(p.nb * p.np * 64);
+  return *s_off + align256(p.nb * p.np * 4);
+}
+
+__global__ void __launch_bounds__(256) lin_pack_kernel(LinPack p, int64_t xblocks, int64_t wblocks) {
+  const bool t32 = p.tile == 32;
+  int64_t b = blockIdx.x;
+  if (b < xblocks) {  // a thread: 8 values of a row
+    const int64_t per_row = t32 ? p.nb * 4 : p.nb * 8;
+    const int64_t u = b * 256 + threadIdx.x;
+    if (u >= p.rows * per_row) return;
+    const int64_t r = u / per_row, c = u - r * per_row, k0 = c * 8;
+    uint32_t h[8], l[8];
+    const int64_t left = p.in_f - k0;
+    if (p.f32) {
+      const float* x = (const float*)p.x + r * p.in_f + k0;
+      float v[8];
+      if (left >= 8 && ((uintptr_t)x & 15) == 0) {
+        const float4 v0 = *(const float4*)x, v1 = *(const float4*)(x + 4);
+        v[0] = v0.x, v[1] = v0.y, v[2] = v0.z, v[3] = v0.w;
+        v[4] = v1.x, v[5] = v1.y, v[6] = v1.z, v[7] = v1.w;
+      } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = q < left ? x[q] : 0.0f;
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) split_bf16(v[q], h[q], l[q]);
+    } else {
+      const uint16_t* x = (const uint16_t*)p.x + r * p.in_f + k0;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        h[q] = q < left ? x[q] : 0u;
+        l[q] = 0u;
+      }
+    }
+    uint16_t* o = p.xp + r * p.ldx + (t32 ? (c >> 2) * 64 + (c & 3) * 8 : k0);
+    *(uint4*)o = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
+    if (p.f32 || t32)
+      *(uint4*)(o + (t32 ? 32 : p.nb * 64)) =
+          make_uint4(l[0] | (l[1] << 16), l[2] | (l[3] << 16), l[4] | (l[5] << 16), l[6] | (l[7] << 16));
+    return;
+  }
+  b -= xblocks;
+  if (b < wblocks) {  // a thread: 16 codes of a column's block
+    const int64_t u = b * 256 + threadIdx.x;
+    if (u >= p.nb * p.np * 4) return;
+    const int64_t ch = u & 3, kb = (u >> 2) / p.np, n = (u >> 2) - kb * p.np;
+    const int64_t k0 = t32 ? kb * 32 + (ch & 1) * 16 : kb * 64 + ch * 16;
+    const int64_t left = n < p.out_f ? p.in_f - k0 : 0;
+    uint32_t d[4] = {0u, 0u, 0u, 0u};
+    const uint8_t* w = p.w + n * p.in_f + k0;
+    if (left >= 16 && ((uintptr_t)w & 3) == 0) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) d[q] = ((const uint32_t*)w)[q];
+    } else {
+#pragma unroll
+      for (int q = 0; q < 16; ++q) d[q >> 2] |= (q < left ? (uint32_t)w[q] : 0u) << (8 * (q & 3));
+    }
+    *(uint4*)(p.wp + u * 16) = make_uint4(canon4(d[0]), canon4(d[1]), canon4(d[2]), canon4(d[3]));
+    return;
+  }
+  const int64_t u = (b - wblocks) * 256 + threadIdx.x;
+  if (u >= p.nb * p.np) return;
+  const int64_t kb = u / p.np, n = u - kb * p.np;
+  p.sp[u] = n < p.out_f ? p.s[n * p.nt + (t32 ? kb : kb * 64 / p.tile)] : 0.0f;
+}
+
+// Whether a call takes the packed path: not what smaul_fp8_linear's LDS-DMA
+// instances read in place, more rows than the small tile's, 32-bit offsets,
+// and enough K stages.  The register-staged GEMM takes about 7 us per 64-wide
+// stage on unaligned rows, 3.2 on aligned fp32 and 1.6 on aligned bf16, the
+// packed one 0.7 to 0.9 after 10 us of a second launch and of the caller's
+// workspace, so the line lies at 3, 6 and 12 stages: 3001 x 1000 -> 777, tile
+// 32, fp32 124 against 35 us (16 stages); 16000 x 150 -> 130 24.4 against 20.8
+// (3), 300 x 101 -> 150 16.1 against 18.3 (2); aligned: 100 x 512 -> 512, tile
+// 128, fp32 27.4 against 18.2 (8), bf16 14.9 against 18.4 (8), 300 x 1024 ->
+// 1024 bf16 23.5 against 19.4 (16).  Tiles of 32 in bf16 leave half of every
+// packed block empty: 3001 x 1024 -> 768 24.7 against 34.6, so aligned ones stay.
+bool lin_pack_ok(const void* x, int x_dtype, const uint8_t* w, int64_t rows, int64_t in_f, int64_t out_f,
+                 int64_t tile) {
+  if (rows <= 64 || rows > 32 * 65535 || kmode_of(tile) < 0) return false;
+  const bool f32 = x_dtype == SMAUL_DTYPE_F32, vec = in_f % 16 == 0 && aligned16(x) && aligned16(w);
+  if (tile == 64 && in_f % 64 == 0 && out_f % 128 == 0 && vec) return false;
+  if (vec && !f32 && tile == 32) return false;
+  if ((in_f + 63) / 64 < (!vec ? 3 : f32 ? 6 : 12)) return false;
+  LinPack p{};
+  int64_t wo, so;
+  lin_pack_shape(p, x, x_dtype, rows, in_f, out_f, tile, &wo, &so);
+  const int64_t lim = (int64_t)1 << 31, ldx = p.ldx ? p.ldx : in_f;
+  return rows * ldx * 2 < lim && p.nb * p.np * 64 < lim;
+}
+
+int lin_pack_launch(const void* x, int x_dtype, const uint8_t* w, const float* s, float* y, int64_t rows,
+                    int64_t in_f, int64_t out_f, int64_t tile, char* ws, hipStream_t stream) {
+  LinPack p{};
+  int64_t wo, so;
+  lin_pack_shape(p, x, x_dtype, rows, in_f, out_f, tile, &wo, &so);
+  p.x = x;
+  p.w = w;
+  p.s = s;
+  p.xp = (uint16_t*)ws;
+  p.wp = (uint8_t*)(ws + wo);
+  p.sp = (float*)(ws + so);
+  const int64_t xb = p.ldx ? (rows * p.nb * (tile == 32 ? 4 : 8) + 255) / 256 : 0;
+  const int64_t wb = (p.nb * p.np * 4 + 255) / 256, sb = (p.nb * p.np + 255) / 256;
+  hipLaunchKernelGGL(lin_pack_kernel, dim3((unsigned)(xb + wb + sb)), dim3(256), 0, stream, p, xb, wb);
+  const int rc = check_launch("lin_pack_kernel");
+  if (rc != SMAUL_OK) return rc;
+  const bool planes = p.f32 && tile != 32;
+  GemmArgs a{};
+  a.x = p.ldx ? (const void*)p.xp : x;
+  a.ldx = p.ldx ? p.ldx : in_f;
+  a.w = p.wp;
+  a.s = p.sp;
+  a.y = y;
+  a.ldy = out_f;
+  a.n_out = out_f;
+  a.kw = planes ? p.nb * 64 : 0;
+  a.K = planes ? 2 * a.kw : p.nb * 64;
+  a.N = p.np;
+  a.nt = p.nb;
+  a.tile = 64;
+  a.R = rows;
+  a.E = 1;
+  a.tiled = 1;
+  const int dt = pick_dense_tile(false, rows, p.np);
+  return planes ? launch_dense_dma<false, true, true, ACT_PLANES>(a, dt, stream)
+                : launch_dense_dma<false, true, true>(a, dt, stream);
+}
+
+}  // namespace
+
 // Up to this many rows, fp32 x takes smaul_fp8_linear's in-LDS split (X32)
 // rather than the planes pass: a separate launch costs more than it saves on
 // short calls (C-ABI timings: 512 x 512 -> 1536 12.6 vs 16.4 us, 300 x 256 ->
@@ -4151,12 +4331,28 @@ int64_t smaul_fp8_linear_workspace_size(int64_t rows, int64_t in_f, int x_dtype)
   return (x_dtype == SMAUL_DTYPE_F32 && rows >= PLANES_MIN_ROWS) ? rows * in_f * 4 : 0;
 }
 
+int64_t smaul_fp8_linear_workspace(const void* x, int x_dtype, const uint8_t* w, int64_t rows, int64_t in_f,
+                                   int64_t out_f, int64_t tile) {
+  if (rows < 0 || in_f <= 0 || out_f <= 0 || tile <= 0 || !dtype_ok(x_dtype)) return -1;
+  if (rows >= PLANES_MIN_ROWS && planes_tile(x_dtype, x, w, rows, in_f, out_f, tile, 0) >= 0)
+    return smaul_fp8_linear_workspace_size(rows, in_f, x_dtype);
+  if (!lin_pack_ok(x, x_dtype, w, rows, in_f, out_f, tile)) return 0;
+  LinPack p{};
+  int64_t wo, so;
+  return lin_pack_shape(p, x, x_dtype, rows, in_f, out_f, tile, &wo, &so);
+}
+
 int smaul_fp8_linear_ws(const void* x, int x_dtype, const uint8_t* w, const float* s, void* y, int y_dtype,
                         int64_t rows, int64_t in_f, int64_t out_f, int64_t tile, int flags, void* workspace,
                         int64_t workspace_bytes, hipStream_t stream) {
   const int dt = (rows >= PLANES_MIN_ROWS && y && s && y_dtype == SMAUL_DTYPE_F32 && kmode_of(tile) >= 0)
                      ? planes_tile(x_dtype, x, w, rows, in_f, out_f, tile, flags)
                      : -1;
+  if (dt < 0 && workspace && ((uintptr_t)workspace & 255) == 0 && x && w && s && y && tile > 0 && in_f > 0 &&
+      out_f > 0 && dtype_ok(x_dtype) && y_dtype == SMAUL_DTYPE_F32 && !(flags & SMAUL_FLAG_TILED_LAYOUT) &&
+      lin_pack_ok(x, x_dtype, w, rows, in_f, out_f, tile) &&
+      workspace_bytes >= smaul_fp8_linear_workspace(x, x_dtype, w, rows, in_f, out_f, tile))
+    return lin_pack_launch(x, x_dtype, w, s, (float*)y, rows, in_f, out_f, tile, (char*)workspace, stream);
   if (dt < 0 || !workspace || !aligned16(workspace) ||
       workspace_bytes < smaul_fp8_linear_workspace_size(rows, in_f, x_dtype))
     return smaul_fp8_linear(x, x_dtype, w, s, y, y_dtype, rows, in_f, out_f, tile, flags, stream);

@@ -166,6 +166,39 @@ def test_fp8_linear_fp32_two_planes(rows, in_f, out_f, tile):
     assert rel_max(y[idx], ref) < 1e-5, rel_max(y[idx], ref)
 
 
+@pytest.mark.parametrize("rows,in_f,out_f,tile,dtype,offset", [
+    # calls packed into the form the LDS-DMA GEMM reads: the fewest K stages of
+    # each rule, ragged last blocks and columns, every kind of scale tile
+    (65, 129, 127, 64, "f32", 0), (300, 1000, 129, 32, "f32", 0), (130, 161, 100, 32, "bf16", 0),
+    (100, 321, 130, 128, "f32", 0), (257, 705, 200, 192, "bf16", 0), (66, 352, 256, 32, "f32", 0),
+    (200, 384, 384, 64, "f32", 1), (90, 768, 100, 128, "bf16", 0), (5000, 200, 300, 64, "bf16", 1),
+])
+def test_fp8_linear_packed(rows, in_f, out_f, tile, dtype, offset):
+    """The packed path against the oracle (the bars of the two dtypes) and
+    against the general kernel that a call without a workspace runs.  `offset`
+    elements make x's first row unaligned."""
+    from smaulnative_amd import _lib
+    print(f"case fp8_linear packed rows={rows} in_f={in_f} out_f={out_f} tile={tile} {dtype} +{offset}", flush=True)
+    lib = _lib.load()
+    gen = torch.Generator().manual_seed(rows + in_f * 3 + out_f + tile)
+    x = torch.randn(rows, in_f, generator=gen).to(torch.float32 if dtype == "f32" else torch.bfloat16)
+    w = torch.randint(0, 256, (out_f, in_f), generator=gen, dtype=torch.int64).to(torch.uint8)  # every code
+    s = torch.rand(out_f, -(-in_f // tile), generator=gen) * 0.01 + 1e-3
+    xd = torch.empty(rows * in_f + offset, dtype=x.dtype, device=DEV)[offset:].view(rows, in_f)
+    xd.copy_(x)
+    wd, sd = w.to(DEV), s.to(DEV)
+    act = _lib.DTYPE_F32 if dtype == "f32" else _lib.DTYPE_BF16
+    assert lib.smaul_fp8_linear_workspace(xd.data_ptr(), act, wd.data_ptr(), rows, in_f, out_f, tile) > 0
+    y = be().fp8_forward(xd, wd, sd, in_f, out_f, tile).cpu()
+    plain = torch.empty(rows, out_f, device=DEV)
+    rc = lib.smaul_fp8_linear_ws(xd.data_ptr(), act, wd.data_ptr(), sd.data_ptr(), plain.data_ptr(), _lib.DTYPE_F32,
+                                 rows, in_f, out_f, tile, 0, None, 0, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "fp8_linear_ws")
+    bar = 1e-5 if dtype == "f32" else 2e-6
+    ref = oracle.fp8_forward(x.float(), w, s, in_f, out_f, tile)
+    assert rel_max(y, ref) < bar and rel_max(plain, ref) < bar, (rel_max(y, ref), rel_max(plain, ref))
+
+
 def test_fp8_linear_ws_abi_fallbacks():
     """smaul_fp8_linear_ws through the C-ABI: the two-plane path with a large
     enough workspace and smaul_fp8_linear itself (the in-LDS split) without
