@@ -434,6 +434,21 @@ int smaul_fp8_quantize_tiles(const float* w, int64_t out_f, int64_t in_f, int64_
                              unsigned long long* nonfinite, hipStream_t stream);
 
 /*
+ * One weight update of a tiled-FP8 matrix (FP8Linear.requant and
+ * fused_lion_requant, kernel/fp8_tile.py:240-285): w = decode(w8) * sc, times
+ * `keep` when `decay`, minus `update` (fp32, or NULL) -- or, with g and m,
+ * minus sign(b1 m + c1 g) lr, m (fp32, in place) advancing to b2 m + c2 g --
+ * quantized as smaul_fp8_quantize_tiles does into codes [out_f, in_f] and
+ * scales [out_f, ceil(in_f/tile)], which must not overlap the inputs.  g fp32 or
+ * bf16.  Codes, scales and momentum are those of the reference's tensor
+ * operations, bit for bit.
+ */
+int smaul_fp8_requant(const uint8_t* w8, const float* sc, int64_t out_f, int64_t in_f, int64_t tile,
+                      const float* update, int decay, float keep, const void* g, int g_dtype, float* m, float lr,
+                      float b1, float c1, float b2, float c2, const uint8_t* order, const float* bounds,
+                      uint8_t* codes, float* scales, unsigned long long* nonfinite, hipStream_t stream);
+
+/*
  * Input gradient of the tiled-FP8 linear: dx[rows, in_f] = g[rows, out_f] .
  * decode(w, s), fp32.  Replaces the reference's native fp8_backward_input
  * (kernel/fp8_cpu.cpp:167-259; backend entry kernel/compute.py:145-153).

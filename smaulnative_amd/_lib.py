@@ -64,6 +64,8 @@ SIGNATURES = {
     "smaul_attn_step": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, ctypes.c_float, _P]),
     "smaul_attn_backward": (_I, [_P] * 9 + [_I64, _I64, _I64, _I64, ctypes.c_float, _P, _I64, _P]),
     "smaul_fp8_quantize_tiles": (_I, [_P, _I64, _I64, _I64, _P, _P, _P, _I64, _P, _P, _P]),
+    "smaul_fp8_requant": (_I, [_P, _P, _I64, _I64, _I64, _P, _I, ctypes.c_float, _P, _I, _P] + [ctypes.c_float] * 5
+                          + [_P] * 6),
     "smaul_fp8_backward_input": (_I, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P]),
     "smaul_fp8_weight_grad": (_I, [_P, _P, _I, _P, _I64, _I64, _I64, _I, _P]),
     "smaul_wait_timeouts": (_I, [_P, _I, _P]),

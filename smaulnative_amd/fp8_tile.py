@@ -195,14 +195,31 @@ class FP8Linear(nn.Module):
         for o0 in range(0, self.out_f, step):
             yield o0, min(o0 + step, self.out_f)
 
+    def _device_requant(self, *tensors):
+        """Whether the backend's one-pass update takes these buffers (with the
+        ``[out_f, in_f]`` tensors of the update), else the tensor operations do."""
+        return self.w8.is_cuda and hasattr(get_backend(), "fp8_requant") and self.w8.dtype == torch.uint8 and \
+            self.sc.dtype == torch.float32 and self.w8.is_contiguous() and self.sc.is_contiguous() and \
+            all(t.device == self.w8.device and t.is_contiguous() and tuple(t.shape) == (self.out_f, self.in_f)
+                for t in tensors)
+
     @torch.no_grad()
-    def _requant_rows(self, o0, o1, update, decay):
-        w = decode_block(self.w8, self.sc, o0, o1, self.in_f, self.tile)
-        if decay:
-            w.mul_(1 - decay)
-        if update is not None:
-            w.sub_(update.to(w.dtype))
-        codes, scales = quantize_tiles(w, self.tile)
+    def _requant_rows(self, o0, o1, update, decay, lion=None):
+        if lion is not None or (self._device_requant() and (update is None or update.device == self.w8.device)):
+            if update is not None:
+                update = update.to(torch.float32).contiguous()
+            codes, scales, nonfinite = get_backend().fp8_requant(self.w8[o0:o1], self.sc[o0:o1], self.tile, decay,
+                                                                 update, lion)
+            if nonfinite:
+                warnings.warn(f"quantize_tiles: {nonfinite} non-finite weight(s) saturated to finite E4M3",
+                              RuntimeWarning)
+        else:
+            w = decode_block(self.w8, self.sc, o0, o1, self.in_f, self.tile)
+            if decay:
+                w.mul_(1 - decay)
+            if update is not None:
+                w.sub_(update.to(w.dtype))
+            codes, scales = quantize_tiles(w, self.tile)
         self.w8[o0:o1].copy_(codes)
         self.sc[o0:o1].copy_(scales)
 
@@ -227,7 +244,12 @@ class FP8Linear(nn.Module):
         b2*m + (1-b2)*g; the same elementwise formulas as the reference
         (kernel/fp8_tile.py:266-282), so codes and momentum match it bit for bit.
         Clears ``_gw``."""
+        on_device = gw.dtype in (torch.float32, torch.bfloat16) and st.dtype == torch.float32 and \
+            self._device_requant(gw, st)
         for o0, o1 in self._row_groups():
+            if on_device:
+                self._requant_rows(o0, o1, None, lr * wd, (gw[o0:o1], st[o0:o1], lr, b1, b2))
+                continue
             g = gw[o0:o1].float()
             m = st[o0:o1]
             step = (m * b1 + g * (1.0 - b1)).sign() * lr

@@ -244,6 +244,45 @@ class RocmBackend:
         _lib.check(rc, "fp8_quantize_tiles")
         return codes, sc, int(bad.item())
 
+    def fp8_requant(self, w8, sc, tile, decay, update=None, lion=None):
+        """(codes [out_f, in_f], scales, non-finite count) of an FP8Linear weight
+        after one update, in one pass on the device (kernel/fp8_tile.py:240-285,
+        bit-identical): decode(w8, sc) * (1 - decay) - update, quantized.
+
+        ``update``: fp32 [out_f, in_f] or None.  ``lion``: (g, m, lr, b1, b2)
+        instead, the update sign(b1*m + (1-b1)*g) * lr with the fp32 momentum m
+        advanced in place; g fp32 or bf16.  All contiguous, on one device.
+        """
+        from smaulnative_amd import codebook
+        lib = _lib.load()
+        g, m, lr, b1, b2 = lion if lion is not None else (None, None, 0.0, 0.0, 0.0)
+        _need_device("fp8_requant", w8, sc, update, g, m)
+        out_f, in_f = w8.shape
+        nt = (in_f + tile - 1) // tile
+        if w8.dtype != torch.uint8 or sc.dtype != torch.float32 or tuple(sc.shape) != (out_f, nt):
+            raise RuntimeError(f"fp8_requant: w8 uint8 [{out_f}, {in_f}] and sc float32 [{out_f}, {nt}] expected, got "
+                               f"{w8.dtype}, {sc.dtype} {tuple(sc.shape)}")
+        for name, t, dtypes in (("update", update, (torch.float32,)), ("g", g, tuple(_ACT)),
+                                ("m", m, (torch.float32,))):
+            if t is not None and (t.dtype not in dtypes or tuple(t.shape) != (out_f, in_f)):
+                raise RuntimeError(f"fp8_requant: {name} must be {dtypes} [{out_f}, {in_f}], got {t.dtype} "
+                                   f"{tuple(t.shape)}")
+        if not all(t is None or t.is_contiguous() for t in (w8, sc, update, g, m)):
+            raise RuntimeError("fp8_requant: tensors must be contiguous")
+        dev = w8.device
+        _, mids, order8 = codebook.encode_tables(dev)
+        codes, scales = torch.empty_like(w8), torch.empty_like(sc)
+        bad = torch.empty(1, dtype=torch.int64, device=dev)
+        with torch.cuda.device(dev):
+            rc = lib.smaul_fp8_requant(w8.data_ptr(), sc.data_ptr(), out_f, in_f, tile,
+                                       None if update is None else update.data_ptr(), int(bool(decay)), 1 - decay,
+                                       None if g is None else g.data_ptr(), 0 if g is None else _ACT[g.dtype],
+                                       None if m is None else m.data_ptr(), lr, b1, 1.0 - b1, b2, 1.0 - b2,
+                                       order8.data_ptr(), mids.data_ptr(), codes.data_ptr(), scales.data_ptr(),
+                                       bad.data_ptr(), _stream_handle(dev))
+        _lib.check(rc, "fp8_requant")
+        return codes, scales, int(bad.item())
+
     # ---- linear attention (compute.py:265-322, attn_cpu.cpp) ---------------
     @staticmethod
     def _attn_check(name, eps, tensors):

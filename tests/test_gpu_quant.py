@@ -67,3 +67,56 @@ def test_device_quantizer_warns_on_nonfinite():
     assert any("2 non-finite" in str(r.message) for r in rec)
     ref_c, ref_s = oracle.quantize_tiles(w, 64)
     assert torch.equal(c.cpu(), ref_c) and torch.equal(s.cpu(), ref_s)
+
+
+@pytest.mark.parametrize("out_f,in_f,tile,gdtype", [
+    # the four-weights-a-lane kernel (4 to 256 wide tiles, ragged last ones), the
+    # scalar ones (widths and tiles it does not take)
+    (70, 1024, 64, torch.bfloat16), (33, 100, 32, torch.float32), (5, 4, 4, torch.bfloat16),
+    (9, 516, 256, torch.float32), (33, 333, 32, torch.bfloat16), (17, 200, 48, torch.bfloat16),
+    (3, 1500, 512, torch.float32), (40, 90, 2, torch.float32)])
+def test_device_requant_is_the_tensor_operations(out_f, in_f, tile, gdtype):
+    """requant and the Lion step in one pass against the tensor operations they
+    replace (decode_block, in-place arithmetic, quantize_tiles): codes, scales
+    and momentum bit for bit, non-finite weights and every code included."""
+    from smaulnative_amd.fp8_tile import FP8Linear, decode_block
+    print(f"case requant {out_f}x{in_f} tile={tile} {gdtype}", flush=True)
+    gen = torch.Generator().manual_seed(out_f * 13 + in_f + tile)
+    w8 = torch.randint(0, 256, (out_f, in_f), generator=gen, dtype=torch.int64).to(torch.uint8).to(DEV)
+    sc = (torch.rand(out_f, -(-in_f // tile), generator=gen) * 0.01 + 1e-4).to(DEV)
+    upd = (torch.randn(out_f, in_f, generator=gen) * 0.1).to(DEV)
+    upd[0, 0], upd[-1, -1] = float("nan"), float("inf")
+    g = (torch.randn(out_f, in_f, generator=gen) * 1e-3).to(gdtype).to(DEV)
+    m = (torch.randn(out_f, in_f, generator=gen) * 1e-3).to(DEV)
+    m[0, :2] = 0.0
+    g[0, :2] = 0.0   # a zero step
+    lr, wd, b1, b2 = 1e-2, 0.1, 0.9, 0.99
+
+    def module():
+        lin = FP8Linear(in_f, out_f, tile).to(DEV)
+        lin.w8.copy_(w8)
+        lin.sc.copy_(sc)
+        return lin
+
+    for update, decay in ((upd, 0.0), (upd, 0.03), (None, 0.03), (None, 0.0)):
+        w = decode_block(w8, sc, 0, out_f, in_f, tile)
+        if decay:
+            w.mul_(1 - decay)
+        if update is not None:
+            w.sub_(update)
+        with warnings.catch_warnings(record=True) as rec:
+            warnings.simplefilter("always")
+            rc, rs = quantize_tiles(w, tile)
+            lin = module()
+            version = lin.w8._version
+            lin.requant(update, decay)
+        assert len(rec) == (0 if update is None else 2) and len({str(r.message) for r in rec}) <= 1
+        assert lin.w8._version > version   # what caches made from the codes go by
+        assert torch.equal(lin.w8, rc) and torch.equal(lin.sc, rs)
+    st, ref = m.clone(), m.clone()
+    lin = module()
+    lin.fused_lion_requant(g, st, lr, wd, b1, b2)
+    step = (ref * b1 + g.float() * (1.0 - b1)).sign() * lr
+    ref.mul_(b2).add_(g.float(), alpha=1.0 - b2)
+    rc, rs = quantize_tiles(decode_block(w8, sc, 0, out_f, in_f, tile).mul_(1 - lr * wd).sub_(step), tile)
+    assert torch.equal(st, ref) and torch.equal(lin.w8, rc) and torch.equal(lin.sc, rs)
