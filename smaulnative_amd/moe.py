@@ -86,7 +86,14 @@ class SwiFFN(nn.Module):
         return self.down((F.silu(self.gate(x).float()) * self.up(x).float()).to(odt))
 
     def buffers6(self):
-        return (self.gate.w8, self.gate.sc, self.up.w8, self.up.sc, self.down.w8, self.down.sc)
+        # straight from the modules' dictionaries: nine attribute searches per
+        # expert through nn.Module.__getattr__ take a decode call 3 us each expert
+        try:
+            mods = self._modules
+            g, u, d = mods["gate"]._buffers, mods["up"]._buffers, mods["down"]._buffers
+            return (g["w8"], g["sc"], u["w8"], u["sc"], d["w8"], d["sc"])
+        except (KeyError, AttributeError):  # a buffer replaced by a plain attribute
+            return (self.gate.w8, self.gate.sc, self.up.w8, self.up.sc, self.down.w8, self.down.sc)
 
 
 class SwiFFN_MoE(nn.Module):
@@ -148,9 +155,9 @@ class SwiFFN_MoE(nn.Module):
         experts = [ex.buffers6() for ex in self.experts]
         out, prob, topi, counts = be.moe_forward(x, self.gate.weight, self.gate.bias, experts,
                                                  self.top_k, self.tile)
-        self.last_prob = prob
-        self.last_topi = topi
-        self._counts_dev = counts
+        # plain attributes, set past nn.Module.__setattr__ (3 us each): none is a
+        # parameter, buffer or module
+        self.__dict__.update(last_prob=prob, last_topi=topi, _counts_dev=counts)
         return out
 
     def _forward_train(self, x):

@@ -27,7 +27,9 @@ Behaviour differences from the reference CPU backend, all deliberate:
 """
 from __future__ import annotations
 
+import contextlib
 import math
+import operator
 import os
 import threading
 import weakref
@@ -40,8 +42,19 @@ from smaulnative_amd import _lib
 _ACT = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}
 
 
+_HERE = contextlib.nullcontext()
+
+
+def _device(device):
+    """``torch.cuda.device(device)``, or nothing to enter where it is the current
+    one already (a device switch and back costs a small call 3 us)."""
+    index = device.index
+    return _HERE if index is None or index == torch.cuda.current_device() else torch.cuda.device(index)
+
+
 def _stream_handle(device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    index = torch.cuda.current_device() if device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 class _CacheEntry(dict):
@@ -160,7 +173,7 @@ class RocmBackend:
         # LDS-DMA GEMM does not take as they are through packed operands
         nws = lib.smaul_fp8_linear_workspace(xc.data_ptr(), _ACT[xc.dtype], wc.data_ptr(), rows, in_f, out_f, tile)
         ws = torch.empty(max(nws, 0), dtype=torch.uint8, device=x.device) if nws > 0 else None
-        with torch.cuda.device(x.device):
+        with _device(x.device):
             rc = lib.smaul_fp8_linear_ws(xc.data_ptr(), _ACT[xc.dtype], wc.data_ptr(), sc.data_ptr(),
                                          y.data_ptr(), _lib.DTYPE_F32, rows, in_f, out_f, tile, 0,
                                          None if ws is None else ws.data_ptr(), max(nws, 0),
@@ -188,7 +201,7 @@ class RocmBackend:
         sc = s.reshape(-1)
         sc = (sc if sc.dtype == torch.float32 else sc.float()).contiguous()
         dx = torch.empty(g.shape[0], in_f, dtype=torch.float32, device=g.device)
-        with torch.cuda.device(g.device):
+        with _device(g.device):
             rc = lib.smaul_fp8_backward_input(gc.data_ptr(), wc.data_ptr(), sc.data_ptr(), dx.data_ptr(), g.shape[0],
                                               in_f, out_f, tile, _stream_handle(g.device))
         _lib.check(rc, "fp8_backward_input")
@@ -209,7 +222,7 @@ class RocmBackend:
         if not gw.is_contiguous():
             raise RuntimeError("fp8_weight_grad: gw must be contiguous (it is updated in place)")
         gc, xc = (t if t.is_contiguous() else t.contiguous() for t in (g, x))
-        with torch.cuda.device(g.device):
+        with _device(g.device):
             rc = lib.smaul_fp8_weight_grad(gc.data_ptr(), xc.data_ptr(), _ACT[x.dtype], gw.data_ptr(), x.shape[0],
                                            x.shape[1], gw.shape[0], int(bool(fresh)), _stream_handle(g.device))
         _lib.check(rc, "fp8_weight_grad")
@@ -237,7 +250,7 @@ class RocmBackend:
         codes = torch.empty(out_f, nt * tile, dtype=torch.uint8, device=dev)
         sc = torch.empty(out_f, nt, dtype=torch.float32, device=dev)
         bad = torch.empty(1, dtype=torch.int64, device=dev)
-        with torch.cuda.device(dev):
+        with _device(dev):
             rc = lib.smaul_fp8_quantize_tiles(w.data_ptr(), out_f, in_f, tile, order8.data_ptr(), mids.data_ptr(),
                                               codes.data_ptr(), nt * tile, sc.data_ptr(), bad.data_ptr(),
                                               _stream_handle(dev))
@@ -273,7 +286,7 @@ class RocmBackend:
         _, mids, order8 = codebook.encode_tables(dev)
         codes, scales = torch.empty_like(w8), torch.empty_like(sc)
         bad = torch.empty(1, dtype=torch.int64, device=dev)
-        with torch.cuda.device(dev):
+        with _device(dev):
             rc = lib.smaul_fp8_requant(w8.data_ptr(), sc.data_ptr(), out_f, in_f, tile,
                                        None if update is None else update.data_ptr(), int(bool(decay)), 1 - decay,
                                        None if g is None else g.data_ptr(), 0 if g is None else _ACT[g.dtype],
@@ -321,7 +334,7 @@ class RocmBackend:
             z = torch.empty(0, dtype=torch.float32, device=dev)
         ws_bytes = lib.smaul_attn_workspace_size(B, H, D, int(bool(need_state)))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
-        with torch.cuda.device(dev):
+        with _device(dev):
             rc = lib.smaul_attn_forward(Qc.data_ptr(), Kc.data_ptr(), Vc.data_ptr(), Y.data_ptr(),
                                         None if DEN is None else DEN.data_ptr(),
                                         S.data_ptr() if need_state else None, z.data_ptr() if need_state else None,
@@ -346,7 +359,7 @@ class RocmBackend:
             raise RuntimeError(f"attn_step: D={D} out of the supported range (0, 2048]")
         qc, kc, vc = (t if t.is_contiguous() else t.contiguous() for t in (q, k, v))
         y = torch.empty_like(qc)
-        with torch.cuda.device(q.device):
+        with _device(q.device):
             rc = lib.smaul_attn_step(S.data_ptr(), z.data_ptr(), qc.data_ptr(), kc.data_ptr(), vc.data_ptr(),
                                      y.data_ptr(), B, H, D, float(eps), _stream_handle(q.device))
         _lib.check(rc, "attn_step")
@@ -374,7 +387,7 @@ class RocmBackend:
         dQ, dK, dV = torch.empty_like(Qc), torch.empty_like(Qc), torch.empty_like(Qc)
         ws_bytes = lib.smaul_attn_backward_workspace_size(B, T, H, D)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
-        with torch.cuda.device(dev):
+        with _device(dev):
             rc = lib.smaul_attn_backward(dYc.data_ptr(), Qc.data_ptr(), Kc.data_ptr(), Vc.data_ptr(), Yc.data_ptr(),
                                          DENc.data_ptr(), dQ.data_ptr(), dK.data_ptr(), dV.data_ptr(), B, T, H, D,
                                          float(eps), None if ws is None else ws.data_ptr(), ws_bytes,
@@ -418,11 +431,11 @@ class RocmBackend:
             if len(ex) != 6:
                 raise ValueError("each expert is (gate_w8, gate_sc, up_w8, up_sc, down_w8, down_sc)")
             flat.extend(ex)
-        key = (str(device), d, h, tile, tuple(t.data_ptr() for t in flat))
-        versions = tuple(t._version for t in flat)
+        key = (str(device), d, h, tile, tuple([t.data_ptr() for t in flat]))
+        versions = tuple([t._version for t in flat])
         with self._lock:
             ent = self._ptr_cache.get(key)
-        if ent is not None and all(r() is t for r, t in zip(ent["refs"], flat)):
+        if ent is not None and all(map(operator.is_, [r() for r in ent["refs"]], flat)):
             if ent["versions"] != versions:
                 self._refresh(ent, flat, lib, device)
                 ent["versions"] = versions
@@ -490,7 +503,7 @@ class RocmBackend:
                 codes = codes if codes.is_contiguous() else codes.contiguous()
                 sc = sc if (sc.dtype == torch.float32 and sc.is_contiguous()) else sc.float().contiguous()
                 N, K = codes.shape
-                with torch.cuda.device(device):
+                with _device(device):
                     rc = lib.smaul_fp8_tile_layout(codes.data_ptr(), sc.data_ptr(), ent["copies"][n].data_ptr(),
                                                    ent["copies"][n + 1].data_ptr(), N, K, stream)
                 _lib.check(rc, "fp8_tile_layout")
@@ -499,7 +512,7 @@ class RocmBackend:
             if n % 2 == 0:
                 src = t if t.is_contiguous() else t.contiguous()
                 dst = ent["copies"][n]
-                with torch.cuda.device(device):
+                with _device(device):
                     rc = lib.smaul_fp8_canonicalize(src.data_ptr(), dst.data_ptr(), src.numel(), stream)
                 _lib.check(rc, "fp8_canonicalize")
             elif not (t.dtype == torch.float32 and t.is_contiguous()):
@@ -535,7 +548,7 @@ class RocmBackend:
         out = torch.empty_like(x2)
         ws_bytes = lib.smaul_swiffn_workspace_size(rows, h, _ACT[x.dtype])
         ws = torch.empty(max(1, ws_bytes), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
+        with _device(dev):
             rc = lib.smaul_swiffn_forward(x2.data_ptr(), _ACT[x.dtype], *[ptrs[i][0] for i in range(6)],
                                           out.data_ptr(), ws.data_ptr(), ws_bytes, rows, d, h, tile,
                                           ent["flags"], _stream_handle(dev))
@@ -560,7 +573,7 @@ class RocmBackend:
         topw = torch.empty(T, top_k, dtype=torch.float32, device=x2.device)
         gw = gate_w.detach().float().contiguous()
         gb = None if gate_b is None else gate_b.detach().float().contiguous()
-        with torch.cuda.device(x2.device):
+        with _device(x2.device):
             rc = lib.smaul_moe_router(x2.data_ptr(), _ACT[x2.dtype], gw.data_ptr(),
                                       None if gb is None else gb.data_ptr(), prob.data_ptr(),
                                       topi.data_ptr(), topw.data_ptr(), T, d, E, top_k,
@@ -592,7 +605,7 @@ class RocmBackend:
         }
         ws_bytes = lib.smaul_moe_dispatch_workspace_size(T, E)
         ws = torch.empty(max(1, ws_bytes), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
+        with _device(dev):
             rc = lib.smaul_moe_dispatch(topi.contiguous().data_ptr(), topw.contiguous().data_ptr(),
                                         out["counts"].data_ptr(), out["seg_off"].data_ptr(),
                                         out["tile_off"].data_ptr(), out["perm_row"].data_ptr(),
@@ -637,7 +650,7 @@ class RocmBackend:
         rec = (lambda i: events[i].record(stream)) if events else (lambda i: None)
         tp = table.data_ptr()
         row = E * 8
-        with torch.cuda.device(dev):
+        with _device(dev):
             rec(0)
             prob, topi, topw = self.moe_router(x2, gw, gb, top_k)
             rec(1)
@@ -684,7 +697,7 @@ class RocmBackend:
             w = weight.detach().reshape(d)
             w = w if (w.dtype == torch.float32 and w.is_contiguous()) else w.float().contiguous()
         out = torch.empty_like(x2)
-        with torch.cuda.device(x.device):
+        with _device(x.device):
             rc = lib.smaul_rms_norm(x2.data_ptr(), _ACT[x.dtype], None if w is None else w.data_ptr(),
                                     out.data_ptr(), x2.shape[0], d, eps, _stream_handle(x.device))
         _lib.check(rc, "rms_norm")
@@ -703,7 +716,7 @@ class RocmBackend:
         lib = _lib.load()
         dev = torch.device("cuda", torch.cuda.current_device()) if device is None else torch.device(device)
         buf = torch.empty(1, dtype=torch.int32, device=dev)
-        with torch.cuda.device(dev):
+        with _device(dev):
             rc = lib.smaul_wait_timeouts(buf.data_ptr(), int(bool(reset)), _stream_handle(dev))
         _lib.check(rc, "wait_timeouts")
         return int(buf.item())
@@ -819,7 +832,7 @@ class RocmBackend:
                     tp, tp + row, tp + 2 * row, tp + 3 * row, tp + 4 * row, tp + 5 * row,
                     out.data_ptr(), prob.data_ptr(), topi.data_ptr(), topw.data_ptr(),
                     counts.data_ptr(), ws.data_ptr(), ws_bytes, T, d, h, E, top_k, tile, eflags]
-            with torch.cuda.device(dev):
+            with _device(dev):
                 if norm is None:
                     rc = lib.smaul_moe_forward(*args, _stream_handle(dev))
                 elif routing is None and nxt is None:
@@ -836,7 +849,8 @@ class RocmBackend:
                                                      _stream_handle(dev))
             _lib.check(rc, "moe_forward")
         lead = x.shape[:-1]
-        res = (out.reshape(*lead, d), prob.reshape(*lead, E), topi.reshape(*lead, top_k), counts)
+        res = (out, prob, topi, counts) if x.dim() == 2 else \
+            (out.reshape(*lead, d), prob.reshape(*lead, E), topi.reshape(*lead, top_k), counts)
         if norm is None:
             return res
         res = res + (normed.reshape(*lead, d),)
