@@ -1439,6 +1439,8 @@ struct RouteOut {
   float* perm_w;
   int32_t* inv;
   int block_m;
+  // fp32 x only: its bf16 hi / lo planes [T][2 d] for the GEMMs, or nullptr
+  uint16_t* planes;
 };
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -1575,6 +1577,31 @@ __device__ __forceinline__ void route_load_x(const void* x, int64_t T, int64_t t
           xr[q][a][0] = ldg16((const float*)x + t * d + c0 + g * 8);
           xr[q][a][XW - 1] = ldg16((const float*)x + t * d + c0 + g * 8 + 4);
         }
+      }
+    }
+  }
+}
+
+// The fp32 values of route_load_x split into their bf16 hi / lo planes (as
+// split_planes_kernel writes them), two 16-byte stores per token and group.
+template <int TB, int EMAX>
+__device__ __forceinline__ void route_split(const uint4 (&xr)[RouteShape<EMAX>::XG][TB][2], uint16_t* planes,
+                                            int64_t T, int64_t tw0, int c0, int cw, int d, int lane) {
+#pragma unroll
+  for (int q = 0; q < RouteShape<EMAX>::XG; ++q) {
+    const int g = lane + 64 * q;
+    if (g < (cw >> 3)) {
+#pragma unroll
+      for (int a = 0; a < TB; ++a) {
+        if (tw0 + a >= T) continue;
+        const uint32_t v[8] = {xr[q][a][0].x, xr[q][a][0].y, xr[q][a][0].z, xr[q][a][0].w,
+                               xr[q][a][1].x, xr[q][a][1].y, xr[q][a][1].z, xr[q][a][1].w};
+        uint32_t h[8], l[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) split_bf16(__uint_as_float(v[i]), h[i], l[i]);
+        uint16_t* o = planes + (tw0 + a) * 2 * d + c0 + g * 8;
+        *(uint4*)o = make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
+        *(uint4*)(o + d) = make_uint4(l[0] | (l[1] << 16), l[2] | (l[3] << 16), l[4] | (l[5] << 16), l[6] | (l[7] << 16));
       }
     }
   }
@@ -2794,6 +2821,8 @@ router_kernel(const void* __restrict__ x, const float* __restrict__ gw, const fl
     }
     __syncthreads();
     route_fma<XBF16, TB, EMAX>(xr, sW, cw, lane, acc);
+    if constexpr (!XBF16)
+      if (o.planes) route_split<TB, EMAX>(xr, o.planes, T, tw0, c0, cw, d, lane);
   }
   {
     const int vidx = route_butterfly<TB, EMAX>(acc, lane);
@@ -3916,6 +3945,9 @@ struct CfgDmaDownN {
 struct CfgDmaGU64 {  // 64 rows x 128 outputs (gate+up), 4 waves of 64 rows x 32 outputs
   static constexpr int BM = 64, BN = 256, WM = 1, WN = 4, NSTAGE = 2;
 };
+struct CfgDmaGU32 {  // 32 rows x 128 outputs (gate+up)
+  static constexpr int BM = 32, BN = 256, WM = 1, WN = 4, NSTAGE = 3;
+};
 struct CfgDma64x128 {  // 64 rows x 128 outputs
   static constexpr int BM = 64, BN = 128, WM = 1, WN = 4, NSTAGE = 3;
 };
@@ -5017,9 +5049,20 @@ __global__ void wait_timeouts_kernel(int32_t* out, int reset) {
   if (reset) __hip_atomic_fetch_sub(&g_wait_timeouts, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Whether fp32 activations run the LDS-DMA grouped GEMMs over planes, on
-// 64-row tiles: tile 64, d and h multiples of 128, codes promised 16-byte
-// aligned, the kernels' 32-bit offsets for the planes of x and of hdn.
+// The row tiles of the planes GEMMs: 64, or 32 with deeper pipelines where a
+// 64-row gate+up grid gives a CU at most two workgroups, so that a tile's
+// latency is the launch's (whole layer, graph replay, us, 64 / 32 rows: T 1, d
+// 512, E 4 38.0 / 29.5; T 64, d 1024, E 8 65.4 / 50.2; T 300 79.9 / 71.4; at 2.7
+// workgroups a CU T 2048, d 512 73.8 / 80.1, at 3.1 T 1000, d 1024 119.1 /
+// 119.7, at 11 T 4000 302 / 326).
+static int64_t planes_block_m(int64_t h, int64_t E, int64_t R) {
+  return ((R + DMA_SMALL_BM - 1) / DMA_SMALL_BM + E) * (h / 128) < 2 * (int64_t)cu_count() ? CfgDmaGU32::BM
+                                                                                           : DMA_SMALL_BM;
+}
+
+// Whether fp32 activations run the LDS-DMA grouped GEMMs over planes: tile 64,
+// d and h multiples of 128, codes promised 16-byte aligned, the kernels' 32-bit
+// offsets for the planes of x and of hdn.
 static bool f32_planes_ok(int64_t T, int64_t d, int64_t h, int64_t E, int64_t tile, int flags, int64_t R) {
   if (tile != 64 || d % 128 != 0 || h % 128 != 0 || !(flags & SMAUL_FLAG_ALIGNED_CODES)) return false;
   const int64_t lim = (int64_t)1 << 31;
@@ -5028,7 +5071,8 @@ static bool f32_planes_ok(int64_t T, int64_t d, int64_t h, int64_t E, int64_t ti
 }
 
 // The grouped gate+up and down of fp32 x (after the dispatch, on the tile
-// table of block_m rows): x split into bf16 hi / lo planes ([T][2d]); gate+up
+// table of block_m rows): x as its bf16 hi / lo planes ([T][2d], which the
+// router has written on its way over x, else `split` has them made); gate+up
 // over both planes of the gathered rows (K doubled, weight blocks wrapped)
 // with the SwiGLU product kept in fp32 and stored as the planes of hdn
 // ([R][2h], the fp32 hdn's bytes); down over those planes with fp32 output
@@ -5038,7 +5082,7 @@ static int moe_f32_planes(const float* x, uint16_t* xplanes, const int32_t* perm
                           const float* const* gs, const uint8_t* const* uw, const float* const* us,
                           const uint8_t* const* dw, const float* const* ds, uint16_t* hplanes, float* yperm,
                           const int32_t* seg_off, const int32_t* tile_off, int64_t max_tiles, int64_t T, int64_t d,
-                          int64_t h, int64_t E, int64_t bm, int flags, hipStream_t stream) {
+                          int64_t h, int64_t E, int64_t bm, int flags, bool split, hipStream_t stream) {
   GemmArgs g{};
   g.x = xplanes;
   g.row_idx = perm_row;
@@ -5077,8 +5121,15 @@ static int moe_f32_planes(const float* x, uint16_t* xplanes, const int32_t* perm
   if (!dma_gemm_ok(g, SMAUL_DTYPE_BF16, flags, T, 128) || !dma_gemm_ok(dn, SMAUL_DTYPE_BF16, flags, max_tiles * bm, 128))
     return fail(SMAUL_ERR_UNSUPPORTED, "moe_forward: fp32 planes shapes outside the LDS-DMA kernels");
   const bool canon = (flags & SMAUL_FLAG_CANONICAL_CODES) != 0;
-  int rc = launch_split_planes(x, xplanes, T, d, stream);
+  int rc = split ? launch_split_planes(x, xplanes, T, d, stream) : SMAUL_OK;
   if (rc != SMAUL_OK) return rc;
+  if (bm == CfgDmaGU32::BM) {
+    rc = canon ? launch_gemm_dma<CfgDmaGU32, true, true, true, ACT_PLANES>(g, max_tiles, stream)
+               : launch_gemm_dma<CfgDmaGU32, true, false, true, ACT_PLANES>(g, max_tiles, stream);
+    if (rc != SMAUL_OK) return rc;
+    return canon ? launch_gemm_dma<CfgDma32x128, false, true, true, ACT_PLANES>(dn, max_tiles, stream)
+                 : launch_gemm_dma<CfgDma32x128, false, false, true, ACT_PLANES>(dn, max_tiles, stream);
+  }
   rc = canon ? launch_gemm_dma<CfgDmaGU64, true, true, true, ACT_PLANES>(g, max_tiles, stream)
              : launch_gemm_dma<CfgDmaGU64, true, false, true, ACT_PLANES>(g, max_tiles, stream);
   if (rc != SMAUL_OK) return rc;
@@ -5140,7 +5191,7 @@ static int moe_forward_impl(const void* x, int act_dtype, const float* gate_w, c
   // fp32 x on the LDS-DMA kernels over bf16 hi / lo planes, else the
   // register-staged kernels
   const bool planes = act_dtype == SMAUL_DTYPE_F32 && f32_planes_ok(T, d, h, E, tile, flags, R);
-  if (planes) bm = DMA_SMALL_BM;
+  if (planes) bm = planes_block_m(h, E, R);
   if (bm == CfgBig::BM && act_dtype == SMAUL_DTYPE_BF16 &&
       ((R + CfgBig::BM - 1) / CfgBig::BM + E) * (h / 128) < 4 * (int64_t)cu_count()) {
     // a 128-row gate/up grid under four workgroups per CU: 64-row tiles
@@ -5175,6 +5226,7 @@ static int moe_forward_impl(const void* x, int act_dtype, const float* gate_w, c
   o.topw = topw;
   o.blockcnt = blockcnt;
   o.block_m = (int)bm;
+  o.planes = planes ? xplanes : nullptr;
   RouteOut od = o;
   od.counts = counts;
   od.seg_off = seg_off;
@@ -5285,7 +5337,7 @@ static int moe_forward_impl(const void* x, int act_dtype, const float* gate_w, c
   }
   if (planes) {
     rc = moe_f32_planes((const float*)x, xplanes, perm_row, gate_w8, gate_s, up_w8, up_s, down_w8, down_s,
-                        (uint16_t*)hdn, (float*)yperm, seg_off, tile_off, max_tiles, T, d, h, E, bm, flags, stream);
+                        (uint16_t*)hdn, (float*)yperm, seg_off, tile_off, max_tiles, T, d, h, E, bm, flags, routed, stream);
   } else {
     rc = smaul_moe_gate_up(x, act_dtype, perm_row, gate_w8, gate_s, up_w8, up_s, hdn, seg_off, tile_off,
                            max_tiles, E, d, h, tile, bm, flags, stream);

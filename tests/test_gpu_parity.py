@@ -567,6 +567,25 @@ def test_moe_decode_c4_shape(T, skew):
     assert err < 2e-3
 
 
+@pytest.mark.parametrize("T,d,h,E,k", [
+    (1, 256, 640, 4, 2), (32, 256, 384, 2, 1), (33, 512, 1280, 4, 2), (200, 1024, 2560, 8, 2),  # 32-row tiles
+    (1500, 512, 1280, 4, 2), (65, 2048, 5120, 16, 3)])                                          # 64
+def test_moe_f32_planes_row_tiles(T, d, h, E, k):
+    """fp32 x on 32- and 64-row tiles of the two-plane GEMMs, the planes written
+    by the router; and with the routing given, where a pass of its own writes
+    them: the same bits.  Against the oracle at the fp32 bar."""
+    print(f"case moe f32 planes T={T} d={d} h={h} E={E} k={k}", flush=True)
+    x, gw, gb, experts = make_moe(T + d, T, d, h, E, k, torch.float32)
+    ref = oracle.moe_forward(x, gw, gb, experts, k, 64)
+    out, prob, topi, counts = gpu_moe(x, gw, gb, experts, k)
+    assert torch.equal(topi.reshape(-1, k), ref.topi.reshape(-1, k)) and counts.tolist() == ref.counts
+    assert rel_l2(out, ref.out) < 1e-5
+    exd = to_dev_experts(experts)
+    routing = be().moe_router(x.to(DEV), gw.to(DEV), gb.to(DEV), k)
+    again = be().moe_forward_norm(x.to(DEV), gw.to(DEV), gb.to(DEV), exd, k, 64, routing=routing)[0]
+    assert torch.equal(again.cpu(), out)
+
+
 def test_moe_skewed_segments():
     """Config-5 style skew (one expert ~40 %, three < 1 %) at a reduced size."""
     x, gw, gb, experts = make_moe(55, 2048, 256, 640, 16, 2, skew=(2.2, [13, 14, 15], 4.0))
