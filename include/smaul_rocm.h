@@ -471,6 +471,15 @@ int smaul_fp8_weight_grad(const float* g, const void* x, int x_dtype, void* gw, 
                           int64_t out_f, int fresh, hipStream_t stream);
 
 /*
+ * The SwiGLU product of n values, out = silu(g) * u (model.py:289-290), and its
+ * gradients dg, du from dout; computed in fp32, stored in `dtype` (f32 or bf16),
+ * which all tensors have.
+ */
+int smaul_swiglu(const void* g, const void* u, void* out, int64_t n, int dtype, hipStream_t stream);
+int smaul_swiglu_backward(const void* dout, const void* g, const void* u, void* dg, void* du, int64_t n, int dtype,
+                          hipStream_t stream);
+
+/*
  * Measured ceilings for the roofline figures (bench.py --peaks); no
  * counterpart in the reference and not on the MoE path.
  * smaul_peak_mfma: `workgroups` x 4 waves, each issuing `iters` rounds of 8

@@ -68,6 +68,8 @@ SIGNATURES = {
                           + [_P] * 6),
     "smaul_fp8_backward_input": (_I, [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P]),
     "smaul_fp8_weight_grad": (_I, [_P, _P, _I, _P, _I64, _I64, _I64, _I, _P]),
+    "smaul_swiglu": (_I, [_P, _P, _P, _I64, _I, _P]),
+    "smaul_swiglu_backward": (_I, [_P, _P, _P, _P, _P, _I64, _I, _P]),
     "smaul_wait_timeouts": (_I, [_P, _I, _P]),
     "smaul_debug_tail_wait": (_I, [_I, _I]),
     "smaul_peak_mfma": (_I, [_P, _I, _I, _P]),

@@ -370,6 +370,48 @@ fp8_weight_grad_kernel(const float* __restrict__ g, const X* __restrict__ x, uin
   }
 }
 
+// ---- SwiGLU product of the training path (model.py:289-290) -----------------
+// out = silu(g) * u and its gradients, fp32 arithmetic whatever the dtype, each
+// one pass where the tensor operations take two and four (with the fp32
+// intermediates between them).  HBM-bound: 3 and 5 tensors' bytes.
+template <typename X>
+__device__ __forceinline__ void sg_store(X* p, float v) {
+  if constexpr (sizeof(X) == 4)
+    *p = v;
+  else
+    *p = (uint16_t)pack_bf16(v, 0.0f);
+}
+
+template <typename X, bool BACK>
+__global__ void __launch_bounds__(256)
+swiglu_kernel(const X* __restrict__ g, const X* __restrict__ u, const X* __restrict__ dout, X* __restrict__ a,
+              X* __restrict__ b, int64_t n) {
+  for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x); i < n; i += (int64_t)gridDim.x * 256) {
+    const float gv = wg_load(g + i), uv = wg_load(u + i);
+    const float sig = 1.0f / (1.0f + expf(-gv));
+    if constexpr (BACK) {
+      const float d = wg_load(dout + i);
+      sg_store(a + i, d * uv * sig * (1.0f + gv * (1.0f - sig)));
+      sg_store(b + i, d * (gv * sig));
+    } else {
+      sg_store(a + i, gv * sig * uv);
+    }
+  }
+}
+
+template <bool BACK>
+int swiglu_launch(const void* g, const void* u, const void* dout, void* a, void* b, int64_t n, int dtype,
+                  hipStream_t stream) {
+  const unsigned blocks = (unsigned)((n + 255) / 256 < 65536 ? (n + 255) / 256 : 65536);
+  if (dtype == SMAUL_DTYPE_F32)
+    hipLaunchKernelGGL((swiglu_kernel<float, BACK>), dim3(blocks), dim3(256), 0, stream, (const float*)g,
+                       (const float*)u, (const float*)dout, (float*)a, (float*)b, n);
+  else
+    hipLaunchKernelGGL((swiglu_kernel<uint16_t, BACK>), dim3(blocks), dim3(256), 0, stream, (const uint16_t*)g,
+                       (const uint16_t*)u, (const uint16_t*)dout, (uint16_t*)a, (uint16_t*)b, n);
+  return check_launch("swiglu_kernel");
+}
+
 }  // namespace
 
 extern "C" {
@@ -420,6 +462,23 @@ int smaul_fp8_weight_grad(const float* g, const void* x, int x_dtype, void* gw, 
     hipLaunchKernelGGL((fp8_weight_grad_kernel<uint16_t>), grid, dim3(256), 0, stream, g, (const uint16_t*)x,
                        (uint16_t*)gw, rows, out_f, in_f, fresh);
   return check_launch("fp8_weight_grad_kernel");
+}
+
+int smaul_swiglu(const void* g, const void* u, void* out, int64_t n, int dtype, hipStream_t stream) {
+  if (n < 0 || (dtype != SMAUL_DTYPE_F32 && dtype != SMAUL_DTYPE_BF16))
+    return fail(SMAUL_ERR_INVALID, "swiglu: need n >= 0 and f32|bf16");
+  if (n == 0) return SMAUL_OK;
+  if (!g || !u || !out) return fail(SMAUL_ERR_INVALID, "swiglu: null pointer");
+  return swiglu_launch<false>(g, u, nullptr, out, nullptr, n, dtype, stream);
+}
+
+int smaul_swiglu_backward(const void* dout, const void* g, const void* u, void* dg, void* du, int64_t n, int dtype,
+                          hipStream_t stream) {
+  if (n < 0 || (dtype != SMAUL_DTYPE_F32 && dtype != SMAUL_DTYPE_BF16))
+    return fail(SMAUL_ERR_INVALID, "swiglu_backward: need n >= 0 and f32|bf16");
+  if (n == 0) return SMAUL_OK;
+  if (!dout || !g || !u || !dg || !du) return fail(SMAUL_ERR_INVALID, "swiglu_backward: null pointer");
+  return swiglu_launch<true>(g, u, dout, dg, du, n, dtype, stream);
 }
 
 }  // extern "C"

@@ -65,6 +65,62 @@ def _needs_grad(module: nn.Module, x: torch.Tensor) -> bool:
     return x.requires_grad or any(p.requires_grad for p in module.parameters())
 
 
+class _SwiGLU(torch.autograd.Function):
+    """(silu(gate.float()) * up.float()).to(gate.dtype) and its gradients, a device
+    pass each."""
+
+    @staticmethod
+    def forward(ctx, gate, up):
+        ctx.save_for_backward(gate, up)
+        return get_backend().swiglu(gate, up)
+
+    @staticmethod
+    def backward(ctx, dout):
+        gate, up = ctx.saved_tensors
+        if torch.is_grad_enabled():  # a graph of the gradients is wanted: tensor operations
+            g, u, d = gate.float(), up.float(), dout.float()
+            sig = torch.sigmoid(g)
+            return (d * u * sig * (1 + g * (1 - sig))).to(gate.dtype), (d * (g * sig)).to(up.dtype)
+        return tuple(get_backend().swiglu_backward(dout, gate, up))
+
+
+def _swiglu(gate, up, dtype):
+    """(silu(gate.float()) * up.float()).to(dtype) of a SwiFFN being trained."""
+    if gate.is_cuda and gate.dtype == up.dtype == dtype and dtype in (torch.float32, torch.bfloat16) and \
+            hasattr(get_backend(), "swiglu"):
+        return _SwiGLU.apply(gate, up)
+    return (F.silu(gate.float()) * up.float()).to(dtype)
+
+
+def _sum_slots(y, at, weight=None):
+    """[T, d]: the sum over each token's slots of y[at] (times weight [T, k, 1]);
+    a slot with at < 0 has no row and adds nothing (``at`` is full: none has)."""
+    at, full = at
+    T, k = at.shape
+    rows = (at if full else at.clamp_min(0)).view(-1)
+    yk = y.index_select(0, rows).view(T, k, y.shape[1])
+    if weight is not None:
+        yk = yk * weight
+    if not full:
+        yk = torch.where((at >= 0).unsqueeze(-1), yk, torch.zeros_like(yk))
+    return yk.sum(1)
+
+
+class _GatherRows(torch.autograd.Function):
+    """x[rows], every expert's rows; the gradient gathers a token's slots in order
+    (index_select's own would add them up with atomics)."""
+
+    @staticmethod
+    def forward(ctx, x, rows, at, full):
+        ctx.save_for_backward(at)
+        ctx.full = full
+        return x.index_select(0, rows)
+
+    @staticmethod
+    def backward(ctx, dy):
+        return _sum_slots(dy, (ctx.saved_tensors[0], ctx.full)), None, None, None
+
+
 class SwiFFN(nn.Module):
     """model.py:282-290: down((silu(gate(x).float()) * up(x).float()).to(x.dtype))."""
 
@@ -83,7 +139,7 @@ class SwiFFN(nn.Module):
             xf = x if x.is_floating_point() else x.float()
             return be.swiffn_forward(xf, self.buffers6(), self.gate.tile)
         odt = x.dtype if x.is_floating_point() else torch.float32
-        return self.down((F.silu(self.gate(x).float()) * self.up(x).float()).to(odt))
+        return self.down(_swiglu(self.gate(x), self.up(x), odt))
 
     def buffers6(self):
         # straight from the modules' dictionaries: nine attribute searches per
@@ -182,6 +238,17 @@ class SwiFFN_MoE(nn.Module):
         self.last_topi = topi.detach().view(*lead, self.top_k)
         total = topv.sum(-1, keepdim=True)
         topv = torch.where(total < 1e-6, torch.full_like(topv, 1.0 / self.top_k), topv / total.clamp_min(1e-9))
+        if xs.is_cuda and 0 < xs.shape[0] * self.top_k < 1 << 31 and self.num_experts <= 64 and self.top_k <= 8 and \
+                hasattr(get_backend(), "moe_dispatch"):
+            out, counts = self._experts_dispatched(xs, topi, topv)
+        else:
+            out, counts = self._experts_by_mask(xs, topi, topv)
+        self.expert_token_counts = counts
+        return out.view(x.shape).to(x.dtype if x.is_floating_point() else torch.float32)
+
+    def _experts_by_mask(self, xs, topi, topv):
+        """The experts' weighted outputs [T, d] fp32 and token counts, each expert's
+        rows found by its own mask (a host synchronisation per expert)."""
         out = torch.zeros(xs.shape, dtype=torch.float32, device=xs.device)
         counts = []
         for e, expert in enumerate(self.experts):
@@ -191,8 +258,24 @@ class SwiFFN_MoE(nn.Module):
             if counts[-1]:
                 y = expert(xs.index_select(0, rows)).float() * weight.index_select(0, rows).unsqueeze(-1)
                 out = out.index_add(0, rows, y)
-        self.expert_token_counts = counts
-        return out.view(x.shape).to(x.dtype if x.is_floating_point() else torch.float32)
+        return out, counts
+
+    def _experts_dispatched(self, xs, topi, topv):
+        """The same from the backend's dispatch: one synchronisation, one gather of
+        every expert's rows (ascending tokens, as the masks give them) and, per
+        token, its experts' outputs in ascending expert order."""
+        T, k = topi.shape
+        disp = get_backend().moe_dispatch(topi, topv.detach(), self.num_experts, 64)
+        counts = disp["counts"].tolist()
+        n = sum(counts)
+        if n == 0:
+            return torch.zeros(xs.shape, dtype=torch.float32, device=xs.device), counts
+        order = topi.argsort(-1) if k > 1 else torch.zeros_like(topi)
+        at = disp["inv"][:T * k].view(T, k).gather(1, order)  # the slots' rows, by expert
+        full = n == T * k
+        rows = _GatherRows.apply(xs, disp["perm_row"][:n], at, full).split(counts)
+        y = torch.cat([expert(r) for expert, r in zip(self.experts, rows) if r.shape[0]]).float()
+        return _sum_slots(y, (at, full), topv.gather(1, order).unsqueeze(-1)), counts
 
     def routing_stats(self) -> dict:
         counts = list(self.expert_token_counts)

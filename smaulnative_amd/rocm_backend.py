@@ -227,6 +227,30 @@ class RocmBackend:
                                            x.shape[1], gw.shape[0], int(bool(fresh)), _stream_handle(g.device))
         _lib.check(rc, "fp8_weight_grad")
 
+    def swiglu(self, gate, up):
+        """silu(gate) * up (model.py:289-290) in the tensors' dtype, computed in fp32."""
+        return self._swiglu_call("swiglu", (gate, up), 1)[0]
+
+    def swiglu_backward(self, dout, gate, up):
+        """(dgate, dup) of ``swiglu`` from the gradient of its output."""
+        return self._swiglu_call("swiglu_backward", (dout, gate, up), 2)
+
+    @staticmethod
+    def _swiglu_call(name, ins, outs):
+        lib = _lib.load()
+        _need_device(name, *ins)
+        dtype, shape, dev = ins[0].dtype, ins[0].shape, ins[0].device
+        if dtype not in _ACT or any(t.dtype != dtype or t.shape != shape for t in ins):
+            raise RuntimeError(f"{name}: float32 or bfloat16 tensors of one shape expected, got "
+                               f"{[(t.dtype, tuple(t.shape)) for t in ins]}")
+        ins = [t if t.is_contiguous() else t.contiguous() for t in ins]
+        res = [torch.empty(shape, dtype=dtype, device=dev) for _ in range(outs)]
+        with _device(dev):
+            rc = getattr(lib, "smaul_" + name)(*[t.data_ptr() for t in ins], *[t.data_ptr() for t in res],
+                                               ins[0].numel(), _ACT[dtype], _stream_handle(dev))
+        _lib.check(rc, name)
+        return res
+
     def fp8_quantize_tiles(self, w32, tile):
         """(codes uint8 [out_f, nt*tile], scales fp32 [out_f, nt], non-finite count) on the device.
 

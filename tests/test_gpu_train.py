@@ -203,3 +203,61 @@ def test_moe_training_step_vs_reference():
     print({k: f"{v:.2e}" for k, v in errs.items()}, flush=True)
     for k, v in errs.items():
         assert v <= 2e-3, (k, v)
+
+
+@pytest.mark.parametrize("T,E,k,dtype", [(1, 4, 2, torch.float32), (70, 8, 3, torch.bfloat16),
+                                         (257, 5, 1, torch.float32), (130, 2, 2, torch.float32)])
+def test_training_dispatch_is_the_masked_loop(T, E, k, dtype):
+    """The experts of a training step through the backend's dispatch against the
+    loop over masks: outputs, counts and the gradients of x and of the routing
+    weights, with slots of zero weight (no row) and an expert without a token.
+    The same rows go through the same kernels, each token's k products added in
+    the same order: fp32 rounding of k terms apart (k = 3, 2^-22)."""
+    print(f"case training dispatch T={T} E={E} k={k} {dtype}", flush=True)
+    torch.manual_seed(T + E)
+    moe = SwiFFN_MoE(MoEConfig(d_model=128, ffn_mult=2.5, tile=64, num_experts=E, num_experts_per_tok=k)).to(DEV)
+    moe.train()
+    topi = torch.stack([torch.randperm(max(k, E - 1), device=DEV)[:k] for _ in range(T)])
+    w0 = torch.rand(T, k, device=DEV)
+    if T > 64:
+        w0[::7, 0] = 0.0
+    x0 = torch.randn(T, 128, device=DEV).to(dtype)
+    c = torch.randn(T, 128, device=DEV)
+    got = []
+    for f in (moe._experts_by_mask, moe._experts_dispatched):
+        for ex in moe.experts:
+            for m in (ex.gate, ex.up, ex.down):
+                m._gw = None
+        x, w = x0.clone().requires_grad_(True), w0.clone().requires_grad_(True)
+        out, counts = f(x, topi, w)
+        (out * c).sum().backward()
+        gws = [None if m._gw is None else m._gw.clone() for ex in moe.experts for m in (ex.gate, ex.up, ex.down)]
+        got.append((out.detach(), x.grad, torch.where(w0 > 0, w.grad, torch.zeros_like(w0)), counts, gws))
+    (o0, gx0, gw0, c0, g0), (o1, gx1, gw1, c1, g1) = got
+    assert c0 == c1 and sum(c0) == int((w0 > 0).sum())
+    bar = 2.0 ** -22 if dtype == torch.float32 else 2.0 ** -7   # x.grad is rounded to bf16 per term or once
+    assert rel(o1, o0) <= 2.0 ** -22 and rel(gw1, gw0) < 1e-5 and rel(gx1, gx0) <= 4 * bar
+    for a, b in zip(g0, g1):
+        assert (a is None) == (b is None) and (a is None or torch.equal(a, b))
+
+
+@pytest.mark.parametrize("shape,dtype", [((3, 5), torch.float32), ((257, 1280), torch.float32),
+                                         ((64, 640), torch.bfloat16), ((0, 64), torch.float32)])
+def test_swiglu_vs_float64(shape, dtype):
+    """The training path's SwiGLU product and gradients against float64: a few
+    fp32 roundings (2^-20 of the largest value), then the dtype's."""
+    from smaulnative_amd.compute import get_backend
+    print(f"case swiglu {shape} {dtype}", flush=True)
+    torch.manual_seed(5)
+    g, u, d = ((3 * torch.randn(shape, device=DEV)).to(dtype) for _ in range(3))
+    be = get_backend("rocm")
+    out = be.swiglu(g, u)
+    dg, du = be.swiglu_backward(d, g, u)
+    g64, u64 = g.double().requires_grad_(True), u.double().requires_grad_(True)
+    ref = F.silu(g64) * u64
+    ref.backward(d.double())
+    step = 0.0 if dtype == torch.float32 else 2.0 ** -8
+    for a, r in ((out, ref.detach()), (dg, g64.grad), (du, u64.grad)):
+        assert a.dtype == dtype and a.shape == r.shape
+        if a.numel():
+            assert bool(((a.double() - r).abs() <= step * r.abs() + 2.0 ** -20 * r.abs().max()).all())
