@@ -7,8 +7,8 @@
 // the reference's native kernel kernel/fp8_cpu.cpp:167-259.  Training only;
 // not on the forward path.
 //
-// Two kernels, each a workgroup per 64 x 64 tile of dx walking the output
-// dimension o in chunks of 32, whose sums over o run in another order than
+// Two kernels, each a workgroup per 64 x 64 (or 32 x 64) tile of dx walking the
+// output dimension o in chunks, whose sums over o run in another order than
 // the reference's eight-way split: results agree to fp32 rounding (relative
 // 1e-6), not bitwise.
 //  - fp8_backward_input_mfma_kernel (tile a multiple of 64, so the tile's 64
@@ -63,26 +63,30 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // Four waves, each 32 rows x 32 columns of the tile (v_mfma_f32_32x32x16_bf16:
 // lane l holds row / column l % 32 of the operands at k = 8 (l / 32) + 0..7,
 // and column l % 32, rows (r / 4) 8 + (l / 32) 4 + r % 4 of the sums).  Per
-// chunk of BWM_K = 64 o: every thread turns 16 values of g * s (one row, 16
+// chunk of BK o: every thread turns 16 values of g * s (one row, 16
 // consecutive o) into their three bf16 terms and writes them to LDS, and
 // transposes a 4 x 4 block of codes (4 o x 4 columns, v_perm) into four
 // column words of 4 o; the loads of the next chunk are issued before the
 // chunk's MFMAs.  VEC: g rows and code rows are
 // 16-byte aligned and whole chunks are in range (out_f % 64 == 0, in_f % 64
 // == 0), so they load as 16-byte vectors.
-constexpr int BWM_K = 64;
-
-template <bool CANON, bool VEC>
+//
+// BM = 64: the four waves are 2 x 2 over the tile, chunks of 64 o.  BM = 32, for
+// grids that leave CUs without a tile: two waves over the columns and two over
+// the halves of a chunk of 128 o (their sums meet in LDS), so a tile takes half
+// the steps and there are twice as many.
+template <bool CANON, bool VEC, int BM>
 __global__ void __launch_bounds__(256)
 fp8_backward_input_mfma_kernel(const float* __restrict__ g, const uint8_t* __restrict__ w,
                                const float* __restrict__ s, float* __restrict__ dx, int64_t rows, int64_t in_f,
                                int64_t out_f, int64_t tile, int64_t nt) {
-  __shared__ __attribute__((aligned(16))) uint16_t sa[3][BW_T][BWM_K + 8];  // terms of g * s, [row][o]
-  // codes, [column][o]; rows of 72 bytes: the word writes of a wave meet at
-  // most two to a bank, the 8-byte fragment reads none
-  __shared__ __attribute__((aligned(16))) uint8_t sw[BW_T][BWM_K + 8];
+  constexpr int BK = 4096 / BM;  // o per chunk
+  __shared__ __attribute__((aligned(16))) uint16_t sa[3][BM][BK + 8];  // terms of g * s, [row][o]
+  // codes, [column][o]; rows of 72 (136) bytes: the word writes of a wave meet
+  // at most two to a bank, the 8-byte fragment reads none
+  __shared__ __attribute__((aligned(16))) uint8_t sw[BW_T][BK + 8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = BM == 64 ? wave >> 1 : 0, wn = wave & 1, wk = BM == 64 ? 0 : wave >> 1;
   // Workgroup b runs on XCD b % 8: each XCD takes a contiguous band of the
   // tiles in row order, so the column tiles that read the same g rows share
   // one L2 (in launch order they went to eight L2s, with a 38 % hit rate at
@@ -92,16 +96,17 @@ fp8_backward_input_mfma_kernel(const float* __restrict__ g, const uint8_t* __res
     const int64_t nc = gridDim.x, total = nc * gridDim.y, full = (total / 8) * 8;
     int64_t lin = (int64_t)blockIdx.y * nc + blockIdx.x;
     if (lin < full) lin = (lin % 8) * (full / 8) + lin / 8;
-    r0 = (lin / nc) * BW_T;
+    r0 = (lin / nc) * BM;
     c0 = (lin % nc) * BW_T;
   }
   const int64_t kb = c0 / tile;
   // this thread's staging: g row ar, 16 o from ao; codes of o wo..wo+3 x columns wc..wc+3
-  const int ar = tid >> 2, ao = (tid & 3) * 16;
-  const int wo = (tid >> 4) * 4, wc = (tid & 15) * 4;
+  constexpr int TPR = BK / 16, NC = BK / 64;  // threads per g row, code blocks per thread
+  const int ar = tid / TPR, ao = (tid % TPR) * 16;
+  const int wo = (tid >> 4) * 4, wc = (tid & 15) * 4;  // code block b: o + 64 b
   const int64_t gr = r0 + ar;
   float gv[16], sv[16];
-  uint32_t cw[4];  // row wo + r, columns wc..wc+3 (byte c = column wc + c)
+  uint32_t cw[NC][4];  // row wo + r, columns wc..wc+3 (byte c = column wc + c)
   auto load = [&](int64_t o0) {
     if constexpr (VEC) {
       const float4* gp = (const float4*)(g + (gr < rows ? gr : rows - 1) * out_f + o0 + ao);
@@ -113,13 +118,17 @@ fp8_backward_input_mfma_kernel(const float* __restrict__ g, const uint8_t* __res
         gv[4 * q + 2] = v.z;
         gv[4 * q + 3] = v.w;
       }
-      // the wave's lanes hold the chunk's 64 scales, lane l that of o = (l & 3) * 16 + (l >> 2),
-      // and each lane gathers its 16 (ao = (l & 3) * 16) with cross-lane reads
-      const float sl = s[(o0 + (lane & 3) * 16 + (lane >> 2)) * nt + kb];
+      // the wave's lanes hold the chunk's scales, lane l those of o = (l % TPR) * 16 + l / TPR
+      // (+ 8), and each lane gathers its 16 (ao = (l % TPR) * 16) with cross-lane reads
+      float sl[NC];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) sv[j] = __shfl(sl, (j << 2) | (lane & 3), 64);
+      for (int q = 0; q < NC; ++q) sl[q] = s[(o0 + (lane % TPR) * 16 + lane / TPR + 8 * q) * nt + kb];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) cw[r] = *(const uint32_t*)(w + (o0 + wo + r) * in_f + c0 + wc);
+      for (int j = 0; j < 16; ++j) sv[j] = __shfl(sl[NC == 1 ? 0 : j >> 3], (j % (16 / NC)) * TPR | (lane % TPR), 64);
+#pragma unroll
+      for (int b = 0; b < NC; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) cw[b][r] = *(const uint32_t*)(w + (o0 + 64 * b + wo + r) * in_f + c0 + wc);
     } else {
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
@@ -128,23 +137,25 @@ fp8_backward_input_mfma_kernel(const float* __restrict__ g, const uint8_t* __res
         sv[j] = o < out_f ? s[o * nt + kb] : 0.0f;
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t o = o0 + wo + r;
-        uint32_t v = 0;
+      for (int b = 0; b < NC; ++b)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int64_t i = c0 + wc + c;
-          v |= ((o < out_f && i < in_f) ? (uint32_t)w[o * in_f + i] : 0u) << (8 * c);  // code 0 decodes to +0
+        for (int r = 0; r < 4; ++r) {
+          const int64_t o = o0 + 64 * b + wo + r;
+          uint32_t v = 0;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const int64_t i = c0 + wc + c;
+            v |= ((o < out_f && i < in_f) ? (uint32_t)w[o * in_f + i] : 0u) << (8 * c);  // code 0 decodes to +0
+          }
+          cw[b][r] = v;
         }
-        cw[r] = v;
-      }
     }
   };
   f32x16_t acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
   load(0);
-  for (int64_t o0 = 0; o0 < out_f; o0 += BWM_K) {
+  for (int64_t o0 = 0; o0 < out_f; o0 += BK) {
     {
       uint32_t t[3][8];
 #pragma unroll
@@ -164,20 +175,23 @@ fp8_backward_input_mfma_kernel(const float* __restrict__ g, const uint8_t* __res
       }
       // 4 x 4 byte transpose: column word c = (row 0 byte c, ..., row 3 byte c)
       // (v_perm: selector bytes 0-3 pick from the second operand, 4-7 from the first)
-      const uint32_t lo01 = __builtin_amdgcn_perm(cw[1], cw[0], 0x05010400u);
-      const uint32_t hi01 = __builtin_amdgcn_perm(cw[1], cw[0], 0x07030602u);
-      const uint32_t lo23 = __builtin_amdgcn_perm(cw[3], cw[2], 0x05010400u);
-      const uint32_t hi23 = __builtin_amdgcn_perm(cw[3], cw[2], 0x07030602u);
-      *(uint32_t*)&sw[wc + 0][wo] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
-      *(uint32_t*)&sw[wc + 1][wo] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
-      *(uint32_t*)&sw[wc + 2][wo] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
-      *(uint32_t*)&sw[wc + 3][wo] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+#pragma unroll
+      for (int b = 0; b < NC; ++b) {
+        const uint32_t lo01 = __builtin_amdgcn_perm(cw[b][1], cw[b][0], 0x05010400u);
+        const uint32_t hi01 = __builtin_amdgcn_perm(cw[b][1], cw[b][0], 0x07030602u);
+        const uint32_t lo23 = __builtin_amdgcn_perm(cw[b][3], cw[b][2], 0x05010400u);
+        const uint32_t hi23 = __builtin_amdgcn_perm(cw[b][3], cw[b][2], 0x07030602u);
+        *(uint32_t*)&sw[wc + 0][64 * b + wo] = __builtin_amdgcn_perm(lo23, lo01, 0x05040100u);
+        *(uint32_t*)&sw[wc + 1][64 * b + wo] = __builtin_amdgcn_perm(lo23, lo01, 0x07060302u);
+        *(uint32_t*)&sw[wc + 2][64 * b + wo] = __builtin_amdgcn_perm(hi23, hi01, 0x05040100u);
+        *(uint32_t*)&sw[wc + 3][64 * b + wo] = __builtin_amdgcn_perm(hi23, hi01, 0x07060302u);
+      }
     }
     __syncthreads();
-    if (o0 + BWM_K < out_f) load(o0 + BWM_K);
+    if (o0 + BK < out_f) load(o0 + BK);
 #pragma unroll
-    for (int ks = 0; ks < BWM_K / 16; ++ks) {
-      const int ob = ks * 16 + (lane >> 5) * 8;
+    for (int ks = 0; ks < 4; ++ks) {
+      const int ob = wk * 64 + ks * 16 + (lane >> 5) * 8;
       const int fr = wm * 32 + (lane & 31), fc = wn * 32 + (lane & 31);
       const uint2 c = *(const uint2*)&sw[fc][ob];
       uint32_t d[4];
@@ -189,6 +203,18 @@ fp8_backward_input_mfma_kernel(const float* __restrict__ g, const uint8_t* __res
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8_t*)&sa[p][fr][ob], bf, acc, 0, 0, 0);
     }
     __syncthreads();
+  }
+  if constexpr (BM == 32) {  // the upper half's sums to the lower half's wave, through sa
+    float* part = (float*)&sa[0][0][0];
+    static_assert(sizeof(sa) >= 2 * 16 * 64 * 4, "partial sums fit the staging rows");
+    if (wk == 1) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) part[(wn * 16 + r) * 64 + lane] = acc[r];
+    }
+    __syncthreads();
+    if (wk == 1) return;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = acc[r] + part[(wn * 16 + r) * 64 + lane];
   }
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
@@ -262,8 +288,8 @@ fp8_backward_input_kernel(const float* __restrict__ g, const uint8_t* __restrict
 // v_mfma_f32_32x32x2_f32.  That instruction wants, per lane, one o (or i) of
 // one row, and g and x are row-major: a wave's operand is two rows' 32
 // consecutive values as they lie in memory, so both go from global memory to
-// registers without LDS.  A workgroup owns 64 x 64 outputs; each of its four
-// waves all of them over every fourth chunk of WG_U row pairs (the next
+// registers without LDS.  A workgroup owns 32 NT x 32 NT outputs; each of its
+// four waves all of them over every fourth chunk of WG_U row pairs (the next
 // chunk's loads in flight), and the four partial sums meet in LDS in wave
 // order.
 //
@@ -272,7 +298,6 @@ fp8_backward_input_kernel(const float* __restrict__ g, const uint8_t* __restrict
 // 1024 rows, 1280 x 512: one launch of 28 us (46 TFLOP/s; 4096 rows 87 us, 62)
 // against 20 library GEMMs of 64 output rows and 20 adds, 424 us; the error
 // against float64 is that of the bf16 rounding, 1.66e-3, both ways.
-constexpr int WG_T = 64;
 constexpr int WG_U = 8;   // row pairs whose operands are loaded together
 
 template <typename X>
@@ -283,31 +308,32 @@ __device__ __forceinline__ float wg_load(const X* p) {
     return bf2f(*p);
 }
 
-template <typename X>
+template <typename X, int NT>
 __global__ void __launch_bounds__(256)
 fp8_weight_grad_kernel(const float* __restrict__ g, const X* __restrict__ x, uint16_t* __restrict__ gw, int64_t rows,
                        int64_t out_f, int64_t in_f, int fresh) {
-  __shared__ float part[4][64][64];  // [wave][accumulator][lane]
+  constexpr int WG_T = 32 * NT;             // outputs of a side
+  __shared__ float part[4][16 * NT * NT][64];  // [wave][accumulator][lane]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t o0 = (int64_t)blockIdx.y * WG_T, i0 = (int64_t)blockIdx.x * WG_T;
   // outputs past the edge read the last column and are not stored; offsets
   // from the first row of a pair (a lane of the upper half is one row on)
-  int64_t oc[2], ic[2];
+  int64_t oc[NT], ic[NT];
 #pragma unroll
-  for (int p = 0; p < 2; ++p) {
+  for (int p = 0; p < NT; ++p) {
     const int64_t o = o0 + p * 32 + (lane & 31), i = i0 + p * 32 + (lane & 31);
     oc[p] = (o < out_f ? o : out_f - 1) + (lane >> 5) * out_f;
     ic[p] = (i < in_f ? i : in_f - 1) + (lane >> 5) * in_f;
   }
-  f32x16_t acc[2][2];
+  f32x16_t acc[NT][NT];
 #pragma unroll
-  for (int p = 0; p < 2; ++p)
+  for (int p = 0; p < NT; ++p)
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int q = 0; q < NT; ++q)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[p][q][r] = 0.0f;
-  float a[2][WG_U][2], b[2][WG_U][2];
+  float a[2][WG_U][NT], b[2][WG_U][NT];
   const int64_t chunks = (rows + 2 * WG_U - 1) / (2 * WG_U);
   auto load = [&](int set, int64_t c) {
     const int64_t r0 = c * 2 * WG_U;
@@ -317,7 +343,7 @@ fp8_weight_grad_kernel(const float* __restrict__ g, const X* __restrict__ x, uin
 #pragma unroll
       for (int u = 0; u < WG_U; ++u, gr += 2 * out_f, xr += 2 * in_f)
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
+        for (int p = 0; p < NT; ++p) {
           a[set][u][p] = gr[oc[p]];
           b[set][u][p] = wg_load(xr + ic[p]);
         }
@@ -327,7 +353,7 @@ fp8_weight_grad_kernel(const float* __restrict__ g, const X* __restrict__ x, uin
     for (int u = 0; u < WG_U; ++u, gr += 2 * out_f, xr += 2 * in_f) {
       const bool in = r0 + 2 * u + (lane >> 5) < rows;
 #pragma unroll
-      for (int p = 0; p < 2; ++p) {
+      for (int p = 0; p < NT; ++p) {
         a[set][u][p] = in ? gr[oc[p]] : 0.0f;
         b[set][u][p] = in ? wg_load(xr + ic[p]) : 0.0f;
       }
@@ -337,9 +363,9 @@ fp8_weight_grad_kernel(const float* __restrict__ g, const X* __restrict__ x, uin
 #pragma unroll
     for (int u = 0; u < WG_U; ++u)
 #pragma unroll
-      for (int p = 0; p < 2; ++p)
+      for (int p = 0; p < NT; ++p)
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
+        for (int q = 0; q < NT; ++q)
           acc[p][q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[set][u][p], b[set][u][q], acc[p][q], 0, 0, 0);
   };
   int64_t c = wave;
@@ -351,16 +377,16 @@ fp8_weight_grad_kernel(const float* __restrict__ g, const X* __restrict__ x, uin
     multiply(1);
   }
 #pragma unroll
-  for (int p = 0; p < 2; ++p)
+  for (int p = 0; p < NT; ++p)
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int q = 0; q < NT; ++q)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) part[wave][(p * 2 + q) * 16 + r][lane] = acc[p][q][r];
+      for (int r = 0; r < 16; ++r) part[wave][(p * NT + q) * 16 + r][lane] = acc[p][q][r];
   __syncthreads();
-  const int p = wave >> 1, q = wave & 1;  // this wave's 32 x 32 of the tile
+  // each wave finishes a quarter of the accumulators
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int n = wave * 16 + r;
+  for (int r4 = 0; r4 < 4 * NT * NT; ++r4) {
+    const int n = wave * 4 * NT * NT + r4, p = n / (16 * NT), q = n / 16 % NT, r = n % 16;
     const float sum = part[0][n][lane] + part[1][n][lane] + part[2][n][lane] + part[3][n][lane];
     const int64_t o = o0 + p * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3), i = i0 + q * 32 + (lane & 31);
     if (o < out_f && i < in_f) {
@@ -429,13 +455,22 @@ int smaul_fp8_backward_input(const float* g, const uint8_t* w, const float* s, f
   if (gx > 2147483647LL || gy > 65535) return fail(SMAUL_ERR_UNSUPPORTED, "fp8_backward_input: grid too large");
   const int64_t nt = (in_f + tile - 1) / tile;
   if (tile % BW_T == 0) {  // a dx tile's columns share one scale column
-    const bool vec = out_f % BWM_K == 0 && in_f % BW_T == 0 && ((uintptr_t)g & 15) == 0 && ((uintptr_t)w & 15) == 0;
-    if (vec)
-      hipLaunchKernelGGL((fp8_backward_input_mfma_kernel<false, true>), dim3((unsigned)gx, (unsigned)gy), dim3(256), 0,
-                         stream, g, w, s, dx, rows, in_f, out_f, tile, nt);
+    const bool vec = out_f % 64 == 0 && in_f % BW_T == 0 && ((uintptr_t)g & 15) == 0 && ((uintptr_t)w & 15) == 0;
+    // BM = 32 under four 64-row tiles per CU (64 / 32 rows, us: 64 x 640 -> 256
+    // 15.2 / 9.7, 1024 x 1280 -> 512 28.4 / 18.2 (128 tiles), 500 x 2560 -> 1024
+    // 52.6 / 31.5, 2048 x 1280 -> 512 30.0 / 24.5, 4096 x 1280 -> 512 39.5 / 39.2
+    // (512), 4096 x 512 -> 1280 36.2 / 38.9 (1280))
+    const bool small = gx * gy < 1024 && (!vec || out_f % 128 == 0);
+    auto go = [&](auto kernel, int64_t grid_y) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)grid_y), dim3(256), 0, stream, g, w, s, dx, rows, in_f,
+                         out_f, tile, nt);
+    };
+    if (small)
+      vec ? go(fp8_backward_input_mfma_kernel<false, true, 32>, (rows + 31) / 32)
+          : go(fp8_backward_input_mfma_kernel<false, false, 32>, (rows + 31) / 32);
     else
-      hipLaunchKernelGGL((fp8_backward_input_mfma_kernel<false, false>), dim3((unsigned)gx, (unsigned)gy), dim3(256),
-                         0, stream, g, w, s, dx, rows, in_f, out_f, tile, nt);
+      vec ? go(fp8_backward_input_mfma_kernel<false, true, 64>, gy)
+          : go(fp8_backward_input_mfma_kernel<false, false, 64>, gy);
     return check_launch("fp8_backward_input_mfma_kernel");
   }
   hipLaunchKernelGGL(fp8_backward_input_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, stream, g, w, s, dx,
@@ -452,15 +487,23 @@ int smaul_fp8_weight_grad(const float* g, const void* x, int x_dtype, void* gw, 
     return fail(SMAUL_ERR_INVALID, "fp8_weight_grad: x must be f32 or bf16");
   if (in_f == 0 || out_f == 0 || (rows == 0 && !fresh)) return SMAUL_OK;
   if (!gw || (rows > 0 && (!g || !x))) return fail(SMAUL_ERR_INVALID, "fp8_weight_grad: null pointer");
-  const int64_t gx = (in_f + WG_T - 1) / WG_T, gy = (out_f + WG_T - 1) / WG_T;
+  const int64_t tiles = ((in_f + 63) / 64) * ((out_f + 63) / 64);
+  // 32 x 32 outputs where 64 x 64 leave half of the CUs idle (64 / 32, us: 64
+  // rows, 640 x 256 8.8 / 5.3, 1024 rows 25.0 / 10.4, 3000 rows 65.5 / 26.5; 160
+  // tiles: 1024 rows, 1280 x 512 28.6 / 29.8, 4096 rows 86 / 98)
+  const int64_t side = tiles < 128 && out_f <= 32 * 65535 ? 32 : 64;
+  const int64_t gx = (in_f + side - 1) / side, gy = (out_f + side - 1) / side;
   if (gx > 2147483647LL || gy > 65535) return fail(SMAUL_ERR_UNSUPPORTED, "fp8_weight_grad: grid too large");
   const dim3 grid((unsigned)gx, (unsigned)gy);
+  auto go = [&](auto kernel, auto* xp) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, g, xp, (uint16_t*)gw, rows, out_f, in_f, fresh);
+  };
   if (x_dtype == SMAUL_DTYPE_F32)
-    hipLaunchKernelGGL((fp8_weight_grad_kernel<float>), grid, dim3(256), 0, stream, g, (const float*)x, (uint16_t*)gw,
-                       rows, out_f, in_f, fresh);
+    side == 32 ? go(fp8_weight_grad_kernel<float, 1>, (const float*)x)
+               : go(fp8_weight_grad_kernel<float, 2>, (const float*)x);
   else
-    hipLaunchKernelGGL((fp8_weight_grad_kernel<uint16_t>), grid, dim3(256), 0, stream, g, (const uint16_t*)x,
-                       (uint16_t*)gw, rows, out_f, in_f, fresh);
+    side == 32 ? go(fp8_weight_grad_kernel<uint16_t, 1>, (const uint16_t*)x)
+               : go(fp8_weight_grad_kernel<uint16_t, 2>, (const uint16_t*)x);
   return check_launch("fp8_weight_grad_kernel");
 }
 

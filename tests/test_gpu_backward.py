@@ -40,11 +40,25 @@ def test_backward_input_vs_oracle(rows, in_f, out_f, tile):
     assert rel_max(dx, ref) < 1e-5, rel_max(dx, ref)
 
 
+@pytest.mark.parametrize("rows,in_f,out_f", [
+    # 32-row tiles and chunks of 128 (under 1024 tiles of 64 rows): a row tile's
+    # edge, out_f a multiple of 64 but not of 128, ragged both; then 64-row ones
+    (1, 64, 128), (33, 128, 640), (95, 192, 320), (40, 100, 130), (2100, 2048, 128)])
+def test_backward_input_row_tiles(rows, in_f, out_f):
+    print(f"case backward tiles rows={rows} in_f={in_f} out_f={out_f}", flush=True)
+    gen = torch.Generator().manual_seed(rows + in_f + out_f)
+    g = torch.randn(rows, out_f, generator=gen)
+    w, s = oracle.quantize_tiles(torch.randn(out_f, in_f, generator=gen) * 0.05, 64)
+    dx = get_backend("rocm").fp8_backward_input(g.to(DEV), w.to(DEV), s.to(DEV), in_f, out_f, 64)
+    assert rel_max(dx, oracle.fp8_backward_input(g, w, s, in_f, out_f, 64)) < 1e-5
+
+
 @pytest.mark.parametrize("rows,in_f,out_f,dtype", [
     # rows about the kernel's chunks of 16 (four waves take every fourth) and
     # outputs about its 64 x 64 tiles
     (1, 64, 64, torch.float32), (15, 65, 63, torch.float32), (64, 1, 129, torch.bfloat16),
-    (129, 192, 100, torch.float32), (1000, 512, 320, torch.bfloat16), (0, 40, 24, torch.float32)])
+    (129, 192, 100, torch.float32), (1000, 512, 320, torch.bfloat16), (0, 40, 24, torch.float32),
+    (70, 700, 800, torch.float32)])  # over 128 of them: 64 x 64 tiles, else 32 x 32
 def test_weight_grad_vs_float64(rows, in_f, out_f, dtype):
     """gw += g^T x in fp32, one rounding to bf16: against the float64 sum the
     fp32 sum is within rows * 2^-24 * sum |g||x| (any order), and the rounding
