@@ -100,7 +100,8 @@ def test_attn_forward_empty_and_zero_keys():
     assert torch.equal(Y.cpu(), Yr) and torch.equal(DEN.cpu(), DENr) and torch.equal(S.cpu(), Sr)
 
 
-@pytest.mark.parametrize("B,H,D", [(2, 8, 64), (1, 3, 13), (1, 2, 300)])
+@pytest.mark.parametrize("B,H,D", [(2, 8, 64), (1, 3, 13), (1, 2, 300),
+                                   (2, 1, 1), (1, 2, 16), (3, 2, 48), (1, 2, 65), (2, 2, 100), (2, 3, 128)])
 def test_attn_step_bit_exact_and_chains(B, H, D):
     """attn_step advances (S, z) in place, bit-identical to the reference step;
     prefill over T-3 tokens then 3 steps equals the forward over T tokens."""
