@@ -99,10 +99,12 @@ def _sum_slots(y, at, weight=None):
     T, k = at.shape
     rows = (at if full else at.clamp_min(0)).view(-1)
     yk = y.index_select(0, rows).view(T, k, y.shape[1])
+    if not full:  # before the product: a dropped slot's weight may be NaN, its gradients are zero
+        has = (at >= 0).unsqueeze(-1)
+        yk = torch.where(has, yk, torch.zeros_like(yk))
+        weight = weight if weight is None else torch.where(has, weight, torch.zeros_like(weight))
     if weight is not None:
         yk = yk * weight
-    if not full:
-        yk = torch.where((at >= 0).unsqueeze(-1), yk, torch.zeros_like(yk))
     return yk.sum(1)
 
 

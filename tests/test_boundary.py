@@ -186,3 +186,29 @@ def test_staged_entries_need_device_tensors():
         be.moe_stages(x, gw, None, [()] * 4, 2, 64)
     with pytest.raises(RuntimeError, match="HIP device"):
         be.moe_forward(x, gw, torch.zeros(4), [()] * 4, 2, 64)
+
+
+@pytest.mark.parametrize("poison", [float("nan"), float("inf")])
+def test_a_dropped_slot_leaves_no_gradient(poison):
+    """A slot without a row (weight 0, or NaN from a token whose router logits
+    are) adds nothing to the sum and to no other token's or expert's gradient,
+    whatever its weight or the row it is clamped to holds."""
+    from smaulnative_amd.moe import _sum_slots
+    at = torch.tensor([[0, 1], [-1, 2], [3, -1]], dtype=torch.int32)
+    y = torch.randn(4, 5)
+    w = torch.rand(3, 2, 1)
+    w[1, 0], w[2, 1] = float("nan"), 0.0
+    kept = (at >= 0).unsqueeze(-1)
+    y.requires_grad_(True)
+    w.requires_grad_(True)
+    out = _sum_slots(y, (at, False), w)
+    c = torch.randn_like(out)
+    (out * c).sum().backward()
+    ref = torch.stack([w[0, 0] * y[0] + w[0, 1] * y[1], w[1, 1] * y[2], w[2, 0] * y[3]])
+    assert torch.allclose(out, ref) and bool(torch.isfinite(y.grad).all())
+    assert bool((w.grad[~kept] == 0).all())
+    y2 = y.detach().clone()
+    y2[0, 0] = poison  # the row that an empty slot is clamped to
+    w2 = w.detach().clone().requires_grad_(True)
+    (_sum_slots(y2, (at, False), w2) * c).sum().backward()
+    assert torch.equal(w2.grad[1:], w.grad[1:])
