@@ -455,7 +455,9 @@ int smaul_fp8_backward_input(const float* g, const uint8_t* w, const float* s, f
   if (gx > 2147483647LL || gy > 65535) return fail(SMAUL_ERR_UNSUPPORTED, "fp8_backward_input: grid too large");
   const int64_t nt = (in_f + tile - 1) / tile;
   if (tile % BW_T == 0) {  // a dx tile's columns share one scale column
-    const bool vec = out_f % 64 == 0 && in_f % BW_T == 0 && ((uintptr_t)g & 15) == 0 && ((uintptr_t)w & 15) == 0;
+    // VEC reads its first chunk unguarded, so an empty sum goes to the guarded kernel
+    const bool vec = out_f > 0 && out_f % 64 == 0 && in_f % BW_T == 0 && ((uintptr_t)g & 15) == 0 &&
+                     ((uintptr_t)w & 15) == 0;
     // BM = 32 under four 64-row tiles per CU (64 / 32 rows, us: 64 x 640 -> 256
     // 15.2 / 9.7, 1024 x 1280 -> 512 28.4 / 18.2 (128 tiles), 500 x 2560 -> 1024
     // 52.6 / 31.5, 2048 x 1280 -> 512 30.0 / 24.5, 4096 x 1280 -> 512 39.5 / 39.2

@@ -146,3 +146,16 @@ def test_backward_input_zero_sizes_abi():
     torch.cuda.synchronize()
     assert torch.equal(dx.cpu(), torch.zeros(3, 5))
     assert lib.smaul_fp8_backward_input(None, None, None, dx.data_ptr(), 3, -1, 4, 64, stream) == _lib.SMAUL_ERR_INVALID
+
+
+@pytest.mark.parametrize("rows,in_f,tile", [(3, 64, 64), (70, 192, 64), (33, 128, 128), (5, 256, 32)])
+def test_backward_input_empty_sum_reads_nothing(rows, in_f, tile):
+    """out_f == 0 with in_f a multiple of 64 and null g / w / s, whose alignment
+    is that of the vector loads: dx all zeros, nothing read."""
+    from smaulnative_amd import _lib
+    lib = _lib.load()
+    print(f"case backward empty sum rows={rows} in_f={in_f} tile={tile}", flush=True)
+    dx = torch.full((rows, in_f), 7.0, device=DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.check(lib.smaul_fp8_backward_input(None, None, None, dx.data_ptr(), rows, in_f, 0, tile, stream), "out_f 0")
+    assert torch.equal(dx.cpu(), torch.zeros(rows, in_f))
