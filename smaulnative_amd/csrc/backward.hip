@@ -316,7 +316,8 @@ fp8_weight_grad_kernel(const float* __restrict__ g, const X* __restrict__ x, uin
   __shared__ float part[4][16 * NT * NT][64];  // [wave][accumulator][lane]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t o0 = (int64_t)blockIdx.y * WG_T, i0 = (int64_t)blockIdx.x * WG_T;
+  const unsigned nx = (unsigned)((in_f + WG_T - 1) / WG_T);  // the tiles in one dimension, those of a row together
+  const int64_t o0 = (int64_t)(blockIdx.x / nx) * WG_T, i0 = (int64_t)(blockIdx.x % nx) * WG_T;
   // outputs past the edge read the last column and are not stored; offsets
   // from the first row of a pair (a lane of the upper half is one row on)
   int64_t oc[NT], ic[NT];
@@ -493,10 +494,11 @@ int smaul_fp8_weight_grad(const float* g, const void* x, int x_dtype, void* gw, 
   // 32 x 32 outputs where 64 x 64 leave half of the CUs idle (64 / 32, us: 64
   // rows, 640 x 256 8.8 / 5.3, 1024 rows 25.0 / 10.4, 3000 rows 65.5 / 26.5; 160
   // tiles: 1024 rows, 1280 x 512 28.6 / 29.8, 4096 rows 86 / 98)
-  const int64_t side = tiles < 128 && out_f <= 32 * 65535 ? 32 : 64;
-  const int64_t gx = (in_f + side - 1) / side, gy = (out_f + side - 1) / side;
-  if (gx > 2147483647LL || gy > 65535) return fail(SMAUL_ERR_UNSUPPORTED, "fp8_weight_grad: grid too large");
-  const dim3 grid((unsigned)gx, (unsigned)gy);
+  const int64_t side = tiles < 128 ? 32 : 64;
+  const int64_t blocks = ((in_f + side - 1) / side) * ((out_f + side - 1) / side);
+  // a launch dimension holds fewer than 2^32 threads: 6e10 weights, of any shape
+  if (blocks >= (1LL << 32) / 256) return fail(SMAUL_ERR_UNSUPPORTED, "fp8_weight_grad: matrix too large");
+  const dim3 grid((unsigned)blocks);
   auto go = [&](auto kernel, auto* xp) {
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, g, xp, (uint16_t*)gw, rows, out_f, in_f, fresh);
   };

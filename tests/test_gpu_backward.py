@@ -159,3 +159,18 @@ def test_backward_input_empty_sum_reads_nothing(rows, in_f, tile):
     stream = torch.cuda.current_stream().cuda_stream
     _lib.check(lib.smaul_fp8_backward_input(None, None, None, dx.data_ptr(), rows, in_f, 0, tile, stream), "out_f 0")
     assert torch.equal(dx.cpu(), torch.zeros(rows, in_f))
+
+
+def test_weight_grad_of_more_rows_than_a_grid_dimension():
+    """out_f past 64 * 65535, the tiles that fit a launch's second dimension, as
+    the blocks of 64 rows took it: the last rows are computed like the first
+    (the products of two rows are exact in fp32 here, one bf16 rounding)."""
+    out_f, in_f, rows = 64 * 65535 + 65, 3, 2
+    print(f"case weight grad out_f={out_f}", flush=True)
+    gen = torch.Generator(device=DEV).manual_seed(7)
+    g = torch.randint(-8, 9, (rows, out_f), generator=gen, device=DEV).float()
+    x = torch.randint(-8, 9, (rows, in_f), generator=gen, device=DEV).float()
+    gw = torch.randint(-8, 9, (out_f, in_f), generator=gen, device=DEV).to(torch.bfloat16)
+    ref = (gw.float() + g[0, :, None] * x[0] + g[1, :, None] * x[1]).to(torch.bfloat16)
+    get_backend("rocm").fp8_weight_grad(g, x, gw)
+    assert torch.equal(gw, ref)
