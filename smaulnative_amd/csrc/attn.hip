@@ -27,6 +27,7 @@
 #include "smaul_common.h"
 
 using smaul::check_launch;
+using smaul::cu_count;
 using smaul::fail;
 
 namespace {
@@ -438,7 +439,7 @@ attn_fwd_col_kernel(const float* __restrict__ Q, const float* __restrict__ K, co
 // to run two workgroups, and beyond that more of them share the 15.
 int attn_col_width(int64_t tasks, int64_t D) {
   for (int j = 2; j < 8; j *= 2)
-    if (tasks * ((D + AC_W * j - 1) / (AC_W * j)) <= 256) return j;
+    if (tasks * ((D + AC_W * j - 1) / (AC_W * j)) <= cu_count()) return j;
   return 8;
 }
 

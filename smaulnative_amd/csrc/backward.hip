@@ -27,6 +27,7 @@
 #include "smaul_common.h"
 
 using smaul::check_launch;
+using smaul::cu_count;
 using smaul::fail;
 
 namespace {
@@ -463,7 +464,7 @@ int smaul_fp8_backward_input(const float* g, const uint8_t* w, const float* s, f
     // 15.2 / 9.7, 1024 x 1280 -> 512 28.4 / 18.2 (128 tiles), 500 x 2560 -> 1024
     // 52.6 / 31.5, 2048 x 1280 -> 512 30.0 / 24.5, 4096 x 1280 -> 512 39.5 / 39.2
     // (512), 4096 x 512 -> 1280 36.2 / 38.9 (1280))
-    const bool small = gx * gy < 1024 && (!vec || out_f % 128 == 0);
+    const bool small = gx * gy < 4 * (int64_t)cu_count() && (!vec || out_f % 128 == 0);
     auto go = [&](auto kernel, int64_t grid_y) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)grid_y), dim3(256), 0, stream, g, w, s, dx, rows, in_f,
                          out_f, tile, nt);
@@ -494,7 +495,7 @@ int smaul_fp8_weight_grad(const float* g, const void* x, int x_dtype, void* gw, 
   // 32 x 32 outputs where 64 x 64 leave half of the CUs idle (64 / 32, us: 64
   // rows, 640 x 256 8.8 / 5.3, 1024 rows 25.0 / 10.4, 3000 rows 65.5 / 26.5; 160
   // tiles: 1024 rows, 1280 x 512 28.6 / 29.8, 4096 rows 86 / 98)
-  const int64_t side = tiles < 128 ? 32 : 64;
+  const int64_t side = 2 * tiles < cu_count() ? 32 : 64;
   const int64_t blocks = ((in_f + side - 1) / side) * ((out_f + side - 1) / side);
   // a launch dimension holds fewer than 2^32 threads: 6e10 weights, of any shape
   if (blocks >= (1LL << 32) / 256) return fail(SMAUL_ERR_UNSUPPORTED, "fp8_weight_grad: matrix too large");

@@ -1,5 +1,6 @@
 // smaul_common.h -- pieces shared by the translation units of libsmaul_rocm.so:
-// the per-thread error channel behind smaul_last_error() and the launch check.
+// the per-thread error channel behind smaul_last_error(), the launch check and the
+// device's size.
 #ifndef SMAUL_COMMON_H
 #define SMAUL_COMMON_H
 
@@ -27,6 +28,19 @@ inline int check_launch(const char* what) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(SMAUL_ERR_HIP, "%s: launch failed: %s", what, hipGetErrorString(e));
   return SMAUL_OK;
+}
+
+// compute units of the current device (cached per device)
+inline int cu_count() {
+  static int cached[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (cached[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cached[dev] = n;
+  }
+  return cached[dev];
 }
 
 }  // namespace smaul

@@ -51,6 +51,7 @@ namespace {
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 using smaul::check_launch;
+using smaul::cu_count;
 using smaul::fail;
 
 // ---------------------------------------------------------------------------
@@ -2633,19 +2634,6 @@ int ds_kbw(int64_t nkb, bool swiglu) {
     if (nkb % kb == 0 && nkb / kb <= DS_WMAX) return kb;
   }
   return 0;
-}
-
-// compute units of the current device (cached per device)
-int cu_count() {
-  static int cached[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (cached[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
 }
 
 // Returns 1 when the shape has no streaming instance (the caller then runs
