@@ -19,9 +19,12 @@
 //
 // For D <= 128 (every preset of the reference: model.py:1020-1085) the forward
 // and the backward run as systolic arrays over (row, step) that keep every
-// sum's order (below); larger D (the reference accepts D <= 2048) keeps S in
-// global memory, the caller's S_out or a workspace, with one workgroup per
-// (b, h) task.
+// sum's order (below), the forward of many short tasks with a workgroup per
+// (b, h) task and S in registers (attn_use_array); larger D (the reference
+// accepts D <= 2048) keeps S in global memory, the caller's S_out or a
+// workspace, with one workgroup per task.
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "smaul_common.h"
@@ -441,6 +444,111 @@ int attn_col_width(int64_t tasks, int64_t D) {
   for (int j = 2; j < 8; j *= 2)
     if (tasks * ((D + AC_W * j - 1) / (AC_W * j)) <= cu_count()) return j;
   return 8;
+}
+
+// ---- D <= 128, many short tasks: a workgroup per task, a thread per column ---
+// Thread j owns column j (S[0..D-1][j]) and z[j] in registers; a chunk of
+// ATTN_CH steps of q/k/v is staged through LDS, its key norms computed by a
+// thread each.  A task is T * D dependent operations, but with 12 KB of LDS (25
+// for D > 64) and a wave or two a CU runs many of them at once.
+constexpr int ATTN_CH = 16;
+
+template <int DMAX>
+__global__ void __launch_bounds__(DMAX)
+attn_fwd_reg_kernel(const float* __restrict__ Q, const float* __restrict__ K, const float* __restrict__ V,
+                    float* __restrict__ Y, float* __restrict__ DEN, float* __restrict__ S_out,
+                    float* __restrict__ z_out, int64_t T, int H, int D, float eps) {
+  __shared__ __attribute__((aligned(16))) float s_q[ATTN_CH][DMAX];
+  __shared__ __attribute__((aligned(16))) float s_k[ATTN_CH][DMAX];
+  __shared__ __attribute__((aligned(16))) float s_v[ATTN_CH][DMAX];
+  __shared__ __attribute__((aligned(16))) float s_kn[DMAX];
+  __shared__ __attribute__((aligned(16))) float s_z[DMAX];
+  __shared__ float s_inv[ATTN_CH];
+  const int64_t task = blockIdx.x;
+  const int64_t b = task / H, h = task % H;
+  const int j = threadIdx.x;
+  const bool col = j < D;
+  float S[DMAX];
+#pragma unroll
+  for (int i = 0; i < DMAX; ++i) S[i] = 0.0f;
+  float zj = 0.0f;
+  const int64_t rs = (int64_t)H * D;          // stride between time steps
+  const int64_t base = (b * T * H + h) * D;   // (b, t = 0, h)
+  for (int64_t t0 = 0; t0 < T; t0 += ATTN_CH) {
+    const int nt = (int)(T - t0 < ATTN_CH ? T - t0 : ATTN_CH);
+    // stage the chunk: every thread loads its column of each step
+    if (col) {
+#pragma unroll
+      for (int tt = 0; tt < ATTN_CH; ++tt)
+        if (tt < nt) {
+          const int64_t o = base + (t0 + tt) * rs + j;
+          s_q[tt][j] = Q[o];
+          s_k[tt][j] = K[o];
+          s_v[tt][j] = V[o];
+        }
+    }
+    __syncthreads();
+    if (j < nt) s_inv[j] = attn_inv_norm(s_k[j], D);
+    __syncthreads();
+    for (int tt = 0; tt < nt; ++tt) {
+      float vj = 0.0f;
+      if (col) {
+        const float knj = s_k[tt][j] * s_inv[tt];
+        zj = zj + knj;
+        s_kn[j] = knj;
+        s_z[j] = zj;
+        vj = s_v[tt][j];
+      }
+      __syncthreads();
+      float num = 0.0f, den = 0.0f;
+#pragma unroll
+      for (int i = 0; i < DMAX; ++i) {
+        if (i < D) {
+          const float qi = s_q[tt][i];
+          S[i] = S[i] + s_kn[i] * vj;
+          num = num + qi * S[i];
+          den = den + qi * s_z[i];
+        }
+      }
+      const float denc = den < eps ? eps : den;
+      const int64_t t = t0 + tt;
+      if (col) Y[base + t * rs + j] = num / denc;
+      if (DEN && j == 0) DEN[(b * T + t) * H + h] = denc;
+      __syncthreads();  // s_kn / s_z are rewritten by the next step
+    }
+  }
+  if (col) {
+    if (S_out) {
+      float* so = S_out + task * D * D + j;
+#pragma unroll
+      for (int i = 0; i < DMAX; ++i)
+        if (i < D) so[(int64_t)i * D] = S[i];
+    }
+    if (z_out) z_out[task * D + j] = zj;
+  }
+}
+
+// Whether a forward runs as the array: the sooner end of the two, in ns, from
+// what each measures on 256 CUs.  The array's workgroups have a CU each (90 to
+// 135 KB of LDS); one takes 7500 ns (clearing the ring, the first loads and
+// norms, the drain) and its ticks, whole chunks of them.  A step of the other kernel
+// takes 1200 + 45 D ns while the CUs hide one task's latency behind others',
+// beyond that a time per task.  us, array / registers:
+//   D 64    T 1: 512 tasks 70 / 12, 16384 2189 / 43    T 4: 8 tasks 15 / 19, 128 25 / 19
+//   D 64   T 16: 128 tasks 24 / 64, 512 93 / 68, 16384 2919 / 431
+//   D 64  T 256: 8 tasks 31 / 990, 2048 928 / 1154, 16384 7382 / 6907
+//   D 128  T 64: 8 tasks 23 / 456, 512 316 / 502, 16384 10000 / 7915
+//   D 16   T 64: 8 tasks 15 / 117, 512 47 / 121, 2048 182 / 141, 16384 1440 / 826
+// (And a launch dimension holds fewer than 2^32 threads.)
+bool attn_use_array(int64_t tasks, int64_t T, int64_t D, int j, int64_t groups) {
+  if (tasks * groups >= (1LL << 32) / AC_NT) return false;
+  const int rpl = D <= 64 ? 1 : 2, ch = rpl == 1 ? AttnCol<1, 2>::CH : AttnCol<2, 2>::CH;
+  const double cus = cu_count();
+  const double tick = rpl == 1 ? (j == 2 ? 73 : j == 4 ? 94 : 156) : (j == 2 ? 116 : j == 4 ? 160 : 256);
+  const double ticks = (double)((T + (D - 1) / rpl + ch - 1) / ch * ch);
+  const double array = std::ceil(tasks * groups / cus) * (7500 + ticks * tick);
+  const double per_task = (rpl == 1 ? 0.55 + 0.0165 * D : 0.0586 * D) * 256 / cus;
+  return array < 5000 + T * std::max(1200.0 + 45.0 * D, tasks * per_task);
 }
 
 constexpr int ATTN_GTHREADS = 256;
@@ -1161,6 +1269,15 @@ int smaul_attn_forward(const float* Q, const float* K, const float* V, float* Y,
     if (T == 0 && !S_out) return SMAUL_OK;  // T == 0 with a state: the kernel writes zeros
     const int j = attn_col_width(B * H, D);
     const int64_t groups = (D + AC_W * j - 1) / (AC_W * j);
+    if (!attn_use_array(B * H, T, D, j, groups)) {
+      if (D <= 64)
+        hipLaunchKernelGGL((attn_fwd_reg_kernel<64>), grid, dim3(64), 0, stream, Q, K, V, Y, DEN, S_out, z_out, T,
+                           (int)H, (int)D, eps);
+      else
+        hipLaunchKernelGGL((attn_fwd_reg_kernel<128>), grid, dim3(128), 0, stream, Q, K, V, Y, DEN, S_out, z_out, T,
+                           (int)H, (int)D, eps);
+      return check_launch("attn_fwd_reg_kernel");
+    }
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)(B * H * groups)), dim3(AC_NT), 0, stream, Q, K, V, Y, DEN, S_out,
                          z_out, T, (int)H, (int)D, (int)groups, eps);

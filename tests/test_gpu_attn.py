@@ -86,6 +86,46 @@ def test_attn_forward_array_edges(B, T, H, D):
     assert torch.equal(S.cpu(), Sr) and torch.equal(z.cpu(), zr)
 
 
+@pytest.mark.parametrize("B,T,H,D", [
+    # many short tasks: a workgroup each, S in registers (up to 64 wide, and above), steps
+    # about the staged chunk of 16; 24 steps of 512 tasks are the array's
+    (64, 1, 8, 64), (64, 16, 8, 64), (64, 17, 8, 64), (64, 24, 8, 64), (40, 2, 9, 13), (17, 3, 31, 100),
+    (64, 5, 8, 128)])
+def test_attn_forward_many_short_tasks(B, T, H, D):
+    print(f"case attn_forward short B={B} T={T} H={H} D={D}", flush=True)
+    Q, K, V = attn_inputs(B, T, H, D, B + T + D)
+    K[0, T // 2, 0] = 0.0
+    Q[0, T // 3] = -Q[0, T // 3]
+    Yr, DENr, Sr, zr = oracle.attn_forward(Q, K, V)
+    Y, DEN, S, z = be().attn_forward(Q.to(DEV), K.to(DEV), V.to(DEV), 1e-6, True, need_state=True)
+    assert torch.equal(Y.cpu(), Yr) and torch.equal(DEN.cpu(), DENr)
+    assert torch.equal(S.cpu(), Sr) and torch.equal(z.cpu(), zr)
+
+
+def _device_us(f, passes=20):
+    f()
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    a.record()
+    for _ in range(passes):
+        f()
+    b.record()
+    b.synchronize()
+    return a.elapsed_time(b) * 1e3 / passes
+
+
+def test_attn_forward_of_one_token_prompts_is_no_dearer_than_a_step():
+    """16384 tasks of one step each: the forward reads and writes less than
+    attn_step, which moves every task's state (43 and 82 us; as the array, a
+    workgroup per CU, 2190)."""
+    B, H, D = 2048, 8, 64
+    print("case attn_forward one-token prompts", flush=True)
+    q, k, v = (t.to(DEV) for t in attn_inputs(B, 1, H, D, 3))
+    S, z = torch.zeros(B, H, D, D, device=DEV), torch.full((B, H, D), 10.0, device=DEV)
+    step = _device_us(lambda: be().attn_step(S, z, q[:, 0], k[:, 0], v[:, 0], 1e-6))
+    forward = _device_us(lambda: be().attn_forward(q, k, v, 1e-6, False))
+    assert forward < 4 * step, (forward, step)
+
+
 def test_attn_forward_empty_and_zero_keys():
     # T = 0 with the state requested: zeros (attn_cpu.cpp:176-188)
     Q, K, V = attn_inputs(2, 0, 3, 64, 1)
