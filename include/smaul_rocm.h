@@ -407,7 +407,8 @@ int smaul_attn_step(float* S, float* z, const float* q, const float* k, const fl
  * reached through the backend entry kernel/compute.py:314-322 from
  * model.py:249,262; results are bit-identical to it.  All fp32 contiguous;
  * 0 < D <= 2048, eps positive and finite (the forward's).  `workspace`:
- * smaul_attn_backward_workspace_size(B, T, H, D) bytes.  With less (or NULL)
+ * smaul_attn_backward_workspace_size(B, T, H, D) bytes (0 where the call needs
+ * none, as for many short sequences).  With less (or NULL)
  * D <= 128 still runs, on one slower kernel; D > 128 needs
  * smaul_attn_workspace_size(B, H, D, 0) bytes for the per-task state.
  */

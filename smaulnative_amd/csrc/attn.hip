@@ -528,27 +528,30 @@ attn_fwd_reg_kernel(const float* __restrict__ Q, const float* __restrict__ K, co
   }
 }
 
-// Whether a forward runs as the array: the sooner end of the two, in ns, from
-// what each measures on 256 CUs.  The array's workgroups have a CU each (90 to
-// 135 KB of LDS); one takes 7500 ns (clearing the ring, the first loads and
-// norms, the drain) and its ticks, whole chunks of them.  A step of the other kernel
-// takes 1200 + 45 D ns while the CUs hide one task's latency behind others',
-// beyond that a time per task.  us, array / registers:
+// What `workgroups` of the array measure, in ns: each has a CU to itself (90 to
+// 135 KB of LDS) and takes 7500 (clearing the ring, the first loads and norms,
+// the drain) and its ticks, whole chunks of them.
+double attn_array_ns(int64_t workgroups, int64_t T, int64_t D, int j) {
+  const int rpl = D <= 64 ? 1 : 2, ch = rpl == 1 ? AttnCol<1, 2>::CH : AttnCol<2, 2>::CH;
+  const double tick = rpl == 1 ? (j == 2 ? 73 : j == 4 ? 94 : 156) : (j == 2 ? 116 : j == 4 ? 160 : 256);
+  const int64_t cus = cu_count();
+  return (double)((workgroups + cus - 1) / cus) * (7500 + (T + (D - 1) / rpl + ch - 1) / ch * ch * tick);
+}
+
+constexpr int64_t ATTN_GRID_THREADS = 1LL << 32;  // a launch dimension holds fewer
+
+// Whether a forward runs as the array: the sooner end of the two from what they
+// measure.  A step of the other kernel takes 1200 + 45 D ns while the CUs hide
+// one task's latency behind others', beyond that a time per task.  us, array / registers:
 //   D 64    T 1: 512 tasks 70 / 12, 16384 2189 / 43    T 4: 8 tasks 15 / 19, 128 25 / 19
 //   D 64   T 16: 128 tasks 24 / 64, 512 93 / 68, 16384 2919 / 431
 //   D 64  T 256: 8 tasks 31 / 990, 2048 928 / 1154, 16384 7382 / 6907
 //   D 128  T 64: 8 tasks 23 / 456, 512 316 / 502, 16384 10000 / 7915
 //   D 16   T 64: 8 tasks 15 / 117, 512 47 / 121, 2048 182 / 141, 16384 1440 / 826
-// (And a launch dimension holds fewer than 2^32 threads.)
 bool attn_use_array(int64_t tasks, int64_t T, int64_t D, int j, int64_t groups) {
-  if (tasks * groups >= (1LL << 32) / AC_NT) return false;
-  const int rpl = D <= 64 ? 1 : 2, ch = rpl == 1 ? AttnCol<1, 2>::CH : AttnCol<2, 2>::CH;
-  const double cus = cu_count();
-  const double tick = rpl == 1 ? (j == 2 ? 73 : j == 4 ? 94 : 156) : (j == 2 ? 116 : j == 4 ? 160 : 256);
-  const double ticks = (double)((T + (D - 1) / rpl + ch - 1) / ch * ch);
-  const double array = std::ceil(tasks * groups / cus) * (7500 + ticks * tick);
-  const double per_task = (rpl == 1 ? 0.55 + 0.0165 * D : 0.0586 * D) * 256 / cus;
-  return array < 5000 + T * std::max(1200.0 + 45.0 * D, tasks * per_task);
+  if (tasks * groups >= ATTN_GRID_THREADS / AC_NT) return false;
+  const double per_task = (D <= 64 ? 0.55 + 0.0165 * D : 0.0586 * D) * 256 / cu_count();
+  return attn_array_ns(tasks * groups, T, D, j) < 5000 + T * std::max(1200.0 + 45.0 * D, tasks * per_task);
 }
 
 constexpr int ATTN_GTHREADS = 256;
@@ -880,7 +883,7 @@ attn_bwd_kernel(const float* __restrict__ dY, const float* __restrict__ Q, const
 // One workgroup per task walking 2 T dependent steps (attn_bwd_kernel, which
 // the other widths and callers without the workspace keep) takes 5004 us at B
 // 8, T 256, H 8, D 64, these four 124 us; at D = 128 (B 8, T 256, H 16) 10340
-// and 636 us.
+// and 636 us.  Many short tasks are the other way about (attn_bwd_split).
 template <int RPL, int J>
 __global__ void __launch_bounds__(AC_NT)
 attn_bwd_col_kernel(const float* __restrict__ dY, const float* __restrict__ Q, const float* __restrict__ K,
@@ -1174,9 +1177,27 @@ attn_bwd_row_kernel(const float* __restrict__ dY, const float* __restrict__ Q, c
     attn_row<M, true>(sm, dY, Q, K, V, sc, dK, T, H, groups);
 }
 
-// Whether the four-launch backward takes a head width: whole 8-lane rows of a
-// width that is instantiated (the others run attn_bwd_kernel).
-bool attn_bwd_split(int64_t D) { return D == 16 || D == 32 || D == 48 || D == 64 || D == 96 || D == 128; }
+// Whether a backward runs as the four launches: a head width of whole 8-lane
+// rows that is instantiated (the others run attn_bwd_kernel), and the sooner end
+// of the two from what they measure, in ns: 15000 and both column passes, and
+// per task and 32 rows of the row passes 45 and, a step, 0.8 + 0.0095 D (one
+// task alone 2.5 D), against attn_bwd_kernel's steps of 1200 + 300 D, or of a time
+// per task where the CUs are full.  us, four / one:
+//   D 64   T 1: 8 tasks 27 / 29, 512 202 / 31, 16384 5814 / 468    T 4: 128 tasks 77 / 87
+//   D 64  T 16: 128 tasks 81 / 318, 512 262 / 326, 2048 985 / 683, 16384 7812 / 5499
+//   D 64  T 64: 2048 tasks 1393 / 2704
+//   D 128  T 4: 128 tasks 171 / 176, 512 581 / 351, 16384 17468 / 11003    T 16: 16384 tasks 19606 / 41708
+//   D 16   T 4: 8 tasks 23 / 28, 512 80 / 28    T 16: 512 tasks 88 / 98, 2048 318 / 203    T 64: 2048 564 / 809
+bool attn_bwd_split(int64_t tasks, int64_t T, int64_t D) {
+  if (!(D == 16 || D == 32 || D == 48 || D == 64 || D == 96 || D == 128)) return false;
+  const int j = attn_col_width(2 * tasks, D);
+  const int64_t groups = (D + AC_W * j - 1) / (AC_W * j), rgroups = (D + AR_ROWS - 1) / AR_ROWS;
+  if (tasks * groups >= ATTN_GRID_THREADS / AC_NT || tasks * rgroups >= ATTN_GRID_THREADS / AR_NT) return false;
+  const double full = 256.0 / cu_count();
+  const double rows = std::max(2.5 * D * T, tasks * rgroups * (45 + T * (0.8 + 0.0095 * D)) * full);
+  const double step = std::max(1200.0 + 300.0 * D, tasks * (D <= 64 ? 0.9 + 0.31 * D : 1.23 * D) * full);
+  return 15000 + attn_array_ns(2 * tasks * groups, T, D, j) + rows < 5000 + T * step;
+}
 
 int attn_bwd_launch(const float* dY, const float* Q, const float* K, const float* V, const float* Y, const float* DEN,
                     float* dQ, float* dK, float* dV, int64_t B, int64_t T, int64_t H, int64_t D, float eps, float* ws,
@@ -1251,7 +1272,7 @@ int64_t smaul_attn_workspace_size(int64_t B, int64_t H, int64_t D, int need_stat
 
 int64_t smaul_attn_backward_workspace_size(int64_t B, int64_t T, int64_t H, int64_t D) {
   if (B < 0 || T < 0 || H < 0 || D <= 0) return -1;
-  if (attn_bwd_split(D)) return 6 * B * T * H * (int64_t)sizeof(float);
+  if (attn_bwd_split(B * H, T, D)) return 6 * B * T * H * (int64_t)sizeof(float);
   return smaul_attn_workspace_size(B, H, D, 0);
 }
 
@@ -1326,7 +1347,7 @@ int smaul_attn_backward(const float* dY, const float* Q, const float* K, const f
   if (B == 0 || H == 0 || T == 0) return SMAUL_OK;
   if (!dY || !Q || !K || !V || !Y || !DEN || !dQ || !dK || !dV)
     return fail(SMAUL_ERR_INVALID, "attn_backward: null pointer");
-  if (attn_bwd_split(D) && workspace && workspace_bytes >= smaul_attn_backward_workspace_size(B, T, H, D))
+  if (attn_bwd_split(B * H, T, D) && workspace && workspace_bytes >= smaul_attn_backward_workspace_size(B, T, H, D))
     return attn_bwd_launch(dY, Q, K, V, Y, DEN, dQ, dK, dV, B, T, H, D, eps, (float*)workspace, stream);
   const dim3 grid((unsigned)(B * H));
   if (D <= 64) {

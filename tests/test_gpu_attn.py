@@ -308,6 +308,41 @@ def test_attn_backward_split_edges(B, T, H, D):
         assert torch.equal(a.cpu(), r), name
 
 
+@pytest.mark.parametrize("B,T,H,D", [(64, 1, 8, 64), (64, 5, 4, 16), (40, 2, 8, 128), (300, 3, 8, 48),  # one kernel
+                                     (1, 2, 1, 64), (64, 24, 8, 64)])                                    # four
+def test_attn_backward_many_short_tasks(B, T, H, D):
+    """Both sides of the rule that gives many short tasks a workgroup each."""
+    from smaulnative_amd import _lib
+    print(f"case attn_backward short B={B} T={T} H={H} D={D}", flush=True)
+    four = (B, T) in ((1, 2), (64, 24))
+    assert (_lib.load().smaul_attn_backward_workspace_size(B, T, H, D) > 0) == four
+    Q, K, V = attn_inputs(B, T, H, D, B + T + D)
+    dY = torch.randn(B, T, H, D, generator=torch.Generator().manual_seed(T + D))
+    Y, DEN, _, _ = oracle.attn_forward(Q, K, V)
+    ref = oracle.attn_backward(dY, Q, K, V, Y, DEN)
+    got = be().attn_backward(*[t.to(DEV) for t in (dY, Q, K, V, Y, DEN)], 1e-6)
+    for name, a, r in zip(("dQ", "dK", "dV"), got, ref):
+        assert torch.equal(a.cpu(), r), name
+
+
+@pytest.mark.parametrize("B,T,D", [(256, 1, 64), (256, 4, 16), (64, 1, 128), (64, 64, 64)])
+def test_attn_backward_is_not_slower_than_its_one_kernel(B, T, D):
+    """The backend's call against the same without a workspace, which always is
+    the one kernel (2048 tasks of one step at D 64: 61 us, as four launches 748)."""
+    from smaulnative_amd import _lib
+    print(f"case attn_backward time B={B} T={T} D={D}", flush=True)
+    H = 8
+    q, k, v = (t.to(DEV) for t in attn_inputs(B, T, H, D, 3))
+    y, den, _, _ = be().attn_forward(q, k, v, 1e-6, True)
+    dy = torch.randn_like(y)
+    ins, outs = (dy, q, k, v, y, den), [torch.empty_like(q) for _ in range(3)]
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    one = _device_us(lambda: lib.smaul_attn_backward(*[t.data_ptr() for t in (*ins, *outs)], B, T, H, D, 1e-6, None, 0,
+                                                     stream))
+    now = _device_us(lambda: be().attn_backward(*ins, 1e-6))
+    assert now < 2 * one + 30, (now, one)
+
+
 def test_attn_backward_without_den_reruns_forward():
     """With DEN missing (the reference then falls back to autograd through its
     torch recurrence), the backend reruns the forward on the device for it:
