@@ -226,6 +226,8 @@ class RocmBackend:
             rc = lib.smaul_fp8_weight_grad(gc.data_ptr(), xc.data_ptr(), _ACT[x.dtype], gw.data_ptr(), x.shape[0],
                                            x.shape[1], gw.shape[0], int(bool(fresh)), _stream_handle(g.device))
         _lib.check(rc, "fp8_weight_grad")
+        # as an in-place torch operation does: autograd's check of saved tensors
+        torch.autograd.graph.increment_version(gw)
 
     def swiglu(self, gate, up):
         """silu(gate) * up (model.py:289-290) in the tensors' dtype, computed in fp32."""
@@ -318,6 +320,8 @@ class RocmBackend:
                                        order8.data_ptr(), mids.data_ptr(), codes.data_ptr(), scales.data_ptr(),
                                        bad.data_ptr(), _stream_handle(dev))
         _lib.check(rc, "fp8_requant")
+        if m is not None:
+            torch.autograd.graph.increment_version(m)
         return codes, scales, int(bad.item())
 
     # ---- linear attention (compute.py:265-322, attn_cpu.cpp) ---------------

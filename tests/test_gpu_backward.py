@@ -174,3 +174,23 @@ def test_weight_grad_of_more_rows_than_a_grid_dimension():
     ref = (gw.float() + g[0, :, None] * x[0] + g[1, :, None] * x[1]).to(torch.bfloat16)
     get_backend("rocm").fp8_weight_grad(g, x, gw)
     assert torch.equal(gw, ref)
+
+
+def test_kernels_that_write_in_place_bump_the_version():
+    """What autograd saved and a kernel then overwrote is noticed, as with the
+    in-place operations: the accumulated weight gradient and the Lion momentum."""
+    from smaulnative_amd import FP8Linear
+    print("case in-place versions", flush=True)
+    lin = FP8Linear(64, 32).to(DEV).train()
+    x = torch.randn(5, 64, device=DEV, requires_grad=True)
+    lin(x).sum().backward()
+    w = torch.ones(32, 64, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    held = w * lin._gw
+    lin(x).sum().backward()  # adds to _gw in place
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        held.sum().backward()
+    momentum = torch.zeros(32, 64, device=DEV)
+    held = w.float() * momentum
+    lin.fused_lion_requant(lin._gw, momentum, 1e-3, 0.1, 0.9, 0.99)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        held.sum().backward()
