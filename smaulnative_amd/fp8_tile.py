@@ -12,9 +12,9 @@ backend's ``fp8_forward`` and returns it in x's dtype (kernel/fp8_tile.py:
 163-170, 237-239).  On the rocm backend bf16 activations go to the kernel as
 they are (a bf16 value widened to fp32 is the same number).  The backward
 takes the input gradient from the backend's ``fp8_backward_input`` and, in
-training mode, adds the weight gradient to the module's bf16 ``_gw`` in
-64-row blocks -- the storage the reference's optimizers read
-(kernel/fp8_tile.py:172-197); there is no fp32 master weight.
+training mode, adds the weight gradient (one launch of the backend's kernel, or
+blocks of 64 rows) to the module's bf16 ``_gw`` -- the storage the reference's
+optimizers read (kernel/fp8_tile.py:172-197); there is no fp32 master weight.
 
 ``quantize_tiles`` gives the reference's codes and scales bit for bit: the
 backend's device quantizer for HIP tensors (``fp8_quantize_tiles``), and the
@@ -102,6 +102,23 @@ _REQUANT_ELEMS = 1 << 24      # fp32 values decoded at once by requant (64 MB)
 _GW_LOCK = threading.Lock()   # one for every module: it also keeps modules picklable
 
 
+def _grad_in_one_launch(rows, in_f, out_f):
+    """Whether the weight gradient takes the backend's kernel, or the 64-row blocks.
+
+    The kernel walks all rows in every tile, so few tiles over many rows leave
+    most of the device idle, while a block's library product splits the rows;
+    with three blocks or more their launches cost the blocks more than that.  us,
+    kernel / blocks, fp32: out_f 64, in_f 64, 12000 rows 73 / 138, 25000 176 /
+    146, 100000 692 / 329; out_f 16, in_f 4096, 3000 rows 25 / 29, 12000 84 /
+    52; out_f 70, in_f 100, 25000 rows 176 / 237, 100000 687 / 551; out_f 256,
+    in_f 64, 100000 rows 686 / 1311.
+    """
+    blocks = -(-out_f // _GRAD_ROWS)
+    if blocks == 1:
+        return rows < 16384 and rows * in_f < 1 << 24
+    return blocks > 2 or rows < 65536
+
+
 class _FP8Matmul(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w8, sc, in_f, out_f, tile, module):
@@ -128,7 +145,7 @@ class _FP8Matmul(torch.autograd.Function):
             # the weight gradient accumulates in the module's bf16 _gw, which the
             # reference's optimizers read and clear (kernel/fp8_tile.py:172-197):
             # g^T x is formed in fp32 and rounded once, in one launch where the
-            # backend has the kernel, else in blocks of 64 rows
+            # backend has the kernel (_grad_in_one_launch), else in blocks of 64 rows
             be = get_backend()
             xr = x.reshape(-1, in_f)
             with _GW_LOCK:  # backward passes on several threads add to one _gw
@@ -137,8 +154,13 @@ class _FP8Matmul(torch.autograd.Function):
                     gw = torch.empty(out_f, in_f, dtype=GRAD_DTYPE, device=g.device)
                 else:  # where the module moved, keep what it accumulated
                     gw = m._gw if m._gw.device == g.device else m._gw.to(g.device)
-                if g.is_cuda and hasattr(be, "fp8_weight_grad") and gw.dtype == torch.bfloat16 and gw.is_contiguous():
-                    be.fp8_weight_grad(g, xr if xr.dtype == torch.bfloat16 else xr.float(), gw, fresh)
+                if g.is_cuda and hasattr(be, "fp8_weight_grad") and gw.dtype == torch.bfloat16 and \
+                        gw.is_contiguous() and _grad_in_one_launch(g.shape[0], in_f, out_f):
+                    # the kernel reads fp32 x faster than bf16: long calls convert it
+                    # first (us, converted / not: 25000 rows, 5120 x 2048 5144 / 7490;
+                    # 1500, 512 x 1280 42 / 52; 500, 512 x 1280 19 / 18)
+                    as_is = xr.dtype == torch.bfloat16 and (g.shape[0] < 1024 or g.numel() < 1 << 20)
+                    be.fp8_weight_grad(g, xr if as_is else xr.float(), gw, fresh)
                 else:
                     if fresh:
                         gw.zero_()

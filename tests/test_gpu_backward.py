@@ -194,3 +194,30 @@ def test_kernels_that_write_in_place_bump_the_version():
     lin.fused_lion_requant(lin._gw, momentum, 1e-3, 0.1, 0.9, 0.99)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         held.sum().backward()
+
+
+@pytest.mark.parametrize("rows,in_f,out_f,dtype,kernel", [
+    # about the lines of the rule: one block of 64 rows (by rows and by rows x
+    # in_f), two, three; and bf16 x converted for the kernel, or not
+    (16383, 8, 64, torch.float32, torch.float32), (16384, 8, 64, torch.float32, None),
+    (4095, 4096, 16, torch.bfloat16, torch.bfloat16), (4096, 4096, 16, torch.bfloat16, None),
+    (65535, 24, 65, torch.bfloat16, torch.float32), (65536, 24, 65, torch.float32, None),
+    (65536, 24, 129, torch.float32, torch.float32), (1023, 70, 1100, torch.bfloat16, torch.bfloat16),
+    (1024, 70, 1024, torch.bfloat16, torch.float32)])
+def test_weight_grad_route(rows, in_f, out_f, dtype, kernel, monkeypatch):
+    """Few outputs over many rows go to the 64-row blocks (None), which a library
+    product fills the device with; both give g^T x within its fp32 sums' bound."""
+    from smaulnative_amd import FP8Linear
+    print(f"case weight grad route rows={rows} in_f={in_f} out_f={out_f} {dtype}", flush=True)
+    bk = get_backend("rocm")
+    run, took = bk.fp8_weight_grad, []
+    monkeypatch.setattr(bk, "fp8_weight_grad", lambda g, x, gw, fresh: (took.append(x.dtype), run(g, x, gw, fresh)))
+    torch.manual_seed(rows)
+    lin = FP8Linear(in_f, out_f).to(DEV).train()
+    x = torch.randn(rows, in_f, device=DEV).to(dtype).requires_grad_(True)
+    g = torch.randn(rows, out_f, device=DEV).to(dtype)
+    lin(x).backward(g)
+    assert took == ([] if kernel is None else [kernel])
+    ref = g.double().t() @ x.detach().double()
+    slack = rows * 2.0 ** -24 * (g.double().abs().t() @ x.detach().double().abs())
+    assert bool(((lin._gw.double() - ref).abs() <= slack + (ref.abs() + slack) * 2.0 ** -8).all())
