@@ -4285,12 +4285,17 @@ __global__ void __launch_bounds__(256) lin_pack_kernel(LinPack p, int64_t xblock
 // 128, fp32 27.4 against 18.2 (8), bf16 14.9 against 18.4 (8), 300 x 1024 ->
 // 1024 bf16 23.5 against 19.4 (16).  Tiles of 32 in bf16 leave half of every
 // packed block empty: 3001 x 1024 -> 768 24.7 against 34.6, so aligned ones stay.
+// So do aligned fp32 rows for at most one column tile once their row tiles are
+// half the CUs: the register-staged GEMM reads x once (4 bytes a value), the
+// packed path reads, writes and reads it (12; 100000 x 4096 -> 100 648 against 902
+// us, 20000 x 512 -> 64 25.1 against 27.9; below, 4000 x 4096 -> 100 158 against 48).
 bool lin_pack_ok(const void* x, int x_dtype, const uint8_t* w, int64_t rows, int64_t in_f, int64_t out_f,
                  int64_t tile) {
   if (rows <= 64 || rows > 32 * 65535 || kmode_of(tile) < 0) return false;
   const bool f32 = x_dtype == SMAUL_DTYPE_F32, vec = in_f % 16 == 0 && aligned16(x) && aligned16(w);
   if (tile == 64 && in_f % 64 == 0 && out_f % 128 == 0 && vec) return false;
   if (vec && !f32 && tile == 32) return false;
+  if (vec && f32 && out_f <= 128 && rows >= 64 * (int64_t)cu_count()) return false;
   if ((in_f + 63) / 64 < (!vec ? 3 : f32 ? 6 : 12)) return false;
   LinPack p{};
   int64_t wo, so;

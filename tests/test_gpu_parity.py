@@ -199,6 +199,27 @@ def test_fp8_linear_packed(rows, in_f, out_f, tile, dtype, offset):
     assert rel_max(y, ref) < bar and rel_max(plain, ref) < bar, (rel_max(y, ref), rel_max(plain, ref))
 
 
+@pytest.mark.parametrize("rows,in_f,out_f,tile,packed", [
+    (20000, 384, 100, 64, False), (20000, 384, 129, 64, True), (20001, 500, 100, 64, True), (8000, 512, 64, 128, True),
+    (20000, 512, 16, 32, False)])
+def test_fp8_linear_long_calls_of_one_column_tile(rows, in_f, out_f, tile, packed):
+    """Aligned fp32 rows for at most 128 outputs are read once by the
+    register-staged GEMM where the rows fill the device (a rule of 64 rows a
+    CU, either side of it on 126 to 311 CUs); both routes at the fp32 bar."""
+    from smaulnative_amd import _lib
+    print(f"case fp8_linear one column tile rows={rows} in_f={in_f} out_f={out_f} tile={tile}", flush=True)
+    gen = torch.Generator().manual_seed(rows + in_f + out_f)
+    x = torch.randn(rows, in_f, generator=gen)
+    w, s = oracle.quantize_tiles(torch.randn(out_f, in_f, generator=gen) * 0.05, tile)
+    xd, wd, sd = x.to(DEV), w.to(DEV), s.to(DEV)
+    need = _lib.load().smaul_fp8_linear_workspace(xd.data_ptr(), _lib.DTYPE_F32, wd.data_ptr(), rows, in_f, out_f, tile)
+    assert (need > 0) == packed
+    y = be().fp8_forward(xd, wd, sd, in_f, out_f, tile).cpu()
+    idx = torch.randperm(rows, generator=gen)[:300]
+    assert torch.isfinite(y).all()
+    assert rel_max(y[idx], oracle.fp8_forward(x[idx], w, s, in_f, out_f, tile)) < 1e-5
+
+
 def test_fp8_linear_ws_abi_fallbacks():
     """smaul_fp8_linear_ws through the C-ABI: the two-plane path with a large
     enough workspace and smaul_fp8_linear itself (the in-LDS split) without
