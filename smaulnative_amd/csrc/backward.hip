@@ -461,11 +461,15 @@ int smaul_fp8_backward_input(const float* g, const uint8_t* w, const float* s, f
     // VEC reads its first chunk unguarded, so an empty sum goes to the guarded kernel
     const bool vec = out_f > 0 && out_f % 64 == 0 && in_f % BW_T == 0 && ((uintptr_t)g & 15) == 0 &&
                      ((uintptr_t)w & 15) == 0;
-    // BM = 32 under four 64-row tiles per CU (64 / 32 rows, us: 64 x 640 -> 256
-    // 15.2 / 9.7, 1024 x 1280 -> 512 28.4 / 18.2 (128 tiles), 500 x 2560 -> 1024
-    // 52.6 / 31.5, 2048 x 1280 -> 512 30.0 / 24.5, 4096 x 1280 -> 512 39.5 / 39.2
-    // (512), 4096 x 512 -> 1280 36.2 / 38.9 (1280))
-    const bool small = gx * gy < 4 * (int64_t)cu_count() && (!vec || out_f % 128 == 0);
+    // BM = 32 under two 64-row tiles a CU, or half a one for the guarded loads,
+    // which twice the tiles repeat and which want more than one chunk to fill
+    // (64 / 32 rows, us, tiles of 64 rows in brackets): vector 1000 x 1280 -> 512
+    // (128) 26.3 / 17.0, 3000 (376) 35.2 / 28.5, 1000 x 5120 -> 2048 (512) 134 / 142,
+    // 3000 x 512 -> 1280 (940) 25.6 / 28.5; guarded 500 x 777 -> 1000 (128) 48.0
+    // / 36.6, 1000 (256) 48.1 / 48.5, 3000 x 300 -> 200 (188) 19.9 / 22.2,
+    // 20000 x 10000 -> 192 (939) 1703 / 2361, 64 x 32 -> 512 (8) 6.4 / 6.6
+    const int64_t tiles = gx * gy, cus = cu_count();
+    const bool small = vec ? out_f % 128 == 0 && tiles < 2 * cus : out_f > 64 && 2 * tiles <= cus;
     auto go = [&](auto kernel, int64_t grid_y) {
       hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)grid_y), dim3(256), 0, stream, g, w, s, dx, rows, in_f,
                          out_f, tile, nt);

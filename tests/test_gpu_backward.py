@@ -41,11 +41,24 @@ def test_backward_input_vs_oracle(rows, in_f, out_f, tile):
 
 
 @pytest.mark.parametrize("rows,in_f,out_f", [
-    # 32-row tiles and chunks of 128 (under 1024 tiles of 64 rows): a row tile's
-    # edge, out_f a multiple of 64 but not of 128, ragged both; then 64-row ones
+    # 32-row tiles and chunks of 128 (few tiles): a row tile's edge, ragged both;
+    # out_f a multiple of 64 but not of 128, and many tiles, are 64-row ones
     (1, 64, 128), (33, 128, 640), (95, 192, 320), (40, 100, 130), (2100, 2048, 128)])
 def test_backward_input_row_tiles(rows, in_f, out_f):
     print(f"case backward tiles rows={rows} in_f={in_f} out_f={out_f}", flush=True)
+    gen = torch.Generator().manual_seed(rows + in_f + out_f)
+    g = torch.randn(rows, out_f, generator=gen)
+    w, s = oracle.quantize_tiles(torch.randn(out_f, in_f, generator=gen) * 0.05, 64)
+    dx = get_backend("rocm").fp8_backward_input(g.to(DEV), w.to(DEV), s.to(DEV), in_f, out_f, 64)
+    assert rel_max(dx, oracle.fp8_backward_input(g, w, s, in_f, out_f, 64)) < 1e-5
+
+
+@pytest.mark.parametrize("rows,in_f,out_f", [
+    # either side of the lines between 32- and 64-row tiles on 256 CUs: guarded
+    # loads at 128 / 132 tiles and at one chunk of 64 or more, vectors at 511 / 512
+    (2000, 200, 300), (2050, 200, 300), (70, 512, 64 - 3), (70, 512, 64 + 3), (4640, 448, 128), (4090, 512, 256)])
+def test_backward_input_tile_rule(rows, in_f, out_f):
+    print(f"case backward rule rows={rows} in_f={in_f} out_f={out_f}", flush=True)
     gen = torch.Generator().manual_seed(rows + in_f + out_f)
     g = torch.randn(rows, out_f, generator=gen)
     w, s = oracle.quantize_tiles(torch.randn(out_f, in_f, generator=gen) * 0.05, 64)
