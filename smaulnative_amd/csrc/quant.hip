@@ -90,12 +90,13 @@ __device__ __forceinline__ float quant_weight(const QuantSrc& p, int64_t row, in
 __device__ __forceinline__ uint32_t quant_encode(float v, float sc, const float* sb, const uint8_t* so) {
   float n = v / sc;
   if (n != n) n = 0.0f;
+  if (n == 0.0f) return 0u;  // all of a tile's padding, in wide tiles whole waves of it
   n = fminf(fmaxf(n, -448.0f), 448.0f);
   const int mag = __builtin_amdgcn_cvt_pk_fp8_f32(n, n, 0, false) & 0x7f;
   int r = n < 0.0f ? 127 - mag : 128 + mag;
   while (r > 0 && sb[r - 1] >= n) --r;
   while (r < 255 && sb[r] < n) ++r;
-  return n == 0.0f ? 0u : so[r];
+  return so[r];
 }
 
 __device__ __forceinline__ float quant_scale(float amax) {
