@@ -402,7 +402,8 @@ fp8_weight_grad_kernel(const float* __restrict__ g, const X* __restrict__ x, uin
 // ---- SwiGLU product of the training path (model.py:289-290) -----------------
 // out = silu(g) * u and its gradients, fp32 arithmetic whatever the dtype, each
 // one pass where the tensor operations take two and four (with the fp32
-// intermediates between them).  HBM-bound: 3 and 5 tensors' bytes.
+// intermediates between them), every rounding where theirs is.  HBM-bound: 3 and
+// 5 tensors' bytes.
 template <typename X>
 __device__ __forceinline__ void sg_store(X* p, float v) {
   if constexpr (sizeof(X) == 4)
@@ -417,13 +418,13 @@ swiglu_kernel(const X* __restrict__ g, const X* __restrict__ u, const X* __restr
               X* __restrict__ b, int64_t n) {
   for (int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x); i < n; i += (int64_t)gridDim.x * 256) {
     const float gv = wg_load(g + i), uv = wg_load(u + i);
-    const float sig = 1.0f / (1.0f + expf(-gv));
+    const float e = 1.0f + expf(-gv), silu = gv / e;  // one rounding, where g * (1 / e) has two
     if constexpr (BACK) {
-      const float d = wg_load(dout + i);
-      sg_store(a + i, d * uv * sig * (1.0f + gv * (1.0f - sig)));
-      sg_store(b + i, d * (gv * sig));
+      const float d = wg_load(dout + i), sig = 1.0f / e;
+      sg_store(a + i, d * uv * sig * __builtin_fmaf(gv, 1.0f - sig, 1.0f));
+      sg_store(b + i, d * silu);
     } else {
-      sg_store(a + i, gv * sig * uv);
+      sg_store(a + i, silu * uv);
     }
   }
 }

@@ -261,3 +261,31 @@ def test_swiglu_vs_float64(shape, dtype):
         assert a.dtype == dtype and a.shape == r.shape
         if a.numel():
             assert bool(((a.double() - r).abs() <= step * r.abs() + 2.0 ** -20 * r.abs().max()).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("spread", [1.0, 30.0])
+def test_swiglu_is_as_near_float64_as_the_tensor_operations(dtype, spread):
+    """Product and gradients no further from float64 than the operations they
+    replace, F.silu(g.float()) * u.float() and autograd's (1 % for ties of the
+    mean): large and small sigmoids, the underflow of both, infinities."""
+    from smaulnative_amd.compute import get_backend
+    print(f"case swiglu error {dtype} {spread}", flush=True)
+    torch.manual_seed(6)
+    g, u, d = ((s * torch.randn(1 << 18, device=DEV)).to(dtype) for s in (spread, 1.0, 1.0))
+    g[:8] = torch.tensor([0.0, -0.0, 88.0, -88.0, -88.5, -104.0, float("inf"), -float("inf")], device=DEV).to(dtype)
+    be = get_backend("rocm")
+    got = (be.swiglu(g, u), *be.swiglu_backward(d, g, u))
+    gf, uf = g.clone().requires_grad_(True), u.clone().requires_grad_(True)
+    out = (F.silu(gf.float()) * uf.float()).to(dtype)
+    out.backward(d)
+    g64, u64 = g.double().requires_grad_(True), u.double().requires_grad_(True)
+    exact = F.silu(g64) * u64
+    exact.backward(d.double())
+    # relative to each value, where it is a normal number of the arithmetic
+    for a, b, x in zip(got, (out.detach(), gf.grad, uf.grad), (exact.detach(), g64.grad, u64.grad)):
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b))
+        ok = torch.isfinite(x) & (x.abs() > 1e-35)
+        mine, theirs = (((t.double() - x) / x)[ok].square().mean().sqrt() for t in (a, b))
+        print(f"  {float(mine):.4e} {float(theirs):.4e} bits differ {int((a != b).sum())}", flush=True)
+        assert float(mine) <= 1.01 * float(theirs)
