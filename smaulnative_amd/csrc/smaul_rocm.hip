@@ -3973,15 +3973,26 @@ int pick_dense_tile(bool swiglu, int64_t rows, int64_t N) {
   return tiles(64, 128) >= cus ? DT_64x128 : DT_32x128;
 }
 
+constexpr int64_t PLANES_LAUNCH_ROWS = (int64_t)CfgDmaGU64::BM * 65535;
+
 template <bool SWIGLU, bool CANON, bool OUT_F32, ActMode AM = ACT_BF16>
 int launch_dense_dma(const GemmArgs& a, int tile, hipStream_t stream) {
   const int64_t rows = a.R;
   switch (tile) {
     case DT_128x256:
-      // two planes of 128 rows would leave one workgroup per CU: 64 rows
-      if constexpr (AM == ACT_PLANES)
-        return launch_gemm_dma<CfgDmaGU64, SWIGLU, CANON, OUT_F32, AM>(a, (rows + 63) / 64, stream);
-      else
+      // two planes of 128 rows would leave one workgroup per CU: 64 rows, past
+      // the grid's 65535 row tiles in launches of that many
+      if constexpr (AM == ACT_PLANES) {
+        int rc = SMAUL_OK;
+        for (int64_t r0 = 0; r0 < rows && rc == SMAUL_OK; r0 += PLANES_LAUNCH_ROWS) {
+          GemmArgs c = a;
+          c.R = std::min(rows - r0, PLANES_LAUNCH_ROWS);
+          c.x = (const char*)a.x + r0 * a.ldx * 2;
+          c.y = (char*)a.y + r0 * a.ldy * (SWIGLU ? 2 : 4);  // planes of bf16, or fp32
+          rc = launch_gemm_dma<CfgDmaGU64, SWIGLU, CANON, OUT_F32, AM>(c, (c.R + 63) / 64, stream);
+        }
+        return rc;
+      } else
         return launch_gemm_dma<CfgDmaGU, SWIGLU, CANON, OUT_F32, AM>(a, (rows + 127) / 128, stream);
     case DT_64x256_GU:
       if constexpr (SWIGLU) return launch_gemm_dma<CfgDmaGU64, SWIGLU, CANON, OUT_F32, AM>(a, (rows + 63) / 64, stream);
@@ -4158,9 +4169,10 @@ int launch_split_planes(const float* x, uint16_t* planes, int64_t rows, int64_t 
 // 64, shapes the DMA GEMM takes): the dense tile, else -1.
 int planes_tile(int x_dtype, const void* x, const uint8_t* w, int64_t rows, int64_t in_f, int64_t out_f,
                 int64_t tile, int flags) {
-  if (x_dtype != SMAUL_DTYPE_F32 || tile != 64 || rows <= 64 || rows > DMA_SMALL_BM * 65535 || in_f % 64 != 0) return -1;
+  if (x_dtype != SMAUL_DTYPE_F32 || tile != 64 || rows <= 64 || in_f % 64 != 0) return -1;
   if ((flags & SMAUL_FLAG_TILED_LAYOUT) || !aligned16(x) || !aligned16(w) || in_f % 16 != 0) return -1;
-  return pick_dense_tile(false, rows, out_f);
+  const int dt = pick_dense_tile(false, rows, out_f);
+  return rows > PLANES_LAUNCH_ROWS && dt != DT_128x256 ? -1 : dt;  // only those are launched in parts
 }
 
 }  // namespace
@@ -4779,7 +4791,7 @@ static int dense_gemm(bool swiglu, const void* act, int act_dtype, const uint8_t
 static int swiffn_f32_planes(const float* x, const uint8_t* gw, const float* gs, const uint8_t* uw, const float* us,
                              const uint8_t* dw, const float* ds, float* out, char* ws, int64_t hdn_bytes,
                              int64_t rows, int64_t d, int64_t h, int64_t tile, int flags, hipStream_t stream) {
-  if (tile != 64 || d % 128 != 0 || h % 128 != 0 || d > h || rows <= 64 || rows > DMA_SMALL_BM * 65535) return -1;
+  if (tile != 64 || d % 128 != 0 || h % 128 != 0 || d > h || rows <= 64 || rows > PLANES_LAUNCH_ROWS) return -1;
   uint16_t* xplanes = (uint16_t*)ws;
   uint16_t* hplanes = (uint16_t*)(ws + hdn_bytes);
   GemmArgs a{};

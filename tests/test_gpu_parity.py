@@ -220,6 +220,24 @@ def test_fp8_linear_long_calls_of_one_column_tile(rows, in_f, out_f, tile, packe
     assert rel_max(y[idx], oracle.fp8_forward(x[idx], w, s, in_f, out_f, tile)) < 1e-5
 
 
+def test_fp8_linear_planes_past_one_launch():
+    """More fp32 rows than a launch of 64-row tiles takes: the two-plane GEMM in
+    two launches, rows of both and about their meeting against the oracle."""
+    from smaulnative_amd import _lib
+    cut, in_f, out_f = 64 * 65535, 64, 256
+    rows = cut + 101
+    print(f"case fp8_linear rows={rows}", flush=True)
+    x = torch.randn(rows, in_f, generator=torch.Generator(device=DEV).manual_seed(5), device=DEV)
+    w, s = oracle.quantize_tiles(torch.randn(out_f, in_f, generator=torch.Generator().manual_seed(5)) * 0.05, 64)
+    wd = w.to(DEV)
+    assert _lib.load().smaul_fp8_linear_workspace(x.data_ptr(), _lib.DTYPE_F32, wd.data_ptr(), rows, in_f, out_f,
+                                                  64) == rows * in_f * 4
+    y = be().fp8_forward(x, wd, s.to(DEV), in_f, out_f, 64)
+    idx = torch.tensor([0, 1, 63, 64, cut // 2, cut - 65, *range(cut - 3, cut + 5), rows - 65, rows - 64, rows - 1])
+    ref = oracle.fp8_forward(x[idx.to(DEV)].cpu(), w, s, in_f, out_f, 64)
+    assert rel_max(y[idx.to(DEV)].cpu(), ref) < 1e-5
+
+
 def test_fp8_linear_ws_abi_fallbacks():
     """smaul_fp8_linear_ws through the C-ABI: the two-plane path with a large
     enough workspace and smaul_fp8_linear itself (the in-LDS split) without
