@@ -2755,7 +2755,9 @@ int launch_decode(const GemmArgs& a, hipStream_t stream) {
 // selection and the renormalisation, and the block's per-expert dispatch
 // counts are written for the dispatch scan.  With a single block (T <= TB*4)
 // the same workgroup also performs the dispatch.
-template <bool XBF16, int TB, int EMAX, bool EXACT>
+// PLANES (fp32 x): the bf16 hi / lo planes of x are written on the way, by an
+// instance of its own: its stores take 20 registers, a wave of three per SIMD.
+template <bool XBF16, int TB, int EMAX, bool EXACT, bool PLANES>
 __global__ void __launch_bounds__(ROUTE_THREADS)
 router_kernel(const void* __restrict__ x, const float* __restrict__ gw, const float* __restrict__ gb,
               RouteOut o, int64_t T, int d, int E_arg, int k) {
@@ -2809,8 +2811,7 @@ router_kernel(const void* __restrict__ x, const float* __restrict__ gw, const fl
     }
     __syncthreads();
     route_fma<XBF16, TB, EMAX>(xr, sW, cw, lane, acc);
-    if constexpr (!XBF16)
-      if (o.planes) route_split<TB, EMAX>(xr, o.planes, T, tw0, c0, cw, d, lane);
+    if constexpr (PLANES) route_split<TB, EMAX>(xr, o.planes, T, tw0, c0, cw, d, lane);
   }
   {
     const int vidx = route_butterfly<TB, EMAX>(acc, lane);
@@ -4504,11 +4505,14 @@ static int launch_router(const void* x, int x_dtype, const float* gate_w, const 
   const dim3 grid((unsigned)nb), block(ROUTE_THREADS);
 #define SMAUL_ROUTE1(TB, EMAX, EXACT)                                                                     \
   if (bf)                                                                                                 \
-    hipLaunchKernelGGL((router_kernel<true, TB, EMAX, EXACT>), grid, block, 0, stream, x, gate_w, gate_b, o, \
+    hipLaunchKernelGGL((router_kernel<true, TB, EMAX, EXACT, false>), grid, block, 0, stream, x, gate_w, gate_b, o, \
+                       T, (int)d, (int)E, (int)k);                                                        \
+  else if (o.planes)                                                                                      \
+    hipLaunchKernelGGL((router_kernel<false, TB, EMAX, EXACT, true>), grid, block, 0, stream, x, gate_w, gate_b, o, \
                        T, (int)d, (int)E, (int)k);                                                        \
   else                                                                                                    \
-    hipLaunchKernelGGL((router_kernel<false, TB, EMAX, EXACT>), grid, block, 0, stream, x, gate_w, gate_b, \
-                       o, T, (int)d, (int)E, (int)k);
+    hipLaunchKernelGGL((router_kernel<false, TB, EMAX, EXACT, false>), grid, block, 0, stream, x, gate_w, gate_b, o, \
+                       T, (int)d, (int)E, (int)k);
 #define SMAUL_ROUTE(TB, EMAX)    \
   if (E == EMAX) {               \
     SMAUL_ROUTE1(TB, EMAX, true)  \
