@@ -5079,6 +5079,22 @@ static bool f32_planes_ok(int64_t T, int64_t d, int64_t h, int64_t E, int64_t ti
   return T * d * 4 < lim && hrows * h * 4 < lim && 2 * h * d < lim;
 }
 
+// Whether the router writes the planes while it holds x, or a pass of its own
+// does.  The pass is a launch and reads x again; the router's stores go out 16 or
+// 32 tokens a workgroup at a time, and cost it its third wave a SIMD.  Whole
+// layer, graph replay, us, router / pass: E 2, d 512 T 65536 248 / 259; d 1024
+// T 4096 56.6 / 54.6, T 8192 74.6 / 77.5; d 2048 T 64 51.4 / 43.2; d 128 T 16384
+// 54.4 / 49.9, T 8192 32.2 / 31.7.  E 8: d 256 T 65536 189 / 184; d 1024 T 16384
+// 134 / 143; d 2048 T 1024 61.6 / 58.7, T 8192 132 / 138.  E 16, two workgroups a
+// CU at 8192 tokens: d 512 T 4096 49.2 / 50.7, T 8192 73.5 / 68.5.  E 64, d 1024: T
+// 2048 (two) 136 / 137, T 4096 241 / 198.  One token: 1 to 2 less by the router.
+static bool route_writes_planes(int64_t T, int64_t d, int64_t E) {
+  if (E > 8) return route_blocks(T, E, d, SMAUL_DTYPE_F32) < 2 * (int64_t)cu_count();
+  if (d < 512) return T < 8192;
+  if (d >= (E <= 4 ? 1024 : 2048)) return T <= 32 || T >= (E <= 4 ? 8192 : 4096);
+  return true;
+}
+
 // The grouped gate+up and down of fp32 x (after the dispatch, on the tile
 // table of block_m rows): x as its bf16 hi / lo planes ([T][2d], which the
 // router has written on its way over x, else `split` has them made); gate+up
@@ -5235,7 +5251,8 @@ static int moe_forward_impl(const void* x, int act_dtype, const float* gate_w, c
   o.topw = topw;
   o.blockcnt = blockcnt;
   o.block_m = (int)bm;
-  o.planes = planes ? xplanes : nullptr;
+  const bool route_planes = planes && !routed && route_writes_planes(T, d, E);
+  o.planes = route_planes ? xplanes : nullptr;
   RouteOut od = o;
   od.counts = counts;
   od.seg_off = seg_off;
@@ -5346,7 +5363,8 @@ static int moe_forward_impl(const void* x, int act_dtype, const float* gate_w, c
   }
   if (planes) {
     rc = moe_f32_planes((const float*)x, xplanes, perm_row, gate_w8, gate_s, up_w8, up_s, down_w8, down_s,
-                        (uint16_t*)hdn, (float*)yperm, seg_off, tile_off, max_tiles, T, d, h, E, bm, flags, routed, stream);
+                        (uint16_t*)hdn, (float*)yperm, seg_off, tile_off, max_tiles, T, d, h, E, bm, flags,
+                        !route_planes, stream);
   } else {
     rc = smaul_moe_gate_up(x, act_dtype, perm_row, gate_w8, gate_s, up_w8, up_s, hdn, seg_off, tile_off,
                            max_tiles, E, d, h, tile, bm, flags, stream);

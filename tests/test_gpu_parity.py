@@ -625,6 +625,26 @@ def test_moe_f32_planes_row_tiles(T, d, h, E, k):
     assert torch.equal(again.cpu(), out)
 
 
+@pytest.mark.parametrize("T,d,h,E,k", [
+    # either side of the lines between the router's planes and those of a pass: short
+    # and long calls of narrow, wide and widest layers, 4, 8 and 16 experts
+    (8191, 128, 128, 4, 1), (8192, 128, 128, 4, 1), (32, 1024, 256, 4, 2), (33, 1024, 256, 4, 2),
+    (8192, 1024, 128, 2, 1), (33, 2048, 128, 8, 2), (8176, 128, 128, 16, 2), (8192, 128, 128, 16, 2)])
+def test_moe_f32_planes_by_router_or_pass(T, d, h, E, k):
+    """The layer routed within the call, and with the routing given, where a pass
+    always writes the planes: the same bits; and the oracle at the fp32 bar."""
+    print(f"case moe f32 planes by T={T} d={d} h={h} E={E} k={k}", flush=True)
+    x, gw, gb, experts = make_moe(T + d, T, d, h, E, k, torch.float32)
+    exd = to_dev_experts(experts)
+    xd, gwd, gbd = x.to(DEV), gw.to(DEV), gb.to(DEV)
+    out, _, topi, counts = be().moe_forward(xd, gwd, gbd, exd, k, 64)
+    routing = be().moe_router(xd, gwd, gbd, k)
+    assert torch.equal(be().moe_forward_norm(xd, gwd, gbd, exd, k, 64, routing=routing)[0], out)
+    ref = oracle.moe_forward(x, gw, gb, experts, k, 64)
+    assert torch.equal(topi.cpu().reshape(-1, k), ref.topi.reshape(-1, k)) and counts.tolist() == ref.counts
+    assert rel_l2(out.cpu(), ref.out) < 1e-5
+
+
 def test_moe_skewed_segments():
     """Config-5 style skew (one expert ~40 %, three < 1 %) at a reduced size."""
     x, gw, gb, experts = make_moe(55, 2048, 256, 640, 16, 2, skew=(2.2, [13, 14, 15], 4.0))
