@@ -5063,10 +5063,13 @@ __global__ void wait_timeouts_kernel(int32_t* out, int reset) {
 // latency is the launch's (whole layer, graph replay, us, 64 / 32 rows: T 1, d
 // 512, E 4 38.0 / 29.5; T 64, d 1024, E 8 65.4 / 50.2; T 300 79.9 / 71.4; at 2.7
 // workgroups a CU T 2048, d 512 73.8 / 80.1, at 3.1 T 1000, d 1024 119.1 /
-// 119.7, at 11 T 4000 302 / 326).
+// 119.7, at 11 T 4000 302 / 326).  From ten tiles an expert on few are ragged, and
+// the line lies at 1.2 (E 2, d 512, h 512, T 2000 45.6 / 37.7, T 5000 (1.27) 54.9 / 57.1; E 8, d 256, h 256, T 8000 (1.04) 51.3 / 46.6,
+// T 15000 (1.9) 69.2 / 71.6; E 4, d 2048, h 1024, T 3000 (1.6) 127.7 / 139.2).
 static int64_t planes_block_m(int64_t h, int64_t E, int64_t R) {
-  return ((R + DMA_SMALL_BM - 1) / DMA_SMALL_BM + E) * (h / 128) < 2 * (int64_t)cu_count() ? CfgDmaGU32::BM
-                                                                                           : DMA_SMALL_BM;
+  const int64_t cus = cu_count();
+  const int64_t line = R >= 10 * DMA_SMALL_BM * E ? 6 * cus / 5 : 2 * cus;
+  return ((R + DMA_SMALL_BM - 1) / DMA_SMALL_BM + E) * (h / 128) < line ? CfgDmaGU32::BM : DMA_SMALL_BM;
 }
 
 // Whether fp32 activations run the LDS-DMA grouped GEMMs over planes: tile 64,

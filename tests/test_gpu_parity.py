@@ -608,7 +608,8 @@ def test_moe_decode_c4_shape(T, skew):
 
 @pytest.mark.parametrize("T,d,h,E,k", [
     (1, 256, 640, 4, 2), (32, 256, 384, 2, 1), (33, 512, 1280, 4, 2), (200, 1024, 2560, 8, 2),  # 32-row tiles
-    (1500, 512, 1280, 4, 2), (65, 2048, 5120, 16, 3)])                                          # 64
+    (1500, 512, 1280, 4, 2), (65, 2048, 5120, 16, 3), (2049, 512, 1280, 4, 2),                  # 64
+    (640, 256, 4992, 1, 1), (639, 256, 4992, 1, 1)])  # ten 64-row tiles an expert: 64; fewer: 32
 def test_moe_f32_planes_row_tiles(T, d, h, E, k):
     """fp32 x on 32- and 64-row tiles of the two-plane GEMMs, the planes written
     by the router; and with the routing given, where a pass of its own writes
