@@ -109,7 +109,7 @@ def test_fp8_linear_bf16_inputs_vs_oracle(rows, in_f, out_f, tile):
 
 @pytest.mark.parametrize("rows,in_f,out_f,raw_codes", [
     (4096, 512, 1280, False),   # C2 gate: 64x128 tiles
-    (4096, 1280, 512, False),   # C2 down: 32x128 tiles
+    (4096, 1280, 512, False),   # C2 down: 64x128 tiles, a workgroup a CU
     (300, 256, 384, False),     # ragged last row tile
     (16384, 1024, 2560, False), # 128x256 tiles
     (512, 256, 256, True),      # every code, 0x7F/0xFF decoded on the fly
@@ -136,16 +136,17 @@ def test_fp8_linear_bf16_dma_tiles(rows, in_f, out_f, raw_codes):
 
 @pytest.mark.parametrize("rows,in_f,out_f,tile", [
     (4096, 512, 1280, 64),      # C2 gate: two bf16 planes through the 64x128 DMA tiles
-    (4096, 1280, 512, 64),      # C2 down: 32x128 tiles
+    (4096, 1280, 512, 64),      # C2 down: 64x128 tiles, a workgroup a CU
     (300, 256, 384, 64),        # ragged last row tile
-    (2048, 1024, 2560, 64),     # 128x256 tiles
+    (2048, 1024, 2560, 64),     # 64x128 tiles, 16 K blocks
+    (16400, 64, 1024, 64),      # the wide tile (64x256 of two planes): 516 of 128 rows, a ragged last one
     (512, 64, 256, 64),         # in-LDS split (<= 1024 rows), one 64-wide K block
     (1000, 1024, 2560, 64),     # in-LDS split, 64x128 tiles
     (1024, 64, 16384, 64),      # in-LDS split, 128x256 tiles
     (700, 256, 384, 64),        # in-LDS split, 32x128 tiles
     (64, 512, 256, 64),         # rows <= 64: the register-staged split kernel
     (512, 256, 200, 64),        # out_f not a multiple of 128: register-staged
-    (300, 384, 256, 128),       # tile 128: register-staged
+    (300, 384, 256, 128),       # tile 128: packed (six 64-wide blocks)
 ])
 def test_fp8_linear_fp32_two_planes(rows, in_f, out_f, tile):
     """fp32 x (what FP8Linear passes) through fp8_forward: split into bf16 hi and
@@ -172,6 +173,8 @@ def test_fp8_linear_fp32_two_planes(rows, in_f, out_f, tile):
     (65, 129, 127, 64, "f32", 0), (300, 1000, 129, 32, "f32", 0), (130, 161, 100, 32, "bf16", 0),
     (100, 321, 130, 128, "f32", 0), (257, 705, 200, 192, "bf16", 0), (66, 352, 256, 32, "f32", 0),
     (200, 384, 384, 64, "f32", 1), (90, 768, 100, 128, "bf16", 0), (5000, 200, 300, 64, "bf16", 1),
+    # the wide tiles (two planes 64x256, bf16 128x256), the last of them past out_f
+    (16400, 200, 1000, 64, "f32", 0), (16400, 200, 1000, 64, "bf16", 0),
 ])
 def test_fp8_linear_packed(rows, in_f, out_f, tile, dtype, offset):
     """The packed path against the oracle (the bars of the two dtypes) and
@@ -364,7 +367,7 @@ def test_c2_dense_swiglu_pair_full_size():
     (37, 256, 640, torch.bfloat16, 64),     # small row count: 32-row register-staged tiles
     (300, 192, 320, torch.bfloat16, 64),    # d not a multiple of 256: register-staged down
     (300, 256, 640, torch.float32, 64),     # fp32 activations: hi / lo planes through the LDS-DMA kernels
-    (1000, 1024, 2560, torch.float32, 64),  # the same with 128-row gate+up tiles
+    (1000, 1024, 2560, torch.float32, 64),  # the same, two and a half gate+up workgroups a CU
     (64, 256, 640, torch.float32, 64),      # fp32, <= 64 rows: register-staged kernels
     (300, 640, 256, torch.float32, 64),     # fp32, d > h: register-staged kernels
     (300, 192, 320, torch.float32, 64),     # fp32, d not a multiple of 128: register-staged kernels
@@ -544,10 +547,10 @@ def test_moe_golden(tag):
     (1024, 1024, 2560, 8, 2, torch.bfloat16, 64),      # config-3 shape, fewer tokens
     (600, 256, 640, 8, 3, torch.bfloat16, 64),
     (512, 512, 1280, 4, 2, torch.bfloat16, 64),        # config-1 MoE layer shape
-    (333, 256, 640, 8, 2, torch.float32, 64),          # fp32 x: hi / lo planes, 64-row LDS-DMA tiles
-    (4096, 1024, 2560, 8, 2, torch.float32, 64),       # fp32 x: planes, 128-row tiles, 128x128 down
-    (2048, 512, 1024, 8, 2, torch.float32, 64),        # fp32 x: planes, 128x256 down tiles
-    (40, 256, 640, 4, 2, torch.float32, 64),           # fp32 x, decode-sized: planes on 64-row tiles
+    (333, 256, 640, 8, 2, torch.float32, 64),          # fp32 x: hi / lo planes, 32-row LDS-DMA tiles
+    (4096, 1024, 2560, 8, 2, torch.float32, 64),       # fp32 x: planes, 64-row tiles, 64x128 down
+    (2048, 512, 1024, 8, 2, torch.float32, 64),        # fp32 x: planes, 64-row tiles, 64x128 down
+    (40, 256, 640, 4, 2, torch.float32, 64),           # fp32 x, decode-sized: planes on 32-row tiles
     (300, 192, 640, 4, 2, torch.float32, 64),          # fp32 x, d not a multiple of 128: register-staged
     (256, 256, 512, 4, 1, torch.bfloat16, 128),
     (200, 128, 320, 2, 2, torch.bfloat16, 32),
@@ -609,7 +612,8 @@ def test_moe_decode_c4_shape(T, skew):
 @pytest.mark.parametrize("T,d,h,E,k", [
     (1, 256, 640, 4, 2), (32, 256, 384, 2, 1), (33, 512, 1280, 4, 2), (200, 1024, 2560, 8, 2),  # 32-row tiles
     (1500, 512, 1280, 4, 2), (65, 2048, 5120, 16, 3), (2049, 512, 1280, 4, 2),                  # 64
-    (640, 256, 4992, 1, 1), (639, 256, 4992, 1, 1)])  # ten 64-row tiles an expert: 64; fewer: 32
+    (640, 256, 4992, 1, 1), (639, 256, 4992, 1, 1),   # ten 64-row tiles an expert: 64; fewer: 32
+    (8300, 1024, 128, 4, 2)])                         # the wide down tile (64x256), ragged segments
 def test_moe_f32_planes_row_tiles(T, d, h, E, k):
     """fp32 x on 32- and 64-row tiles of the two-plane GEMMs, the planes written
     by the router; and with the routing given, where a pass of its own writes
@@ -787,7 +791,7 @@ def test_moe_fp32_x_abi_layouts(T, d, h, layout):
     """fp32 x through the C-ABI on the caller's buffers: raw stored codes
     (0x7F/0xFF included) without SMAUL_FLAG_ALIGNED_CODES run the
     register-staged kernels; with it, and with tiled canonical copies, the
-    LDS-DMA kernels over bf16 hi / lo planes (64-row tiles at T = 700, 128-row
+    LDS-DMA kernels over bf16 hi / lo planes (32-row tiles at T = 700, 64-row
     at T = 8192).  All within the fp32 bar of the oracle."""
     from smaulnative_amd import _lib
     print(f"case moe fp32 abi T={T} d={d} h={h} {layout}", flush=True)
