@@ -980,7 +980,7 @@ attn_bwd_dk_kernel(const float* __restrict__ K, float* __restrict__ dK, int64_t 
 //
 // What bounds it: LDS reads (4 of 16 bytes per tick and wave for M = 8, all
 // rows reading the same 8 lanes' columns) about level with the 4 M VALU
-// operations per tick, on 2 T / 256 workgroups a CU.
+// operations per tick, on 2 B H D / 32 workgroups of both passes together.
 constexpr int AR_W = 4, AR_NT = (AR_W + 1) * 64, AR_CH = 16, AR_RN = 64, AR_ROWS = AR_W * 8;
 
 template <int M>

@@ -134,9 +134,9 @@ struct GemmArgs {
   int64_t R;
   int E;
   int tiled;                   // codes/scales in the tiled layout (SMAUL_FLAG_TILED_LAYOUT)
-  // The weights' K when the activations carry two K planes (the LDS-DMA GEMM
-  // of fp32 x split into bf16 hi and lo halves side by side, K = 2 * kw, the
-  // ACT_PLANES kernels); 0: the weights span K.
+  // ACT_PLANES only (0 elsewhere): the weights' K, where the activations carry
+  // two K planes, fp32 x split into bf16 hi and lo halves side by side (K = 2 *
+  // kw).  The K loop walks kw / 64 stages, each with both planes of its block.
   int64_t kw;
   // SwiGLU with fp32 output only: when > 0 the products are stored as their
   // bf16 hi / lo split (split_bf16), hi at y[row * ldy + col] and lo at
@@ -3950,6 +3950,8 @@ int launch_gemm_dma(const GemmArgs& a, int64_t m_tiles, hipStream_t stream) {
   const int64_t n_tiles = (a.N + BNO - 1) / BNO;
   if (m_tiles <= 0 || n_tiles <= 0) return SMAUL_OK;
   if (m_tiles > 65535 || n_tiles > 65535) return fail(SMAUL_ERR_UNSUPPORTED, "gemm grid too large");
+  // the other kernels walk K, twice the weights' where x carries planes
+  if (AM == ACT_PLANES ? 2 * a.kw != a.K : a.kw != 0) return fail(SMAUL_ERR_INVALID, "gemm: planes and kernel differ");
   hipLaunchKernelGGL(
       (fp8_gemm_dma_kernel<CF::BM, CF::BN, CF::WM, CF::WN, CF::NSTAGE, SWIGLU, CANON, true, OUT_F32, AM>),
       dim3((unsigned)n_tiles, (unsigned)m_tiles), dim3(CF::WM * CF::WN * 64), 0, stream, a);
@@ -4783,8 +4785,8 @@ static int dense_gemm(bool swiglu, const void* act, int act_dtype, const uint8_t
 }
 
 // SwiFFN with fp32 activations on the LDS-DMA kernels: x is split into bf16
-// hi / lo planes, gate+up runs over both (K doubled, each weight block read
-// for its hi and its lo half) and its SwiGLU epilogue, in fp32, stores the
+// hi / lo planes, gate+up runs over both (a stage holds both planes of a K
+// block, its codes read once) and its SwiGLU epilogue, in fp32, stores the
 // products already split into the two planes of hdn, over which the down
 // projection runs with fp32 output: every value the reference forms in fp32
 // stays within 2^-18 relative of it.  The planes of x go into the workspace's
@@ -5101,8 +5103,8 @@ static bool route_writes_planes(int64_t T, int64_t d, int64_t E) {
 // The grouped gate+up and down of fp32 x (after the dispatch, on the tile
 // table of block_m rows): x as its bf16 hi / lo planes ([T][2d], which the
 // router has written on its way over x, else `split` has them made); gate+up
-// over both planes of the gathered rows (K doubled, weight blocks wrapped)
-// with the SwiGLU product kept in fp32 and stored as the planes of hdn
+// over both planes of the gathered rows (a K block of both a stage) with the
+// SwiGLU product kept in fp32 and stored as the planes of hdn
 // ([R][2h], the fp32 hdn's bytes); down over those planes with fp32 output
 // into yperm.  Every value the reference forms in fp32 stays within 2^-18
 // relative of it.
