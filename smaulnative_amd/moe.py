@@ -213,9 +213,10 @@ class SwiFFN_MoE(nn.Module):
         experts = [ex.buffers6() for ex in self.experts]
         out, prob, topi, counts = be.moe_forward(x, self.gate.weight, self.gate.bias, experts,
                                                  self.top_k, self.tile)
-        # plain attributes, set past nn.Module.__setattr__ (3 us each): none is a
-        # parameter, buffer or module
-        self.__dict__.update(last_prob=prob, last_topi=topi, _counts_dev=counts)
+        # plain attributes (or a subclass's properties), set past
+        # nn.Module.__setattr__ (3 us each): none is a parameter, buffer or module
+        for name, value in (("last_prob", prob), ("last_topi", topi), ("_counts_dev", counts)):
+            object.__setattr__(self, name, value)
         return out
 
     def _forward_train(self, x):

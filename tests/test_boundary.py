@@ -212,3 +212,25 @@ def test_a_dropped_slot_leaves_no_gradient(poison):
     w2 = w.detach().clone().requires_grad_(True)
     (_sum_slots(y2, (at, False), w2) * c).sum().backward()
     assert torch.equal(w2.grad[1:], w.grad[1:])
+
+
+def test_routing_state_reaches_a_subclass_property(monkeypatch):
+    """What forward leaves on the layer goes through a property of a subclass, as
+    attribute assignment does."""
+    from smaulnative_amd import MoEConfig, SwiFFN_MoE, moe
+
+    class Watched(SwiFFN_MoE):
+        seen = []
+        last_prob = property(lambda self: self.seen[-1], lambda self, v: self.seen.append(v))
+
+    class Backend:
+        name = "stub"
+
+        def moe_forward(self, x, *rest):
+            return x, "prob", "topi", torch.zeros(2)
+
+    layer = Watched(MoEConfig(d_model=64, num_experts=2, num_experts_per_tok=1)).eval()
+    monkeypatch.setattr(moe, "get_backend", lambda: Backend())
+    with torch.no_grad():
+        layer(torch.zeros(1, 64))
+    assert layer.last_prob == "prob" and layer.last_topi == "topi" and "last_prob" not in vars(layer)
