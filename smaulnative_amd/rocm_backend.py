@@ -52,9 +52,14 @@ def _device(device):
     return _HERE if index is None or index == torch.cuda.current_device() else torch.cuda.device(index)
 
 
+# the handle without a Stream object around it (3 us a call); not a public name
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_handle(device) -> int:
-    index = torch.cuda.current_device() if device.index is None else device.index
-    return torch._C._cuda_getCurrentRawStream(index)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 class _CacheEntry(dict):

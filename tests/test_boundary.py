@@ -234,3 +234,15 @@ def test_routing_state_reaches_a_subclass_property(monkeypatch):
     with torch.no_grad():
         layer(torch.zeros(1, 64))
     assert layer.last_prob == "prob" and layer.last_topi == "topi" and "last_prob" not in vars(layer)
+
+
+def test_stream_handle_without_the_private_name(monkeypatch):
+    """A torch without the raw-handle function gives it by the public way."""
+    from smaulnative_amd import rocm_backend
+
+    class Stream:
+        cuda_stream = 77
+
+    monkeypatch.setattr(rocm_backend, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: Stream())
+    assert rocm_backend._stream_handle(torch.device("cuda", 0)) == 77
