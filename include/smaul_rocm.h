@@ -82,7 +82,7 @@ int smaul_fp8_linear(const void* x, int x_dtype, const uint8_t* w, const float* 
  * pass and runs the GEMM over both (faster for long calls).  With more than 64
  * rows, the shapes that GEMM does not take as they are (x or w unaligned,
  * other widths, scale tiles of 32 or 128 and more) are packed into the
- * workspace in the form it reads.  With a workspace smaller than
+ * workspace in the form it reads, where that is the faster.  With a workspace smaller than
  * smaul_fp8_linear_workspace says for the call, it is smaul_fp8_linear (the
  * planes alone need smaul_fp8_linear_workspace_size).  Same arguments, results
  * and errors as smaul_fp8_linear within fp32 summation order.  The packed path

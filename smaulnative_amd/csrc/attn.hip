@@ -1177,8 +1177,9 @@ attn_bwd_row_kernel(const float* __restrict__ dY, const float* __restrict__ Q, c
     attn_row<M, true>(sm, dY, Q, K, V, sc, dK, T, H, groups);
 }
 
-// Whether a backward runs as the four launches: a head width of whole 8-lane
-// rows that is instantiated (the others run attn_bwd_kernel), and the sooner end
+// Whether a backward runs as the four launches: a head width that the row pass is
+// instantiated for (whole 8-lane rows, and an even M for its vector reads; the
+// other widths run attn_bwd_kernel), and the sooner end
 // of the two from what they measure, in ns: 15000 and both column passes, and
 // per task and 32 rows of the row passes 45 and, a step, 0.8 + 0.0095 D (one
 // task alone 2.5 D), against attn_bwd_kernel's steps of 1200 + 300 D, or of a time

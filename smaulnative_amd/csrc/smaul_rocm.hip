@@ -4191,10 +4191,10 @@ namespace {
 // make a block of their 32 k twice: [hi | lo] of x against [w | w], so hi . w
 // and lo . w share the tile's scale (bf16: [x | 0]).
 //
-// What bounds it: at 3001 x 1000 -> 777 two launches and the K loop of one
-// round of tiles (35 us; the register-staged GEMM, which loads unaligned rows
-// a byte at a time, 124 us); at 16000 x 2000 -> 2000, tile 128, the GEMM
-// (318 against 749 us).
+// What bounds it: at 3001 x 1000 -> 777, tile 32, two launches (11 us) and the K
+// loop of one round of tiles, 32 stages (24 us; with the caller's workspace 32 us
+// a pass; the register-staged GEMM, which loads unaligned rows a byte at a time,
+// 123 us); at 16000 x 2000 -> 2000, tile 128, the GEMM (318 against 749 us).
 struct LinPack {
   const void* x;
   const uint8_t* w;

@@ -6,8 +6,8 @@ to the reference's own kernel.  Bar: max relative difference 1e-5 -- the
 GPU sums the output dimension in another fp32 order (the reference's own
 test holds its kernel to 1e-5 against autograd, test_linear_fp8.py:186-199).
 The module test runs FP8Linear forward + backward in training mode: the
-input gradient, and the weight gradient accumulated in bf16 ``_gw`` in
-64-row blocks (kernel/fp8_tile.py:172-197).
+input gradient, and the weight gradient accumulated in bf16 ``_gw``
+(kernel/fp8_tile.py:172-197) by the backend's kernel or in 64-row blocks.
 """
 import pytest
 import torch
