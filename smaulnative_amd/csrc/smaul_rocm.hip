@@ -134,9 +134,10 @@ struct GemmArgs {
   int64_t R;
   int E;
   int tiled;                   // codes/scales in the tiled layout (SMAUL_FLAG_TILED_LAYOUT)
-  // ACT_PLANES only (0 elsewhere): the weights' K, where the activations carry
-  // two K planes, fp32 x split into bf16 hi and lo halves side by side (K = 2 *
-  // kw).  The K loop walks kw / 64 stages, each with both planes of its block.
+  // ACT_PLANES and ACT_WRAP only (0 elsewhere): the weights' K, where the
+  // activations carry two K planes, fp32 x split into bf16 hi and lo halves side
+  // by side (K = 2 * kw).  The K loop walks kw / 64 stages, each with both planes
+  // of its block, or 2 kw / 64, the second half with the weights' blocks again.
   int64_t kw;
   // SwiGLU with fp32 output only: when > 0 the products are stored as their
   // bf16 hi / lo split (split_bf16), hi at y[row * ldy + col] and lo at
@@ -668,8 +669,9 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 
 // How the activations reach the LDS-DMA GEMM: bf16 rows; fp32 rows split in
-// LDS; or the bf16 hi and lo planes of fp32 rows, split beforehand.
-enum ActMode { ACT_BF16 = 0, ACT_X32 = 1, ACT_PLANES = 2 };
+// LDS; or the bf16 hi and lo planes of fp32 rows, split beforehand, both of a K
+// block in a stage, or (ACT_WRAP) all hi blocks and then all lo ones.
+enum ActMode { ACT_BF16 = 0, ACT_X32 = 1, ACT_PLANES = 2, ACT_WRAP = 3 };
 
 template <int BM, int BN, int WM, int WN, int NSTAGE, bool SWIGLU, ActMode AM = ACT_BF16>
 struct DmaGemmCfg {
@@ -682,7 +684,7 @@ struct DmaGemmCfg {
   // ACT_X32: the activation rows arrive as fp32 (256 B per 64-wide K block)
   // and are split in place into a bf16 hi plane and a lo plane of 128 B rows;
   // ACT_PLANES: the two planes arrive so
-  static constexpr int A_BYTES = BM * 128 * (AM != ACT_BF16 ? 2 : 1), B_BYTES = BN * 64, S_BYTES = BN * 4;
+  static constexpr int A_BYTES = BM * 128 * (AM == ACT_X32 || AM == ACT_PLANES ? 2 : 1), B_BYTES = BN * 64, S_BYTES = BN * 4;
   static constexpr int STAGE = A_BYTES + B_BYTES + S_BYTES;
   static constexpr int A_INS = A_BYTES / 1024 / NW;      // 1 KB DMA instructions per wave per stage
   static constexpr int B_INS = B_BYTES / 1024 / NW;
@@ -728,9 +730,9 @@ template <int BM, int BN, int WM, int WN, int NSTAGE, bool SWIGLU, bool CANON, b
 // with the two planes of 64 x 256).
 __global__ void __launch_bounds__(WM * WN * 64, (BM * BN <= 128 * 128 && (AM != ACT_PLANES || BM * BN <= 64 * 128) ? 3 : 2))
 fp8_gemm_dma_kernel(GemmArgs p) {
-  constexpr bool X32 = AM == ACT_X32, PLANES = AM == ACT_PLANES, TWO = X32 || PLANES;
+  constexpr bool X32 = AM == ACT_X32, PLANES = AM == ACT_PLANES, TWO = X32 || PLANES, WRAP = AM == ACT_WRAP;
   static_assert(!X32 || (OUT_F32 && !SWIGLU), "fp32 activations split in LDS are the fp8_forward path");
-  static_assert(!PLANES || OUT_F32, "planes are fp32 activations");
+  static_assert(!(PLANES || WRAP) || OUT_F32, "planes are fp32 activations");
   using C = DmaGemmCfg<BM, BN, WM, WN, NSTAGE, SWIGLU, AM>;
   constexpr int NW = C::NW, BNO = C::BNO, TM = C::TM, TN = C::TN, TNO = C::TNO, FM = C::FM, FN = C::FN,
                 FNO = C::FNO, A_BYTES = C::A_BYTES, B_BYTES = C::B_BYTES, STAGE = C::STAGE,
@@ -835,12 +837,13 @@ fp8_gemm_dma_kernel(GemmArgs p) {
   const uint32_t lds0 = lds_offset(&smem[0]);
   auto dma_stage = [&](int kt, int buf) {
     const uint32_t lbase = lds0 + (uint32_t)(buf * STAGE);
-    if (S_INS == NW || wave < S_INS) dma4(s_src + kt * L.sk, s_off, lbase + A_BYTES + B_BYTES + wave * 256);
+    const int kb = WRAP && kt >= (int)(p.kw >> 6) ? kt - (int)(p.kw >> 6) : kt;  // the weights' block
+    if (S_INS == NW || wave < S_INS) dma4(s_src + kb * L.sk, s_off, lbase + A_BYTES + B_BYTES + wave * 256);
     const char* xa = (const char*)p.x + kt * (X32 ? 256 : 128);
 #pragma unroll
     for (int a = 0; a < A_INS; ++a) dma16(xa, a_off[a], lbase + (wave * A_INS + a) * 1024);
 #pragma unroll
-    for (int b = 0; b < B_INS; ++b) dma16(b_src(b) + kt * L.wk, b_off, lbase + A_BYTES + (wave * B_INS + b) * 1024);
+    for (int b = 0; b < B_INS; ++b) dma16(b_src(b) + kb * L.wk, b_off, lbase + A_BYTES + (wave * B_INS + b) * 1024);
   };
 
   // ---- fragment addresses (fixed over K) -----------------------------------
@@ -3951,7 +3954,7 @@ int launch_gemm_dma(const GemmArgs& a, int64_t m_tiles, hipStream_t stream) {
   if (m_tiles <= 0 || n_tiles <= 0) return SMAUL_OK;
   if (m_tiles > 65535 || n_tiles > 65535) return fail(SMAUL_ERR_UNSUPPORTED, "gemm grid too large");
   // the other kernels walk K, twice the weights' where x carries planes
-  if (AM == ACT_PLANES ? 2 * a.kw != a.K : a.kw != 0) return fail(SMAUL_ERR_INVALID, "gemm: planes and kernel differ");
+  if (AM == ACT_PLANES || AM == ACT_WRAP ? 2 * a.kw != a.K : a.kw != 0) return fail(SMAUL_ERR_INVALID, "gemm: planes and kernel differ");
   hipLaunchKernelGGL(
       (fp8_gemm_dma_kernel<CF::BM, CF::BN, CF::WM, CF::WN, CF::NSTAGE, SWIGLU, CANON, true, OUT_F32, AM>),
       dim3((unsigned)n_tiles, (unsigned)m_tiles), dim3(CF::WM * CF::WN * 64), 0, stream, a);
@@ -3984,9 +3987,17 @@ int launch_dense_dma(const GemmArgs& a, int tile, hipStream_t stream) {
   switch (tile) {
     case DT_128x256:
       // two planes of 128 rows would leave one workgroup per CU: 64 rows, past
-      // the grid's 65535 row tiles in launches of that many
+      // the grid's 65535 row tiles in launches of that many.  Few stages over an
+      // output beyond the caches take 128 rows a plane at a time: 64 read the
+      // codes twice as often, which their halved decode does not pay for (two
+      // planes / one, us: 64 -> 512 x 1e6 rows 602 / 564, 131072 76.7 / 76.2; 64 ->
+      // 1024 x 2e5 224 / 215, 66000 68.9 / 71.0; 256 -> 1024 x 2e5 458 / 413, 2e4
+      // 45.9 / 50.5; 512 -> 1024 x 2e5 657 / 669)
       if constexpr (AM == ACT_PLANES) {
         int rc = SMAUL_OK;
+        if constexpr (!SWIGLU)
+          if (a.kw <= 256 && rows >= (1 << 17) && rows * a.N >= (1 << 26) && rows <= 128 * 65535)
+            return launch_gemm_dma<CfgDmaGU, SWIGLU, CANON, OUT_F32, ACT_WRAP>(a, (rows + 127) / 128, stream);
         for (int64_t r0 = 0; r0 < rows && rc == SMAUL_OK; r0 += PLANES_LAUNCH_ROWS) {
           GemmArgs c = a;
           c.R = std::min(rows - r0, PLANES_LAUNCH_ROWS);

@@ -241,6 +241,25 @@ def test_fp8_linear_planes_past_one_launch():
     assert rel_max(y[idx.to(DEV)].cpu(), ref) < 1e-5
 
 
+@pytest.mark.parametrize("rows,in_f,out_f", [
+    (131100, 64, 512),    # 2^26 outputs over one K block: 128 rows a plane at a time, a ragged last tile
+    (131000, 64, 512),    # just under: both planes in a stage
+    (131073, 200, 700),   # packed, four blocks, columns past out_f
+    (131100, 320, 512)])  # five blocks: both planes in a stage
+def test_fp8_linear_fp32_short_k_long_output(rows, in_f, out_f):
+    """Few K blocks over an output beyond the caches: either side of the rule
+    against the oracle, rows sampled, every stored code and scale in use."""
+    print(f"case fp8_linear short K rows={rows} in_f={in_f} out_f={out_f}", flush=True)
+    gen = torch.Generator().manual_seed(rows + in_f)
+    x = torch.randn(rows, in_f, generator=gen)
+    w = torch.randint(0, 256, (out_f, in_f), generator=gen, dtype=torch.int64).to(torch.uint8)
+    s = torch.rand(out_f, -(-in_f // 64), generator=gen) * 0.01 + 1e-3
+    y = be().fp8_forward(x.to(DEV), w.to(DEV), s.to(DEV), in_f, out_f, 64)
+    idx = torch.cat([torch.arange(130), torch.randperm(rows, generator=gen)[:100], torch.arange(rows - 130, rows)])
+    ref = oracle.fp8_forward(x[idx], w, s, in_f, out_f, 64)
+    assert bool(torch.isfinite(y).all()) and rel_max(y[idx.to(DEV)].cpu(), ref) < 1e-5
+
+
 def test_fp8_linear_ws_abi_fallbacks():
     """smaul_fp8_linear_ws through the C-ABI: the two-plane path with a large
     enough workspace and smaul_fp8_linear itself (the in-LDS split) without
