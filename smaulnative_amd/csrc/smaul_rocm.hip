@@ -9,7 +9,7 @@
 //                     (sum_k x[k] * lut[w[k]] * s[k / tile], fp8_cpu.cpp:49-98),
 //                     optional SwiGLU epilogue.
 //   fp8_gemm_kernel   the register-staged grouped / dense GEMM for everything
-//                     else (fp32 activations, tiles 32 and 128*m, short segments).
+//                     else (calls of few rows, tiles 32 and 128*m of the layers).
 //   decode_stream_kernel  T <= 64: units of (segment, 16 columns) streamed
 //                     through a register ring, K split across the waves; the
 //                     gate/up instance dispatches for itself.
@@ -45,6 +45,13 @@
 #include "topk_select.h"
 
 #define SMAUL_VERSION 100
+
+// Alignment of a kernel's code, for the kernels of small calls: 24 to 53 KB that
+// a few workgroups fetch cold.  Code that crosses a 64 KB boundary starts later,
+// and where a kernel lies moves with every kernel before it: a decode pass of
+// eight layers took 314 to 318 us, a layer of 512 tokens 46.5 to 47.5, by other
+// kernels' sizes alone; aligned 313 and 46.8.  (4 KB: as unaligned.)
+#define CODE_ALIGNED(bytes) __attribute__((aligned(bytes)))
 
 namespace {
 
@@ -2585,7 +2592,7 @@ __device__ void cn_tail(const CnrArgs& cr, const void* y, int32_t* arr);
 // (combine_norm_kernel's arithmetic), TAIL_C only combines (combine_kernel's).
 constexpr int TAIL_NONE = 0, TAIL_C = 1, TAIL_CN = 2, TAIL_CNR = 3;
 template <bool SWIGLU, bool CANON, int KBW, bool FUSED, int TAIL = TAIL_NONE, int CEMAX = 8, bool CEXACT = false>
-__global__ void __launch_bounds__(DS_WMAX * 64)
+__global__ void __launch_bounds__(DS_WMAX * 64) CODE_ALIGNED(65536)
 decode_stream_kernel(GemmArgs p, int nw, DsDispatch dd, CnrArgs cr) {
   constexpr int NH = SWIGLU ? 2 : 1;
   static_assert(!FUSED || SWIGLU, "the fused dispatch feeds the gate/up projection");
@@ -2761,7 +2768,7 @@ int launch_decode(const GemmArgs& a, hipStream_t stream) {
 // PLANES (fp32 x): the bf16 hi / lo planes of x are written on the way, by an
 // instance of its own: its stores take 20 registers, a wave of three per SIMD.
 template <bool XBF16, int TB, int EMAX, bool EXACT, bool PLANES>
-__global__ void __launch_bounds__(ROUTE_THREADS)
+__global__ void __launch_bounds__(ROUTE_THREADS) CODE_ALIGNED(65536)
 router_kernel(const void* __restrict__ x, const float* __restrict__ gw, const float* __restrict__ gb,
               RouteOut o, int64_t T, int d, int E_arg, int k) {
   // EXACT: E == EMAX, so every expert guard below is decided at compile time
@@ -2863,7 +2870,7 @@ constexpr int ROUTE_MFMA_THREADS = 512;
 // for the decode step, where a block per 16 tokens shortens each block's
 // loads; the arithmetic per token is the same either way.
 template <int EMAX, bool EXACT, int KSW, int NTT>
-__global__ void __launch_bounds__(ROUTE_MFMA_THREADS)
+__global__ void __launch_bounds__(ROUTE_MFMA_THREADS) CODE_ALIGNED(32768)
 router_mfma_kernel(const uint16_t* __restrict__ x, const float* __restrict__ gw, const float* __restrict__ gb,
                    RouteOut o, int64_t T, int d, int E_arg, int k) {
   static_assert(EMAX <= 16, "the MFMA router covers up to 16 experts");
