@@ -126,7 +126,8 @@ fp8_backward_input_mfma_kernel(const float* __restrict__ g, const uint8_t* __res
 #pragma unroll
       for (int q = 0; q < NC; ++q) sl[q] = s[(o0 + (lane & (TPR - 1)) * 16 + lane / TPR + 8 * q) * nt + kb];
 #pragma unroll
-      for (int j = 0; j < 16; ++j) sv[j] = __shfl(sl[NC == 1 ? 0 : j >> 3], (j % (16 / NC)) * TPR | (lane & (TPR - 1)), 64);
+      for (int j = 0; j < 16; ++j)
+        sv[j] = __shfl(sl[NC == 1 ? 0 : j >> 3], (j % (16 / NC)) * TPR | (lane & (TPR - 1)), 64);
 #pragma unroll
       for (int b = 0; b < NC; ++b)
 #pragma unroll

@@ -1,6 +1,6 @@
 """Writes the golden fixtures under tests/golden/ from the reference itself.
 
-Run in the build container only (the reference is not present on the GPU box):
+Run where the reference is present:
 
     python tests/golden/make_golden.py
 

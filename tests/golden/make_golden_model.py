@@ -2,7 +2,7 @@
 
     python tests/golden/make_golden_model.py
 
-Run in the build container only (the reference is not present on the GPU box).
+Run where the reference is present.
 The model is config 1 cut to 2 layers: d=512, 8
 heads, ffn_mult 2.5, 4 SwiGLU experts top-2, tile 64, byte vocab, batch 2 x
 ctx 256.  Its weights come from tests/_model.draw_state (a seeded recipe keyed

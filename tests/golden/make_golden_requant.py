@@ -1,6 +1,6 @@
 """Writes tests/golden/golden_requant.npz from the reference's own FP8Linear.
 
-Run in the build container only (the reference is not present on the GPU box):
+Run where the reference is present:
 
     python tests/golden/make_golden_requant.py
 

@@ -2,7 +2,7 @@
 
     python tests/golden/make_golden_train.py
 
-Run in the build container only (the reference is not present on the GPU box).
+Run where the reference is present.
 The reference layer (model.py:506-585) at d=128, h=320, E=4, top-2, tile 64,
 in train mode with bf16 activations, through the reference CPU backend whose
 fp8_forward and fp8_backward_input are the reference's own kernel/fp8_cpu.cpp
